@@ -13,9 +13,9 @@
 //     the weight are products of a source and a receiver factor) and the
 //     cosine and sine of the half angle (the reflection-angle factor's
 //     cosine of the mean angle by the addition formula); a trace's weight is
-//     then four products, the angle factor and the aperture taper (7 words
-//     per node and table: T, amplitude, half-angle cosine and sine, and the
-//     gradient for the angle domain's bin);
+//     then four products, the angle factor and the aperture taper (4 words
+//     per node and table: T, amplitude, half-angle cosine and sine; 3 more,
+//     the gradient, for the angle domain's bin);
 //   - the same pass keeps each table's minimum traveltime over every 64
 //     consecutive image points; rounded addition and division being
 //     monotone, a wave whose chunk minima give a time index >= nt holds no
@@ -52,7 +52,9 @@
 namespace seisfat {
 
 constexpr float KDM_EPS = 1e-6f;  // EPS of src/migration/migration.cuh:7
-constexpr int KQ = 7;             // per-table quantities: T, amplitude, cos and sin of half the angle, dT/dx, dT/dz, |grad T| + EPS
+// per-table quantities: T, amplitude, cos and sin of half the angle; the angle
+// domain's bin also needs dT/dx, dT/dz, |grad T| + EPS
+constexpr int kq_words(bool angle) { return angle ? 7 : 4; }
 
 struct KdmK {
   int nz, nx, nzz, npts, nt, nang;
@@ -62,8 +64,11 @@ struct KdmK {
   float zh_dt, zl_dt;  // two-word reciprocal of dt (fdiv)
   int fastdiv_dt;      // fdiv(x, zh_dt, zl_dt) == RN(x / dt) for every 2^-100 <= x < 2^100 (checked exhaustively)
   int taper_rdiv;      // (x - cmp) / sig_e needs no operand rescaling at any node and trace (kdm_weight)
-  int rec_nonneg; // every receiver-table value at an image point is >= 0 (no NaN)
   float dx, dz, dt, da;
+  // k_kdm_prep's constant divisors and their reciprocals RN(1 / b)
+  float dz2, dx2, dxz4, r_dz, r_dx, r_dz2, r_dx2, r_dxz4;
+  int prep_rdiv;        // they lie in [2^-44, 2^44]
+  unsigned nz_recip;    // floor(2^32 / nz) (nz > 1)
   float ntf;     // (float)nt
   float tan_ap;  // tanf(aperture in radians), the reference's sigma / z
   float scale;   // 1 / (2 pi) as the reference rounds it
@@ -76,6 +81,12 @@ __device__ __forceinline__ int f2i_rd(float v) {
   if (v >= 2147483648.0f) return 2147483647;
   if (v < -2147483648.0f) return (-2147483647 - 1);
   return (int)floorf(v);
+}
+
+// Refined reciprocal of b (the r of rdiv).
+__device__ __forceinline__ float recip_refined(float b) {
+  const float r0 = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, r0, 1.0f), r0, r0);
 }
 
 // The per-table quantities of padded table T at interior node (i, j) (padded
@@ -101,53 +112,107 @@ __device__ __forceinline__ int f2i_rd(float v) {
 // be 0).
 __device__ __forceinline__ float min_nan(float a, float b) { return (a != a || b != b) ? __builtin_nanf("") : fminf(a, b); }
 
+//
+// The kernel is bound by instruction issue, so the usual node (prep_rdiv, the
+// nine traveltimes of magnitude in [2^-30, 2^40)) takes a short path: every
+// difference of such floats is 0 or in [2^-54, 2^43), so the divisions by the
+// grid's constants and by the gradient's norm are IEEE division by rdiv and
+// the roots need no rescaling; the amplitude is one reciprocal square root,
+//   amp = num rsqrt(num den), num = det |cos| s', den = norm^2 c'
+// (c' / s' = max(c / S, EPS)), v_rsq_f64 with one Newton step (relative error
+// near 2^-46), rounded once to float.  A wave with any other node (zero, tiny, huge,
+// infinite or NaN traveltimes) takes the general path.  The row of a lane
+// comes from its wave's first point (one scalar division by multiplication).
+// 1001 x 1001, 252 tables, image domain: 1.85 ms; 3.15 ms with IEEE division,
+// two FP64 roots and a division per node and seven words written in either
+// domain.
+__device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+__device__ __forceinline__ float min3f(float a, float b, float c) { return fminf(fminf(a, b), c); }
+
+template <bool ANGLE>
 __global__ __launch_bounds__(256) void k_kdm_prep(const float* __restrict__ tables, int ntab,
                                                   const float* __restrict__ S, KdmK K, float* __restrict__ q,
                                                   float* __restrict__ tmin) {
+  constexpr int KQ = kq_words(ANGLE);
   const int lane = threadIdx.x & 63;
-  const size_t nw = (size_t)ntab * K.nchunk;
-  const size_t wstride = (size_t)gridDim.x * (blockDim.x >> 6);
   const size_t tsize = (size_t)K.nzz * (K.nx + 6);
-  for (size_t w = (size_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); w < nw; w += wstride) {
-    const int tab = (int)(w / K.nchunk);
-    const int p = (int)(w - (size_t)tab * K.nchunk) * 64 + lane;
-    float tv = __builtin_inff();
-    if (p < K.npts) {
-      const int i = p % K.nz + 3, j = p / K.nz + 3;
-      const float* __restrict__ T = tables + tab * tsize;
-      const int nzz = K.nzz;
-      const float c = T[i + j * nzz];
-      const float up = T[(i - 1) + j * nzz], dn = T[(i + 1) + j * nzz];
-      const float lf = T[i + (j - 1) * nzz], rt = T[i + (j + 1) * nzz];
-      const float d_z = 0.5f * (dn - up) / K.dz;
-      const float d_x = 0.5f * (rt - lf) / K.dx;
-      const float d2z = (dn - 2.0f * c + up) / (K.dz * K.dz);
-      const float d2x = (rt - 2.0f * c + lf) / (K.dx * K.dx);
-      const float dxz = (T[(i + 1) + (j + 1) * nzz] - T[(i - 1) + (j + 1) * nzz] - T[(i + 1) + (j - 1) * nzz] +
-                         T[(i - 1) + (j - 1) * nzz]) /
-                        (4.0f * K.dx * K.dz);
-      const float norm = sqrtf(d_x * d_x + d_z * d_z) + KDM_EPS;
-      const float det = fabsf(d2x * d2z - dxz * dxz) + KDM_EPS;
+  const int c = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
+  if (c >= K.nchunk) return;  // whole wave past the end
+  // row and column of the chunk's first point: umulhi(p, floor(2^32 / nz)) is
+  // p / nz or at most two less (p < 2^30)
+  const int pc = c * 64;
+  int jc = K.nz > 1 ? (int)__umulhi((unsigned)pc, K.nz_recip) : pc, ic = pc - jc * K.nz;
+  while (ic >= K.nz) ic -= K.nz, ++jc;
+  const int p = pc + lane;
+  int i = ic + lane, j = jc;
+  while (i >= K.nz) i -= K.nz, ++j;
+  const bool live = p < K.npts;
+  if (!live) i = K.nz - 1, j = K.nx - 1;  // lanes past the end load in bounds and store nothing
+  i += 3;
+  j += 3;
+  const int nzz = K.nzz, o0 = i + j * nzz;
+  const float s = S[o0];
+  for (int tab = blockIdx.y; tab < ntab; tab += gridDim.y) {
+    const float* __restrict__ T = tables + tab * tsize + o0;
+    const float t0 = T[0];
+    const float up = T[-1], dn = T[1], lf = T[-nzz], rt = T[nzz];
+    const float dr = T[1 + nzz], ur = T[-1 + nzz], dl = T[1 - nzz], ul = T[-1 - nzz];
+    const float nzd = 0.5f * (dn - up), nxd = 0.5f * (rt - lf);
+    const float nzzd = dn - 2.0f * t0 + up, nxxd = rt - 2.0f * t0 + lf, nxzd = dr - ur - dl + ul;
+    // the nine magnitudes' least (their greatest is bounded through norm and det; a NaN fails those)
+    const float least = min3f(min3f(fabsf(t0), fabsf(up), fabsf(dn)), min3f(fabsf(lf), fabsf(rt), fabsf(dr)),
+                              min3f(fabsf(ur), fabsf(dl), fabsf(ul)));
+    float d_z = rdiv(nzd, K.dz, K.r_dz), d_x = rdiv(nxd, K.dx, K.r_dx);
+    float norm = rsqrt_rn(d_x * d_x + d_z * d_z) + KDM_EPS;
+    float det = fabsf(rdiv(nxxd, K.dx2, K.r_dx2) * rdiv(nzzd, K.dz2, K.r_dz2) -
+                      [](float a) { return a * a; }(rdiv(nxzd, K.dxz4, K.r_dxz4))) + KDM_EPS;
+    float dot, amp, ch, sh;
+    // (huge, infinite and NaN values show in norm or det)
+    const bool usual = K.prep_rdiv && least >= 0x1p-30f && fabsf(t0) < 0x1p40f && norm < 0x1p40f && det < 0x1p80f;
+    if (__all(usual)) {
+      dot = -rdiv(d_z, norm, recip_refined(norm));  // unit gradient . (0, -1), the surface normal
+      const float cth = fminf(1.0f, fmaxf(-1.0f, dot));
+      const bool far = t0 >= KDM_EPS * s;
+      const double num = (double)det * (double)fabsf(dot) * (double)(far ? s : 1.0f);
+      const double den = (double)norm * (double)norm * (double)(far ? t0 : KDM_EPS);
+      const double x = num * den;
+      const double y = __builtin_amdgcn_rsq(x);
+      const double y1 = __builtin_fma(0.5 * y, __builtin_fma(-x * y, y, 1.0), y);
+      amp = num > 0.0 ? (float)(num * y1) : 0.0f;
+      ch = rsqrt_rn(0.5f * (1.0f + cth));
+      sh = rsqrt_rn(0.5f * (1.0f - cth));
+    } else {
+      d_z = nzd / K.dz;
+      d_x = nxd / K.dx;
+      const float d2z = nzzd / K.dz2, d2x = nxxd / K.dx2, dxz = nxzd / K.dxz4;
+      norm = sqrtf(d_x * d_x + d_z * d_z) + KDM_EPS;
+      det = fabsf(d2x * d2z - dxz * dxz) + KDM_EPS;
       const float ux = d_x / norm, uz = d_z / norm;
-      const float dot = ux * 0.0f + uz * -1.0f;  // unit gradient . (0, -1), the surface normal
+      dot = ux * 0.0f + uz * -1.0f;
       const float cth = fminf(1.0f, fmaxf(-1.0f, dot));  // cos(theta), theta = acos(cth) in the reference
-      const float rs = fmaxf(c / S[i + j * nzz], KDM_EPS);
-      const double amp = sqrt((double)det * (double)fmaxf(0.0f, fabsf(dot))) / ((double)norm * sqrt((double)rs));
+      const float rs = fmaxf(t0 / s, KDM_EPS);
+      amp = (float)(sqrt((double)det * (double)fmaxf(0.0f, fabsf(dot))) / ((double)norm * sqrt((double)rs)));
+      ch = sqrtf(0.5f * (1.0f + cth));
+      sh = sqrtf(0.5f * (1.0f - cth));
+    }
+    if (live) {
       float* __restrict__ o = q + (size_t)tab * KQ * K.npts + p;
-      o[0] = c;
-      o[(size_t)1 * K.npts] = (float)amp;
+      o[0] = t0;
+      o[(size_t)1 * K.npts] = amp;
       // cos and sin of theta / 2 by the half-angle identities (1 +- cth exact
       // where it matters, by Sterbenz): within 5e-8 of those of acos(cth), closer
       // than the cosine and sine of the float acosf(cth)
-      o[(size_t)2 * K.npts] = sqrtf(0.5f * (1.0f + cth));
-      o[(size_t)3 * K.npts] = sqrtf(0.5f * (1.0f - cth));
-      o[(size_t)4 * K.npts] = d_x;
-      o[(size_t)5 * K.npts] = d_z;
-      o[(size_t)6 * K.npts] = norm;
-      tv = c;
+      o[(size_t)2 * K.npts] = ch;
+      o[(size_t)3 * K.npts] = sh;
+      if (ANGLE) {
+        o[(size_t)4 * K.npts] = d_x;
+        o[(size_t)5 * K.npts] = d_z;
+        o[(size_t)6 * K.npts] = norm;
+      }
     }
+    float tv = live ? t0 : __builtin_inff();
     for (int off = 32; off >= 1; off >>= 1) tv = min_nan(tv, __shfl_xor(tv, off, 64));
-    if (lane == 0) tmin[w] = tv;
+    if (lane == 0) tmin[(size_t)tab * K.nchunk + c] = tv;
   }
 }
 
@@ -169,11 +234,34 @@ __global__ __launch_bounds__(256) void k_kdm_tmin2(const float* __restrict__ tmi
   }
 }
 
+// Per table, the least of its super-chunk minima (NaN-propagating): one wave
+// per table.
+__global__ __launch_bounds__(64) void k_kdm_tmin3(const float* __restrict__ tmin2, KdmK K, float* __restrict__ tmin3) {
+  const int lane = threadIdx.x;
+  float v = __builtin_inff();
+  for (int k = lane; k < K.nsup; k += 64) v = min_nan(v, tmin2[(size_t)blockIdx.x * K.nsup + k]);
+  for (int off = 32; off >= 1; off >>= 1) v = min_nan(v, __shfl_xor(v, off, 64));
+  if (lane == 0) tmin3[blockIdx.x] = v;
+}
+
+// Whether no receiver-table value at an image point is negative or NaN: a
+// source may then be passed over on its own minimum.  On the device, so that
+// an operator's launch waits for nothing (reading the chunk minima back took
+// 1 ms on 201 tables of 1001 x 1001).
+__global__ __launch_bounds__(64) void k_kdm_rec_nonneg(const float* __restrict__ rec_tmin3, int nrec,
+                                                       int* __restrict__ flag) {
+  bool ok = true;
+  for (int k = threadIdx.x; k < nrec; k += 64) ok &= rec_tmin3[k] >= 0.0f;
+  const bool all = __all(ok);
+  if (threadIdx.x == 0) *flag = all ? 1 : 0;
+}
+
 struct Q7 {
   float t, amp, ch, sh, dx, dz, norm;
 };
 // The weight's quantities after T (loaded once the node is known to reach the
 // trace).
+template <int KQ>
 __device__ __forceinline__ void q_amp(const float* __restrict__ q, int tab, int p, int npts, Q7& o) {
   const float* __restrict__ b = q + (size_t)tab * KQ * npts + p;
   o.amp = b[(size_t)npts];
@@ -181,6 +269,7 @@ __device__ __forceinline__ void q_amp(const float* __restrict__ q, int tab, int 
   o.sh = b[(size_t)3 * npts];
 }
 // The gradient, for the angle domain's bin.
+template <int KQ>
 __device__ __forceinline__ void q_dir(const float* __restrict__ q, int tab, int p, int npts, Q7& o) {
   const float* __restrict__ b = q + (size_t)tab * KQ * npts + p;
   o.dx = b[(size_t)4 * npts];
@@ -210,12 +299,6 @@ __device__ __forceinline__ int t_index(float xs, const KdmK& K) {
   const float v = (K.fastdiv_dt && mid) ? fdiv(xs, K.zh_dt, K.zl_dt) : xs / K.dt;
   const int it = v != v ? 0 : (int)fminf(fmaxf(floorf(v), -1.0f), (float)K.nt);
   return xs >= K.thr ? K.nt : it;
-}
-
-// Refined reciprocal of b (the r of rdiv).
-__device__ __forceinline__ float recip_refined(float b) {
-  const float r0 = __builtin_amdgcn_rcpf(b);
-  return __builtin_fmaf(__builtin_fmaf(-b, r0, 1.0f), r0, r0);
 }
 
 // True when every node whose traveltime sum is at least RN(a + b) has a time
@@ -306,7 +389,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
                                                      const int* __restrict__ bent, const int* __restrict__ ent,
                                                      const float* __restrict__ tcmp, const int* __restrict__ tcid,
                                                      int nb, int nsrc, const float* __restrict__ data,
-                                                     float* __restrict__ model, float* __restrict__ part, KdmK K) {
+                                                     float* __restrict__ model, float* __restrict__ part,
+                                                     const int* __restrict__ rec_flag, KdmK K) {
+  constexpr int KQ = kq_words(ANGLE);
+  const bool rec_nonneg = *rec_flag != 0;
   const int p0 = blockIdx.x * blockDim.x + threadIdx.x;
   const int nparts = gridDim.y, h = blockIdx.y;
   const int b_begin = (int)((long long)nb * h / nparts), b_end = (int)((long long)nb * (h + 1) / nparts);
@@ -329,7 +415,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
     for (int k = 0; k < SB; ++k) {
       const int sk = bsrc[b * SB + k];
       ms[k] = sk >= 0 ? tmin[(size_t)sk * K.nchunk + c] : 0.0f;
-      const bool u = sk >= 0 && !(K.rec_nonneg && beyond(ms[k], 0.0f, K));
+      const bool u = sk >= 0 && !(rec_nonneg && beyond(ms[k], 0.0f, K));
       use |= (unsigned)__builtin_amdgcn_readfirstlane((int)u) << k;
     }
     if (!use) continue;
@@ -354,8 +440,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
       if (use >> k & 1) {
         const int sk = bsrc[b * SB + k];
         qs[k].t = q[(size_t)sk * KQ * K.npts + p];
-        q_amp(q, sk, p, K.npts, qs[k]);
-        if (ANGLE) q_dir(q, sk, p, K.npts, qs[k]);
+        q_amp<KQ>(q, sk, p, K.npts, qs[k]);
+        if (ANGLE) q_dir<KQ>(q, sk, p, K.npts, qs[k]);
       }
     }
     for (int e0 = e_first; e0 < e1; e0 += 64) {
@@ -435,8 +521,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
         if (!__any(anyok)) continue;  // (the while condition reads the updated m)
         Q7 qr;
         qr.t = rt;
-        q_amp(q, r, p, K.npts, qr);
-        if (ANGLE) q_dir(q, r, p, K.npts, qr);
+        q_amp<KQ>(q, r, p, K.npts, qr);
+        if (ANGLE) q_dir<KQ>(q, r, p, K.npts, qr);
         // every lane of a slot computes its weight; lanes that do not reach
         // the trace add nothing (a select, not a product: their weight may be
         // any value)
@@ -497,6 +583,7 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
                                                      int nsrc,
                                                      const float* __restrict__ model, float* __restrict__ data,
                                                      KdmK K) {
+  constexpr int KQ = kq_words(ANGLE);
   extern __shared__ float hist[];
   const int t = blockIdx.x;
   for (int k = threadIdx.x; k < K.nt; k += blockDim.x) hist[k] = 0.0f;
@@ -524,11 +611,11 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
         const float xs = qs.t + qr.t;
         const int it = t_index(xs, K);
         if ((unsigned)it >= (unsigned)K.nt) continue;
-        q_amp(q, s, p, K.npts, qs);
-        q_amp(q, r, p, K.npts, qr);
+        q_amp<KQ>(q, s, p, K.npts, qs);
+        q_amp<KQ>(q, r, p, K.npts, qr);
         if (ANGLE) {
-          q_dir(q, s, p, K.npts, qs);
-          q_dir(q, r, p, K.npts, qr);
+          q_dir<KQ>(q, s, p, K.npts, qs);
+          q_dir<KQ>(q, r, p, K.npts, qr);
         }
         const int i = p % K.nz, j = p / K.nz;
         const float z = (float)i * K.dz, x = (float)j * K.dx;
@@ -620,9 +707,12 @@ struct seisfat_kdm_s {
   seisfat_kdm_params p{};
   int nsrc = 0, nrec = 0, ntr = 0;
   KdmK K{};
-  float* d_q = nullptr;    // per-table quantities, (nsrc + nrec) x 7 x npts
+  float* d_q = nullptr;    // per-table quantities, (nsrc + nrec) x kq x npts
+  int kq = 0;              // words per node and table (kq_words)
   float* d_tmin = nullptr; // per-table chunk minima of T, (nsrc + nrec) x nchunk
   float* d_tmin2 = nullptr; // per-table minima over 64 chunks, (nsrc + nrec) x nsup
+  float* d_tmin3 = nullptr; // per-table minimum, nsrc + nrec
+  int* d_nonneg = nullptr;  // k_kdm_rec_nonneg's answer
   int* d_src = nullptr;    // trace tables
   int* d_rec = nullptr;
   int nb = 0;              // source blocks of the adjoint
@@ -637,7 +727,7 @@ struct seisfat_kdm_s {
   int tabs_missing = 0;
   unsigned s_version = 0;      // the handle's slowness the set tables were evaluated with
   bool taper_geom = false;     // the divisors and x positions allow rdiv for the taper (taper_geometry_ok)
-  bool rec_dirty = true;       // receiver minima changed since rec_nonneg was derived
+  bool rec_dirty = true;       // receiver minima changed since d_nonneg was derived
 };
 
 namespace {
@@ -698,14 +788,23 @@ bool taper_geometry_ok(const KdmK& K) {
 // The quantities and chunk minima of ntab consecutive tables (padded grids at
 // d_tables) into table slots tab0, tab0 + 1, ...: one wave per chunk.
 void launch_prep(seisfat_kdm_s* k, const float* d_tables, int tab0, int ntab, hipStream_t st) {
-  const size_t nw = (size_t)ntab * k->K.nchunk;
-  const int blocks = (int)std::min<size_t>((nw + 3) / 4, 16384);
-  hipLaunchKernelGGL(k_kdm_prep, dim3(blocks), dim3(256), 0, st, d_tables, ntab, k->h->d_spad, k->K,
-                     k->d_q + (size_t)tab0 * KQ * k->K.npts, k->d_tmin + (size_t)tab0 * k->K.nchunk);
+  // a wave keeps its chunk and walks up to 8 tables (their slowness and
+  // position loaded once), fewer where that leaves the chip short of waves
+  const unsigned bx = (k->K.nchunk + 3) / 4;
+  const unsigned by = (unsigned)std::min<long long>(std::max<long long>((ntab + 7) / 8, 8192 / bx + 1),
+                                                    std::min(ntab, 65535));
+  float* q = k->d_q + (size_t)tab0 * k->kq * k->K.npts;
+  float* tmin = k->d_tmin + (size_t)tab0 * k->K.nchunk;
+  if (k->p.domain == SEISFAT_KDM_ANGLE)
+    hipLaunchKernelGGL(k_kdm_prep<true>, dim3(bx, by), dim3(256), 0, st, d_tables, ntab, k->h->d_spad, k->K, q, tmin);
+  else
+    hipLaunchKernelGGL(k_kdm_prep<false>, dim3(bx, by), dim3(256), 0, st, d_tables, ntab, k->h->d_spad, k->K, q, tmin);
   const size_t ns = (size_t)ntab * k->K.nsup;
   const int blocks2 = (int)std::min<size_t>((ns + 3) / 4, 16384);
-  hipLaunchKernelGGL(k_kdm_tmin2, dim3(blocks2), dim3(256), 0, st, k->d_tmin + (size_t)tab0 * k->K.nchunk, ntab,
-                     k->K, k->d_tmin2 + (size_t)tab0 * k->K.nsup);
+  hipLaunchKernelGGL(k_kdm_tmin2, dim3(blocks2), dim3(256), 0, st, tmin, ntab, k->K,
+                     k->d_tmin2 + (size_t)tab0 * k->K.nsup);
+  hipLaunchKernelGGL(k_kdm_tmin3, dim3(ntab), dim3(64), 0, st, k->d_tmin2 + (size_t)tab0 * k->K.nsup, k->K,
+                     k->d_tmin3 + tab0);
 }
 
 // The operators' launches, one instantiation per domain and taper division.
@@ -714,7 +813,7 @@ void launch_adjoint(seisfat_kdm_s* k, const float* d_data, float* d_model, hipSt
   const dim3 grid((k->K.npts + 255) / 256, k->nparts);
   hipLaunchKernelGGL((k_kdm_adjoint<ANGLE, KDM_SB, RDIV>), grid, dim3(256), 0, st, k->d_q, k->d_tmin, k->h->d_spad,
                      k->d_bsrc, k->d_bent, k->d_ent, k->d_cmp, k->d_cid, k->nb, k->nsrc, d_data, d_model,
-                     ANGLE ? nullptr : k->d_part, k->K);
+                     ANGLE ? nullptr : k->d_part, k->d_nonneg, k->K);
 }
 
 template <bool ANGLE, bool RDIV>
@@ -782,12 +881,22 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   K.npts = (int)npts;
   K.nchunk = (int)((npts + 63) / 64);
   K.nsup = (K.nchunk + 63) / 64;
-  K.rec_nonneg = 0;
   K.nt = p->nt;
   K.ntf = (float)p->nt;
   K.nang = p->domain == SEISFAT_KDM_ANGLE ? p->nang : 0;
   K.dx = h->dx;
   K.dz = h->dz;
+  K.dz2 = K.dz * K.dz;
+  K.dx2 = K.dx * K.dx;
+  K.dxz4 = 4.0f * K.dx * K.dz;
+  K.r_dz = 1.0f / K.dz;
+  K.r_dx = 1.0f / K.dx;
+  K.r_dz2 = 1.0f / K.dz2;
+  K.r_dx2 = 1.0f / K.dx2;
+  K.r_dxz4 = 1.0f / K.dxz4;
+  const auto mid = [](float v) { return v >= 0x1p-20f && v <= 0x1p20f; };
+  K.prep_rdiv = mid(K.dz) && mid(K.dx);
+  K.nz_recip = K.nz > 1 ? (unsigned)(((uint64_t)1 << 32) / (unsigned)K.nz) : 0;
   K.dt = p->dt;
   K.thr = index_threshold(p->dt, p->nt);
   // two-word reciprocal of dt: zh = RN(1/dt); 1 - dt*zh is exact (one fma)
@@ -799,9 +908,12 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   // reference's float argument takes it; 1 / (2 pi) rounded from double
   K.tan_ap = std::tan((float)((double)p->aperture * M_PI / 180.0));
   K.scale = (float)(1.0 / (2.0 * M_PI));
-  hipError_t e = hipMalloc((void**)&k->d_q, (size_t)(nsrc + nrec) * KQ * npts * sizeof(float));
+  k->kq = kq_words(p->domain == SEISFAT_KDM_ANGLE);
+  hipError_t e = hipMalloc((void**)&k->d_q, (size_t)(nsrc + nrec) * k->kq * npts * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin, (size_t)(nsrc + nrec) * K.nchunk * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin2, (size_t)(nsrc + nrec) * K.nsup * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin3, (size_t)(nsrc + nrec) * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_nonneg, sizeof(int));
   if (e == hipSuccess) {
     // exhaustive check of the known-divisor division by dt (every dividend of
     // magnitude in [2^-100, 2^100)) against IEEE division
@@ -823,6 +935,8 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
     kfree(k->d_q);
     kfree(k->d_tmin);
     kfree(k->d_tmin2);
+    kfree(k->d_tmin3);
+    kfree(k->d_nonneg);
     delete k;
     return kfail(SEISFAT_ENOMEM, std::string("hipMalloc of the table quantities: ") + hipGetErrorString(e));
   }
@@ -868,21 +982,22 @@ int seisfat_kdm_set_table(seisfat_kdm_t k, int which, int index, const float* d_
 
 namespace {
 
-// Before a launch: every table set, and rec_nonneg derived from the current
-// receiver minima (a source's run of traces may be passed over on the source
-// minimum alone when no receiver traveltime is negative or NaN).
-int ready(seisfat_kdm_s* k, hipStream_t st) {
+// Before a launch: every table set with the current slowness.
+int ready(seisfat_kdm_s* k) {
   if (k->s_version != k->h->version)
     return kfail(SEISFAT_ESTATE, "the slowness changed since the tables were set (set them again)");
   if (k->tabs_missing) return kfail(SEISFAT_ESTATE, "tables not set (seisfat_kdm_set_tables / _set_table)");
-  if (k->rec_dirty) {
-    std::vector<float> rmin((size_t)k->nrec * k->K.nchunk);
-    KHIP(hipMemcpyAsync(rmin.data(), k->d_tmin + (size_t)k->nsrc * k->K.nchunk, rmin.size() * sizeof(float),
-                        hipMemcpyDeviceToHost, st));
-    KHIP(hipStreamSynchronize(st));
-    k->K.rec_nonneg = std::all_of(rmin.begin(), rmin.end(), [](float v) { return v >= 0.0f; }) ? 1 : 0;
-    k->rec_dirty = false;
-  }
+  return SEISFAT_OK;
+}
+
+// d_nonneg from the current receiver minima, before an adjoint.  A launch that
+// is only being captured has not happened yet: the next call launches it too.
+int derive_nonneg(seisfat_kdm_s* k, hipStream_t st) {
+  if (!k->rec_dirty) return SEISFAT_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  KHIP(hipStreamIsCapturing(st, &cap));
+  hipLaunchKernelGGL(k_kdm_rec_nonneg, dim3(1), dim3(64), 0, st, k->d_tmin3 + k->nsrc, k->nrec, k->d_nonneg);
+  if (cap == hipStreamCaptureStatusNone) k->rec_dirty = false;
   return SEISFAT_OK;
 }
 
@@ -970,9 +1085,10 @@ int seisfat_kdm_set_traces(seisfat_kdm_t k, int ntr, const int* src, const int* 
 int seisfat_kdm_adjoint(seisfat_kdm_t k, const float* d_data, float* d_model, void* stream) {
   if (!k) return kfail(SEISFAT_EINVAL, "null operator");
   hipStream_t st = (hipStream_t)stream;
-  if (const int rc = ready(k, st)) return rc;
+  if (const int rc = ready(k)) return rc;
   if (k->ntr == 0) return SEISFAT_OK;  // no traces: the model is unchanged
   if (!d_data || !d_model) return kfail(SEISFAT_EINVAL, "null buffer");
+  if (const int rc = derive_nonneg(k, st)) return rc;
   const bool rd = k->K.taper_rdiv != 0;
   if (k->p.domain == SEISFAT_KDM_IMAGE) {
     if (rd)
@@ -994,7 +1110,7 @@ int seisfat_kdm_adjoint(seisfat_kdm_t k, const float* d_data, float* d_model, vo
 int seisfat_kdm_forward(seisfat_kdm_t k, const float* d_model, float* d_data, void* stream) {
   if (!k) return kfail(SEISFAT_EINVAL, "null operator");
   hipStream_t st = (hipStream_t)stream;
-  if (const int rc = ready(k, st)) return rc;
+  if (const int rc = ready(k)) return rc;
   if (k->ntr == 0) return SEISFAT_OK;  // no traces to add into
   if (!d_data || !d_model) return kfail(SEISFAT_EINVAL, "null buffer");
   const bool rd = k->K.taper_rdiv != 0;
@@ -1019,6 +1135,8 @@ int seisfat_kdm_destroy(seisfat_kdm_t k) {
   kfree(k->d_q);
   kfree(k->d_tmin);
   kfree(k->d_tmin2);
+  kfree(k->d_tmin3);
+  kfree(k->d_nonneg);
   delete k;
   return SEISFAT_OK;
 }

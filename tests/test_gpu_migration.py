@@ -394,3 +394,33 @@ def test_no_traces_within_the_offset(setup, torch):
     assert img.shape == K.model_shape and not img.any()
     assert tuple(K.forward(torch.ones(K.model_shape, device="cuda")).shape) == (0, K.nt)
     K.close()
+
+
+# the table setup's usual path and its general one (traveltimes that are zero,
+# tiny, huge or not finite, whole tables or single nodes), rows that wrap inside
+# a chunk (nz below, at and above 64, no multiple of it), both domains
+@pytest.mark.parametrize("domain", [mig.IMAGE, mig.ANGLE])
+@pytest.mark.parametrize("nz,nx,scale,spoil", [(5, 41, 1.0, None), (64, 33, 1.0, None), (65, 40, 1e-12, None),
+                                               (131, 30, 1.0, 0.0), (70, 30, 1.0, np.inf), (70, 30, 1.0, np.nan),
+                                               (70, 30, 1.0, 1e30)])
+def test_table_setup_paths(oracle, torch, domain, nz, nx, scale, spoil):
+    m, xs, xr = survey(nz=nz, nx=nx, nsrc=3, nrec=9, seed=nz)
+    e = Eikonal(nz, nx, m.dz, m.dx)
+    e.set_slowness(m.s)
+    ts, tr = (scale * e.traveltime_tables(x, np.full_like(x, 11.0)) for x in (xs, xr))
+    ts, tr = ts.astype(np.float32), tr.astype(np.float32)
+    if spoil is not None:
+        ts[1, 20, nz // 2], tr[4, 12:14, nz // 3] = spoil, spoil
+    K = make(e, m, xs, xr, domain, nt=300, dt=1e-3, tables=(ts, tr), max_offset=400.0)
+    S = oracle.expand_boundary(m.s)
+    op = dict(dt=float(K.dt), dx=m.dx, dz=m.dz, aperture=30.0, da=float(K.da), nang=K.nang)
+    d = np.random.default_rng(3).standard_normal((K.ntr, K.nt)).astype(np.float32)
+    cid = K.cmp_id if domain == mig.ANGLE else None
+    got = K.adjoint(torch.from_numpy(d).cuda()).cpu().numpy()
+    want = oracle.kdm(domain, True, S, ts, tr, K.src, K.rec, K.cmp, cid, d, np.zeros(K.model_shape, np.float32), **op)
+    fin = np.isfinite(want)
+    assert np.array_equal(fin, np.isfinite(got))
+    bad = np.abs(got - want)[fin] > 1e-5 * np.abs(want[fin]).max()
+    assert bad.mean() <= (1e-3 if domain == mig.ANGLE else 0.0)
+    K.close()
+    e.close()
