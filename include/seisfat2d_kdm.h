@@ -83,7 +83,7 @@ int seisfat_kdm_destroy(seisfat_kdm_t k);
  * (unnormalised, size nfft = the power of two >= nt + nw - 1) and shifts by
  * nw/2 + nw/10 samples; here the same linear (cross-)correlation is summed
  * directly in double precision, times nfft.  d_in and d_out: ntr x nt device
- * arrays (distinct). */
+ * arrays (distinct).  In stream order; `wavelet` may be reused on return. */
 int seisfat_trace_convolve(int adjoint, int ntr, int nt, const float* wavelet, int nw, const float* d_in,
                            float* d_out, void* stream);
 

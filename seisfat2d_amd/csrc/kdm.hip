@@ -34,8 +34,8 @@
 //     trace once; the tables' minima over 64 chunks let it pass over 4096
 //     image points with one test;
 //   - convolution: the FFT product of the reference is a linear
-//     (cross-)correlation with the wavelet, summed directly in double, the
-//     trace and the wavelet staged in LDS.
+//     (cross-)correlation with the wavelet, summed directly in double, eight
+//     samples per thread from a trace staged in LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
 // Trace convolution: one thread per output sample.  Adjoint: out[k] =
 // nfft * sum_m w[m] in[k - shift + m] for k >= shift (0 before); forward:
 // out[k] = nfft * sum_m in[m] w[k + shift - m].  Sums in double, in the
-// order of m.
+// order of m.  For wavelets too long for LDS or not finite.
 template <bool ADJ>
 __global__ __launch_bounds__(256) void k_trace_conv(const float* __restrict__ in, float* __restrict__ out, int ntr,
                                                     int nt, const float* __restrict__ w, int nw, int shift,
@@ -664,38 +664,79 @@ __global__ __launch_bounds__(256) void k_trace_conv(const float* __restrict__ in
   out[g] = (float)(acc * nfft);
 }
 
-// The same sums with one workgroup per trace, the trace and the wavelet staged
-// in LDS (nt + nw <= 16384 floats): every tap is read from LDS instead of
-// global memory.  Same operands, same order: the same bits.
-template <bool ADJ>
-__global__ __launch_bounds__(256) void k_trace_conv_lds(const float* __restrict__ in, float* __restrict__ out,
-                                                        int nt, const float* __restrict__ w, int nw, int shift,
-                                                        double nfft) {
+// The same sums, eight consecutive samples per thread.  Both directions are
+//   out[k] = nfft * sum_i h[i] x[k + off + i],  x = 0 outside the trace,
+// with h = w, off = -shift (adjoint) or h = w reversed, off = shift - nw + 1
+// (forward): a thread's eight sums share their samples, so a tap costs one LDS
+// read, one conversion and eight FP64 fmas with h from scalar registers (a
+// thread per sample reads and converts two operands per tap).  A product of
+// two floats is exact in double, so the fma is the plain sum's rounding, and a
+// sample outside the trace adds h * 0 (the host checks that h is finite): the
+// same bits.  A workgroup's threads (at most 256) take `tpw` traces of `groups`
+// groups each, or one segment of CONV_SEG samples of a longer one; the samples lie in
+// LDS with one word of padding per eight, so the threads' reads (stride 9) meet
+// no bank conflict.  Bound by FP64 issue: 3609 traces of 8001 samples, 234
+// taps: 0.282 ms (24 T fma/s), 1.77 ms with a sample per thread; 1001 samples:
+// 0.053 against 0.132-0.144 ms.
+constexpr int CONV_R = 8, CONV_SEG = 256 * CONV_R;
+constexpr int CONV_TAPS = 896;  // wavelet samples per k_put_taps launch (its argument's size)
+struct Taps {
+  float w[CONV_TAPS];
+};
+
+// The wavelet from the kernel's argument to device memory, as doubles: no
+// host buffer has to outlive the launch.
+__global__ __launch_bounds__(256) void k_put_taps(Taps a, int n, double* __restrict__ h) {
+  for (int k = threadIdx.x; k < n; k += 256) h[k] = a.w[k];
+}
+
+__global__ __launch_bounds__(256) void k_trace_conv_reg(const float* __restrict__ in, float* __restrict__ out, int ntr,
+                                                        int nt, const double* __restrict__ h, int nw, int off,
+                                                        int first, double nfft, int tpw, int groups, int span) {
   extern __shared__ float sm[];
-  float* tr = sm;
-  float* wl = sm + nt;
-  const size_t t = blockIdx.x;
-  const float* __restrict__ d = in + t * nt;
-  for (int k = threadIdx.x; k < nt; k += blockDim.x) tr[k] = d[k];
-  for (int k = threadIdx.x; k < nw; k += blockDim.x) wl[k] = w[k];
-  __syncthreads();
-  float* __restrict__ o = out + t * nt;
-  for (int k = threadIdx.x; k < nt; k += blockDim.x) {
-    double acc = 0.0;
-    if (ADJ) {
-      if (k < shift) {
-        o[k] = 0.0f;
-        continue;
-      }
-      const int k0 = k - shift;
-      const int mmax = min(nw - 1, nt - 1 - k0);
-      for (int m = 0; m <= mmax; ++m) acc += (double)wl[m] * (double)tr[k0 + m];
-    } else {
-      const int kk = k + shift;
-      for (int m = max(0, kk - nw + 1); m <= min(kk, nt - 1); ++m) acc += (double)tr[m] * (double)wl[kk - m];
+  const int tl = threadIdx.x / groups;  // the thread's trace in the workgroup
+  const int t0 = blockIdx.x * tpw, k0 = blockIdx.y * CONV_SEG;
+  const int pitch = span + span / CONV_R + 1;
+  for (int tr = 0; tr < tpw; ++tr)
+    for (int q = threadIdx.x; q < span; q += blockDim.x) {
+      const int x = k0 + off + q;
+      sm[tr * pitch + q + q / CONV_R] = (t0 + tr < ntr && x >= 0 && x < nt) ? in[(size_t)(t0 + tr) * nt + x] : 0.0f;
     }
-    o[k] = (float)(acc * nfft);
+  __syncthreads();
+  const int g = threadIdx.x - tl * groups, k = k0 + g * CONV_R;
+  if (tl >= tpw || t0 + tl >= ntr || k >= nt) return;
+  const float* __restrict__ x = sm + tl * pitch + g * (CONV_R + 1);
+  double acc[CONV_R], X[2 * CONV_R];
+#pragma unroll
+  for (int o = 0; o < CONV_R; ++o) {
+    acc[o] = 0.0;
+    X[o] = x[o];
   }
+  int i = 0;
+  for (; i + CONV_R <= nw; i += CONV_R) {
+    x += CONV_R + 1;
+#pragma unroll
+    for (int o = 0; o < CONV_R; ++o) X[CONV_R + o] = x[o];
+#pragma unroll
+    for (int u = 0; u < CONV_R; ++u)
+#pragma unroll
+      for (int o = 0; o < CONV_R; ++o) acc[o] = __builtin_fma(h[i + u], X[u + o], acc[o]);
+#pragma unroll
+    for (int o = 0; o < CONV_R; ++o) X[o] = X[CONV_R + o];
+  }
+  x += CONV_R + 1;
+#pragma unroll
+  for (int o = 0; o < CONV_R - 1; ++o) X[CONV_R + o] = x[o];
+#pragma unroll
+  for (int u = 0; u < CONV_R - 1; ++u) {
+    if (i + u >= nw) break;
+#pragma unroll
+    for (int o = 0; o < CONV_R; ++o) acc[o] = __builtin_fma(h[i + u], X[u + o], acc[o]);
+  }
+  float* __restrict__ d = out + (size_t)(t0 + tl) * nt;
+#pragma unroll
+  for (int o = 0; o < CONV_R; ++o)
+    if (k + o < nt) d[k + o] = k + o < first ? 0.0f : (float)(acc[o] * nfft);
 }
 
 }  // namespace seisfat
@@ -1151,27 +1192,40 @@ int seisfat_trace_convolve(int adjoint, int ntr, int nt, const float* wavelet, i
   while (nfft < (long long)nt + nw - 1) nfft <<= 1;
   const int shift = nw / 2 + nw / 10;
   hipStream_t st = (hipStream_t)stream;
+  const size_t n = (size_t)ntr * nt;
+  // samples a workgroup stages per trace: its outputs, the taps, and up to the next whole group
+  const int groups = std::min((nt + CONV_R - 1) / CONV_R, 256);
+  const long long span = (long long)groups * CONV_R + ((nw + CONV_R - 1) / CONV_R + 1) * CONV_R;
+  const size_t lds1 = (size_t)(span + span / CONV_R + 1) * sizeof(float);
+  if (lds1 <= 65536 && std::all_of(wavelet, wavelet + nw, [](float v) { return std::isfinite(v); })) {
+    // several short traces per workgroup, within 40 KB (four workgroups per CU)
+    const int tpw = (int)std::max<size_t>(1, std::min<size_t>(256 / groups, 40960 / lds1));
+    double* d_h = nullptr;
+    KHIP(hipMallocAsync((void**)&d_h, nw * sizeof(double), st));
+    for (int i0 = 0; i0 < nw; i0 += CONV_TAPS) {
+      Taps a;
+      const int m = std::min(CONV_TAPS, nw - i0);
+      for (int i = 0; i < m; ++i) a.w[i] = adjoint ? wavelet[i0 + i] : wavelet[nw - 1 - (i0 + i)];
+      hipLaunchKernelGGL(k_put_taps, dim3(1), dim3(256), 0, st, a, m, d_h + i0);
+    }
+    const dim3 grid((ntr + tpw - 1) / tpw, (nt + CONV_SEG - 1) / CONV_SEG);
+    hipLaunchKernelGGL(k_trace_conv_reg, grid, dim3((tpw * groups + 63) / 64 * 64), tpw * lds1, st, d_in, d_out, ntr, nt, d_h, nw,
+                       adjoint ? -shift : shift - nw + 1, adjoint ? shift : 0, (double)nfft, tpw, groups, (int)span);
+    const hipError_t e = hipGetLastError();
+    KHIP(hipFreeAsync(d_h, st));
+    KHIP(e);
+    return SEISFAT_OK;
+  }
   float* d_w = nullptr;
   KHIP(hipMallocAsync((void**)&d_w, nw * sizeof(float), st));
   KHIP(hipMemcpyAsync(d_w, wavelet, nw * sizeof(float), hipMemcpyHostToDevice, st));
-  const size_t n = (size_t)ntr * nt;
-  if ((long long)nt + nw <= 16384) {
-    const size_t lds = (size_t)(nt + nw) * sizeof(float);
-    if (adjoint)
-      hipLaunchKernelGGL(k_trace_conv_lds<true>, dim3(ntr), dim3(256), lds, st, d_in, d_out, nt, d_w, nw, shift,
-                         (double)nfft);
-    else
-      hipLaunchKernelGGL(k_trace_conv_lds<false>, dim3(ntr), dim3(256), lds, st, d_in, d_out, nt, d_w, nw, shift,
-                         (double)nfft);
-  } else {
-    const int blocks = (int)((n + 255) / 256);
-    if (adjoint)
-      hipLaunchKernelGGL(k_trace_conv<true>, dim3(blocks), dim3(256), 0, st, d_in, d_out, ntr, nt, d_w, nw, shift,
-                         (double)nfft);
-    else
-      hipLaunchKernelGGL(k_trace_conv<false>, dim3(blocks), dim3(256), 0, st, d_in, d_out, ntr, nt, d_w, nw, shift,
-                         (double)nfft);
-  }
+  const int blocks = (int)((n + 255) / 256);
+  if (adjoint)
+    hipLaunchKernelGGL(k_trace_conv<true>, dim3(blocks), dim3(256), 0, st, d_in, d_out, ntr, nt, d_w, nw, shift,
+                       (double)nfft);
+  else
+    hipLaunchKernelGGL(k_trace_conv<false>, dim3(blocks), dim3(256), 0, st, d_in, d_out, ntr, nt, d_w, nw, shift,
+                       (double)nfft);
   KHIP(hipGetLastError());
   KHIP(hipFreeAsync(d_w, st));
   KHIP(hipStreamSynchronize(st));  // the host wavelet is the caller's

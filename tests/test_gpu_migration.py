@@ -424,3 +424,25 @@ def test_table_setup_paths(oracle, torch, domain, nz, nx, scale, spoil):
     assert bad.mean() <= (1e-3 if domain == mig.ANGLE else 0.0)
     K.close()
     e.close()
+
+
+# the register-blocked convolution at the edges of its groups of 8, segments of
+# 2048, traces per workgroup and taps per upload (896), and the direct kernel
+# for a wavelet that is too long or not finite
+@pytest.mark.parametrize("adjoint", [False, True])
+@pytest.mark.parametrize("ntr,nt,nw", [(1, 1, 1), (70, 7, 9), (33, 8, 16), (3, 1023, 895), (5, 1024, 896), (3, 2047, 897),
+                                       (2, 2048, 8), (2, 2049, 7), (2, 4100, 1793), (2, 300, 13000), (4, 50, -20)])
+def test_convolution_block_edges(oracle, torch, adjoint, ntr, nt, nw):
+    import ctypes as C
+    from seisfat2d_amd import capi
+    rng = np.random.default_rng(nt + abs(nw))
+    w = rng.standard_normal(abs(nw)).astype(np.float32)
+    if nw < 0:
+        w[3] = np.inf
+    x = rng.standard_normal((ntr, nt)).astype(np.float32)
+    xi = torch.from_numpy(x).cuda()
+    out = torch.empty_like(xi)
+    capi.check(capi.lib().seisfat_trace_convolve(int(adjoint), ntr, nt, capi._ptr(w), len(w), C.c_void_p(xi.data_ptr()),
+                                                 C.c_void_p(out.data_ptr()),
+                                                 C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert np.array_equal(out.cpu().numpy(), oracle.trace_convolve(x, w, adjoint), equal_nan=True)
