@@ -73,7 +73,8 @@ int seisfat_kdm_set_traces(seisfat_kdm_t k, int ntr, const int* src, const int* 
 int seisfat_kdm_adjoint(seisfat_kdm_t k, const float* d_data, float* d_model, void* stream);
 /* data += L model: perform_forward for every trace
  * (image_domain_forward_kernel / angle_domain_forward_kernel,
- * src/migration/migration.cu:485-570,665-756). */
+ * src/migration/migration.cu:485-570,665-756).  The first call after tables or
+ * traces were set waits for a count on `stream` (not while it is captured). */
 int seisfat_kdm_forward(seisfat_kdm_t k, const float* d_model, float* d_data, void* stream);
 int seisfat_kdm_destroy(seisfat_kdm_t k);
 

@@ -29,10 +29,11 @@
 //     partial images are added in a fixed order, deterministic, no atomics;
 //     angle domain: adds into the (depth, angle, CMP) bins with atomics, as
 //     the reference (their order varies);
-//   - forward: one workgroup (sixteen waves) per trace accumulates the trace
-//     in an LDS histogram of its nt samples (LDS atomics) and adds it to the
-//     trace once; the tables' minima over 64 chunks let it pass over 4096
-//     image points with one test;
+//   - forward: short records: one workgroup (sixteen waves) per trace
+//     accumulates the trace in an LDS histogram of its nt samples (FP64 LDS
+//     atomics) and adds it to the trace once; the tables' minima over 64 chunks
+//     let it pass over 4096 image points with one test.  Others: one workgroup
+//     per image tile and source block, each trace's samples in an LDS window;
 //   - convolution: the FFT product of the reference is a linear
 //     (cross-)correlation with the wavelet, summed directly in double, eight
 //     samples per thread from a trace staged in LDS.
@@ -333,14 +334,18 @@ __device__ __forceinline__ float exp_nonpos(float x) {
 }
 
 template <bool RDIV>
-__device__ __forceinline__ float kdm_weight(const Q7& s, const Q7& r, float sS, float x, float sig_e, float r_sig,
-                                            float cmp) {
-  const float rf = __builtin_fmaf(0.2f, __builtin_fmaf(s.ch, r.ch, -(s.sh * r.sh)), 1.0f);
+__device__ __forceinline__ float kdm_taper(float x, float cmp, float sig_e, float r_sig) {
   const float n = x - cmp;
   // RDIV: |a| < 2^61, so -0.5 a a is finite and <= 0
   const float a = RDIV ? rdiv(n, sig_e, r_sig) : n / sig_e;
-  const float taper = RDIV ? exp_nonpos(-0.5f * a * a) : expf(-0.5f * a * a);
-  return sS * (s.amp * r.amp) * rf * taper;
+  return RDIV ? exp_nonpos(-0.5f * a * a) : expf(-0.5f * a * a);
+}
+
+template <bool RDIV>
+__device__ __forceinline__ float kdm_weight(const Q7& s, const Q7& r, float sS, float x, float sig_e, float r_sig,
+                                            float cmp) {
+  const float rf = __builtin_fmaf(0.2f, __builtin_fmaf(s.ch, r.ch, -(s.sh * r.sh)), 1.0f);
+  return sS * (s.amp * r.amp) * rf * kdm_taper<RDIV>(x, cmp, sig_e, r_sig);
 }
 
 // Reflection-angle bin of the node for the trace (the reference's aId).
@@ -562,14 +567,15 @@ __global__ __launch_bounds__(256) void k_kdm_sum_parts(float* __restrict__ model
   model[p] = v;
 }
 
-// Forward (image or angle domain): one workgroup per trace, the trace's nt
-// samples in LDS; a wave passes over 4096 image points whose super-chunk
+// Forward (image or angle domain) for records that little of the image reaches:
+// one workgroup per trace, the trace's nt samples in LDS (FP64, see
+// k_kdm_forward_tile); a wave passes over 4096 image points whose super-chunk
 // minima keep them beyond the last sample with one test, then over 64 when
 // the chunk minima do.
 // Threads per trace (one workgroup, sixteen waves sharing the trace's LDS
-// histogram).  Measured on the 1001 x 1001 survey against 256 and 512: the
-// 1 s record's forward 0.224 ms against 0.269 and 0.233 (image), 0.32 against
-// 0.44 and 0.37 (angle); the 8 s record's 19.5 ms against 19.9 and 19.7.
+// histogram).  Measured on the 1001 x 1001 survey against 256 and 512 (FP32
+// histogram): the 1 s record's forward 0.224 ms against 0.269 and 0.233 (image),
+// 0.32 against 0.44 and 0.37 (angle).
 #ifndef SEISFAT_KDM_FWD_THREADS
 #define SEISFAT_KDM_FWD_THREADS 1024
 #endif
@@ -584,9 +590,9 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
                                                      const float* __restrict__ model, float* __restrict__ data,
                                                      KdmK K) {
   constexpr int KQ = kq_words(ANGLE);
-  extern __shared__ float hist[];
+  extern __shared__ double hist[];
   const int t = blockIdx.x;
-  for (int k = threadIdx.x; k < K.nt; k += blockDim.x) hist[k] = 0.0f;
+  for (int k = threadIdx.x; k < K.nt; k += blockDim.x) hist[k] = 0.0;
   __syncthreads();
   const int s = tsrc[t], r = nsrc + trec[t];
   const float cmp = tcmp[t];
@@ -624,16 +630,267 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
         const float w = kdm_weight<RDIV>(qs, qr, sS, x, sig_e, recip_refined(sig_e), cmp);
         if (ANGLE) {
           const int a = kdm_angle_bin(qs, qr, K);
-          if (a >= 0 && a < K.nang) atomicAdd(hist + it, w * model[moff + i + (size_t)a * K.nz]);
+          if (a >= 0 && a < K.nang) atomicAdd(hist + it, (double)(w * model[moff + i + (size_t)a * K.nz]));
         } else {
-          atomicAdd(hist + it, w * model[p]);
+          atomicAdd(hist + it, (double)(w * model[p]));
         }
       }
     }
   }
   __syncthreads();
   float* __restrict__ d = data + (size_t)t * K.nt;
-  for (int k = threadIdx.x; k < K.nt; k += blockDim.x) d[k] += hist[k];
+  for (int k = threadIdx.x; k < K.nt; k += blockDim.x) d[k] += (float)hist[k];
+}
+
+// Forward for records that much of the image reaches: one workgroup per image
+// tile (64 rows x FT_WAVES * NPT columns; lane = row, wave = NPT columns) and
+// slice of a source block's entries (the adjoint's blocks).  A node's source
+// quantities stay in registers for the whole slice and a receiver's are loaded
+// once for up to four traces, where the trace kernel below loads both for every
+// pair (32 B a pair: that, beyond L2, bounds it).  Each trace's contributions
+// gather in an LDS window of the samples the tile can reach: the index of the
+// tile's least and greatest traveltime sums bounds every node's (rounded
+// addition and division are monotone), windows longer than FT_WIN take several
+// rounds.  The windows are flushed to the traces with global atomics, contiguous
+// and several hundred nodes to a sample, and double-buffered, so an entry needs
+// one barrier.  LDS sums are FP64: ds_add_f32 takes 169 cycles per wave
+// instruction on this chip whatever its addresses, ds_add_f64 8 to 20 (39 with
+// pairs of lanes on one address), and the sum is the more exact one.  Bound by
+// instruction issue (about 50 VALU per wave and pair).  1001 x 1001, 3609 traces
+// of 8001 samples: 6.1 ms, against 19.7 ms by trace with an FP32 histogram and
+// 16.8 with an FP64 one.
+constexpr int FT_WAVES = 8, FT_WIN = 1024, FT_LIST = 128;
+constexpr int ft_npt(bool angle) { return angle ? 1 : 2; }
+
+// The least (NaN-propagating) and greatest traveltime of every table over
+// every tile of 64 rows and `cols` columns: one wave per table and tile.
+__global__ __launch_bounds__(256) void k_kdm_tile_bounds(const float* __restrict__ q, int kq, int ntab, int ntz,
+                                                         int ntile, int cols, KdmK K, float* __restrict__ lo,
+                                                         float* __restrict__ hi) {
+  const int lane = threadIdx.x & 63;
+  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile >= ntile) return;
+  const int i = tile % ntz * 64 + lane, j0 = tile / ntz * cols;
+  for (int tab = blockIdx.y; tab < ntab; tab += gridDim.y) {
+    float a = __builtin_inff(), b = -__builtin_inff();
+    if (i < K.nz) {
+      const float* __restrict__ t0 = q + (size_t)tab * kq * K.npts + i;
+#pragma unroll 8
+      for (int j = j0; j < min(j0 + cols, K.nx); ++j) {
+        const float t = t0[(size_t)j * K.nz];
+        a = min_nan(a, t);
+        b = fmaxf(b, t);
+      }
+    }
+    for (int off = 32; off >= 1; off >>= 1) {
+      a = min_nan(a, __shfl_xor(a, off, 64));
+      b = fmaxf(b, __shfl_xor(b, off, 64));
+    }
+    if (lane == 0) {
+      lo[(size_t)tab * ntile + tile] = a;
+      hi[(size_t)tab * ntile + tile] = b;
+    }
+  }
+}
+
+// For launch_forward's choice: cnt[0] += the tiles that each trace reaches,
+// cnt[1] += the window rounds these take.  One wave per trace.
+__global__ __launch_bounds__(64) void k_kdm_tile_count(const float* __restrict__ tlo, const float* __restrict__ thi,
+                                                       int ntile, const int* __restrict__ tsrc,
+                                                       const int* __restrict__ trec, int nsrc, KdmK K,
+                                                       unsigned long long* __restrict__ cnt) {
+  const float* __restrict__ sl = tlo + (size_t)tsrc[blockIdx.x] * ntile;
+  const float* __restrict__ sh = thi + (size_t)tsrc[blockIdx.x] * ntile;
+  const float* __restrict__ rl = tlo + (size_t)(nsrc + trec[blockIdx.x]) * ntile;
+  const float* __restrict__ rh = thi + (size_t)(nsrc + trec[blockIdx.x]) * ntile;
+  unsigned a = 0, b = 0;
+  for (int t = threadIdx.x; t < ntile; t += 64) {
+    if (beyond(sl[t], rl[t], K)) continue;
+    const float w = (fminf(sh[t] + rh[t], K.thr) - fmaxf(sl[t] + rl[t], 0.0f)) / K.dt;
+    ++a;
+    b += 1 + (unsigned)(fminf(fmaxf(w, 0.0f), 16384.0f) / FT_WIN);
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    a += __shfl_xor(a, off, 64);
+    b += __shfl_xor(b, off, 64);
+  }
+  if (threadIdx.x == 0 && a) {
+    atomicAdd(cnt, (unsigned long long)a);
+    atomicAdd(cnt + 1, (unsigned long long)b);
+  }
+}
+
+__global__ void k_kdm_clear(unsigned long long* __restrict__ cnt) { cnt[threadIdx.x] = 0; }
+
+// An entry of the adjoint's list that reaches the tile.
+template <int SB>
+struct FtEntry {
+  int r, pass;                 // receiver table; bit k: slot k reaches, bit 8 + k: by the short index
+  int t[SB], lo[SB], len[SB];  // trace, first sample the tile can reach, samples from there
+  float cmp[SB];
+  int bin[SB];
+};
+
+template <bool ANGLE, int SB, int NPT, bool RDIV>
+__global__ __launch_bounds__(64 * FT_WAVES) void k_kdm_forward_tile(
+    const float* __restrict__ q, const float* __restrict__ tlo, const float* __restrict__ thi, int ntz, int ntile,
+    const float* __restrict__ S, const int* __restrict__ bsrc, const int* __restrict__ bent,
+    const int* __restrict__ ent, const float* __restrict__ tcmp, const int* __restrict__ tcid, int nsplit, int nsrc,
+    const float* __restrict__ model, float* __restrict__ data, KdmK K) {
+  constexpr int KQ = kq_words(ANGLE), THREADS = 64 * FT_WAVES;
+  constexpr float FAR = 0x1p90f;  // traveltime of a lane outside the image: no sample
+  __shared__ double win[2][SB][FT_WIN];
+  __shared__ FtEntry<SB> list[FT_LIST];
+  __shared__ int count[FT_LIST / 64];
+  // workgroups go round robin over the XCDs: the blocks of one tile follow each other on one XCD
+  const int tile = blockIdx.y * 8 + (blockIdx.x & 7), b = (blockIdx.x >> 3) / nsplit, h = (blockIdx.x >> 3) % nsplit;
+  if (tile >= ntile) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int i = tile % ntz * 64 + lane, ic = min(i, K.nz - 1);
+  const int j0 = tile / ntz * (FT_WAVES * NPT) + wave * NPT;
+  const float sig_e = K.tan_ap * ((float)ic * K.dz) + KDM_EPS;
+  const float r_sig = recip_refined(sig_e);
+  int p[NPT];
+  float x[NPT], sS[NPT];
+#pragma unroll
+  for (int n = 0; n < NPT; ++n) {
+    const int jc = min(j0 + n, K.nx - 1);
+    p[n] = ic + jc * K.nz;
+    x[n] = (float)jc * K.dx;
+    sS[n] = 0.0f;
+  }
+  int par = 0;
+  float ms[SB], mh[SB];
+#pragma unroll
+  for (int k = 0; k < SB; ++k) {
+    const int sk = bsrc[b * SB + k];
+    ms[k] = sk >= 0 ? tlo[(size_t)sk * ntile + tile] : 0.0f;
+    mh[k] = sk >= 0 ? thi[(size_t)sk * ntile + tile] : 0.0f;
+  }
+  const int ne = bent[b + 1] - bent[b];
+  const int e1 = bent[b] + (int)((long long)ne * (h + 1) / nsplit);
+  bool started = false;
+  Q7 qs[NPT][SB];
+  for (int e0 = bent[b] + (int)((long long)ne * h / nsplit); e0 < e1; e0 += FT_LIST) {
+    // the first waves list the entries that reach the tile
+    if (wave < FT_LIST / 64) {
+      const int el = e0 + 64 * wave + lane;
+      FtEntry<SB> E;
+      E.pass = 0;
+      if (el < e1) {
+        const int* __restrict__ El = ent + (size_t)el * (1 + SB);
+        E.r = nsrc + El[0];
+        const float rl = tlo[(size_t)E.r * ntile + tile], rh = thi[(size_t)E.r * ntile + tile];
+#pragma unroll
+        for (int k = 0; k < SB; ++k) {
+          E.t[k] = El[1 + k];
+          if (E.t[k] < 0) continue;
+          const float lo = ms[k] + rl, hi = mh[k] + rh;
+          if (beyond(ms[k], rl, K)) continue;
+          E.cmp[k] = tcmp[E.t[k]];
+          if (ANGLE) E.bin[k] = tcid[E.t[k]];
+          // a NaN node's index is 0 and the lower bound NaN
+          E.lo[k] = lo != lo ? 0 : max(t_index(lo, K), 0);
+          E.len[k] = (lo != lo ? K.nt : min(t_index(hi, K) + 1, K.nt)) - E.lo[k];
+          if (E.len[k] <= 0) continue;  // every index negative
+          E.pass |= 1 << k;
+          // every sum in [2^-100, 2^100)
+          if (K.fastdiv_dt && lo >= 0x1p-100f && hi < 0x1p80f) E.pass |= 256 << k;
+        }
+      }
+      const uint64_t m = __ballot(E.pass != 0);
+      if (E.pass) list[64 * wave + (int)__popcll(m & ((1ull << lane) - 1))] = E;
+      if (lane == 0) count[wave] = (int)__popcll(m);
+    }
+    __syncthreads();
+    const int n0 = __builtin_amdgcn_readfirstlane(count[0]), n1 = __builtin_amdgcn_readfirstlane(count[1]);
+    if (!started && n0 + n1) {  // the first entry that reaches the tile
+      started = true;
+      for (int e = threadIdx.x; e < 2 * SB * FT_WIN; e += THREADS) (&win[0][0][0])[e] = 0.0;
+#pragma unroll
+      for (int n = 0; n < NPT; ++n) {
+        sS[n] = K.scale * S[(ic + 3) + (size_t)(min(j0 + n, K.nx - 1) + 3) * K.nzz];
+        if (!ANGLE) sS[n] *= model[p[n]];
+      }
+#pragma unroll
+      for (int k = 0; k < SB; ++k) {
+        const int sk = bsrc[b * SB + k];
+        if (sk < 0) continue;
+#pragma unroll
+        for (int n = 0; n < NPT; ++n) {
+          const bool live = i < K.nz && j0 + n < K.nx;
+          qs[n][k].t = live ? q[(size_t)sk * KQ * K.npts + p[n]] : FAR;
+          q_amp<KQ>(q, sk, p[n], K.npts, qs[n][k]);
+          qs[n][k].amp *= sS[n];
+          qs[n][k].ch *= 0.2f;
+          qs[n][k].sh *= -0.2f;
+          if (ANGLE) q_dir<KQ>(q, sk, p[n], K.npts, qs[n][k]);
+        }
+      }
+      __syncthreads();
+    }
+    for (int l = 0; l < n0 + n1; ++l) {
+      const FtEntry<SB>& E = list[l < n0 ? l : 64 + l - n0];
+      const int r = __builtin_amdgcn_readfirstlane(E.r), pass = __builtin_amdgcn_readfirstlane(E.pass);
+      Q7 qr[NPT];
+#pragma unroll
+      for (int n = 0; n < NPT; ++n) {
+        qr[n].t = q[(size_t)r * KQ * K.npts + p[n]];
+        q_amp<KQ>(q, r, p[n], K.npts, qr[n]);
+        if (ANGLE) q_dir<KQ>(q, r, p[n], K.npts, qr[n]);
+      }
+      bool more;
+      int done = 0;  // samples of the windows already flushed
+      do {
+        more = false;
+        // nothing of a pair is worth keeping in registers for another round
+#pragma unroll
+        for (int n = 0; n < NPT; ++n) asm volatile("" : "+v"(qr[n].t), "+v"(qr[n].amp), "+v"(qr[n].ch), "+v"(qr[n].sh));
+#pragma unroll
+        for (int k = 0; k < SB; ++k) {
+          if (!(pass >> k & 1)) continue;
+          const float cmp = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(E.cmp[k])));
+          const int lo = __builtin_amdgcn_readfirstlane(E.lo[k]) + done;
+          const int len = __builtin_amdgcn_readfirstlane(E.len[k]) - done;
+          more |= len > FT_WIN;
+          const unsigned lim = (unsigned)max(min(len, FT_WIN), 0);
+          const int cb = ANGLE ? __builtin_amdgcn_readfirstlane(E.bin[k]) : 0;
+#pragma unroll
+          for (int n = 0; n < NPT; ++n) {
+            const float xs = qs[n][k].t + qr[n].t;
+            const int it = (pass >> k & 256) ? (int)fdiv(xs, K.zh_dt, K.zl_dt) : t_index(xs, K);
+            const unsigned rel = (unsigned)(it - lo);
+            if (rel >= lim) continue;
+            const float rf = __builtin_fmaf(qs[n][k].ch, qr[n].ch, __builtin_fmaf(qs[n][k].sh, qr[n].sh, 1.0f));
+            float w = (qs[n][k].amp * qr[n].amp) * rf * kdm_taper<RDIV>(x[n], cmp, sig_e, r_sig);
+            if (ANGLE) {
+              const int a = kdm_angle_bin(qs[n][k], qr[n], K);
+              if ((unsigned)a >= (unsigned)K.nang) continue;
+              w *= model[ic + (size_t)a * K.nz + (size_t)cb * K.nang * K.nz];
+            }
+            atomicAdd(&win[par][k][rel], (double)w);
+          }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < SB; ++k) {
+          if (!(pass >> k & 1)) continue;
+          float* __restrict__ d = data + (size_t)E.t[k] * K.nt + E.lo[k] + done;
+          const int n = min(E.len[k] - done, FT_WIN);
+          for (int e = threadIdx.x; e < n; e += THREADS) {
+            const float v = (float)win[par][k][e];
+            if (v != 0.0f) {
+              atomicAdd(d + e, v);
+              win[par][k][e] = 0.0;
+            }
+          }
+        }
+        par ^= 1;
+        done += FT_WIN;
+      } while (more);
+    }
+    __syncthreads();  // the list is about to change
+  }
 }
 
 // Trace convolution: one thread per output sample.  Adjoint: out[k] =
@@ -753,6 +1010,13 @@ struct seisfat_kdm_s {
   float* d_tmin = nullptr; // per-table chunk minima of T, (nsrc + nrec) x nchunk
   float* d_tmin2 = nullptr; // per-table minima over 64 chunks, (nsrc + nrec) x nsup
   float* d_tmin3 = nullptr; // per-table minimum, nsrc + nrec
+  float* d_tlo = nullptr;   // tile bounds of the forward operator, (nsrc + nrec) x ntile each
+  float* d_thi = nullptr;
+  unsigned long long* d_cnt = nullptr;  // k_kdm_tile_count's sums
+  int ntz = 0, ntile = 0, tile_cols = 0;
+  bool bounds_dirty = true;  // tables or traces changed since the bounds and the choice below
+  bool by_tiles = false;     // the forward operator's kernel
+  int nsplit = 1;            // its workgroups per tile and source block (slices of the entries)
   int* d_nonneg = nullptr;  // k_kdm_rec_nonneg's answer
   int* d_src = nullptr;    // trace tables
   int* d_rec = nullptr;
@@ -859,7 +1123,17 @@ void launch_adjoint(seisfat_kdm_s* k, const float* d_data, float* d_model, hipSt
 
 template <bool ANGLE, bool RDIV>
 void launch_forward(seisfat_kdm_s* k, const float* d_model, float* d_data, hipStream_t st) {
-  const size_t lds = (size_t)k->K.nt * sizeof(float);
+  if (k->by_tiles) {
+    hipLaunchKernelGGL((k_kdm_forward_tile<ANGLE, KDM_SB, ft_npt(ANGLE), RDIV>),
+                       dim3(8 * k->nb * k->nsplit, (k->ntile + 7) / 8), dim3(64 * FT_WAVES), 0, st, k->d_q, k->d_tlo,
+                       k->d_thi, k->ntz, k->ntile, k->h->d_spad, k->d_bsrc, k->d_bent, k->d_ent, k->d_cmp, k->d_cid,
+                       k->nsplit, k->nsrc, d_model, d_data, k->K);
+    return;
+  }
+  const size_t lds = (size_t)k->K.nt * sizeof(double);
+  if (lds > 65536)  // at most 16384 samples: 128 of the 160 KB
+    (void)hipFuncSetAttribute((const void*)k_kdm_forward<ANGLE, RDIV>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              131072);
   hipLaunchKernelGGL((k_kdm_forward<ANGLE, RDIV>), dim3(k->ntr), dim3(KDM_FWD_THREADS), lds, st, k->d_q, k->d_tmin,
                      k->h->d_spad, k->d_src, k->d_rec, k->d_cmp, k->d_cid, k->d_tmin2, k->nsrc, d_model, d_data,
                      k->K);
@@ -955,6 +1229,12 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin2, (size_t)(nsrc + nrec) * K.nsup * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin3, (size_t)(nsrc + nrec) * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_nonneg, sizeof(int));
+  k->ntz = (K.nz + 63) / 64;
+  k->tile_cols = FT_WAVES * ft_npt(p->domain == SEISFAT_KDM_ANGLE);
+  k->ntile = k->ntz * ((K.nx + k->tile_cols - 1) / k->tile_cols);
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_tlo, (size_t)(nsrc + nrec) * k->ntile * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_thi, (size_t)(nsrc + nrec) * k->ntile * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_cnt, 2 * sizeof(unsigned long long));
   if (e == hipSuccess) {
     // exhaustive check of the known-divisor division by dt (every dividend of
     // magnitude in [2^-100, 2^100)) against IEEE division
@@ -978,6 +1258,9 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
     kfree(k->d_tmin2);
     kfree(k->d_tmin3);
     kfree(k->d_nonneg);
+    kfree(k->d_tlo);
+    kfree(k->d_thi);
+    kfree(k->d_cnt);
     delete k;
     return kfail(SEISFAT_ENOMEM, std::string("hipMalloc of the table quantities: ") + hipGetErrorString(e));
   }
@@ -1000,6 +1283,7 @@ int seisfat_kdm_set_tables(seisfat_kdm_t k, const float* d_src, const float* d_r
   std::fill(k->tab_set.begin(), k->tab_set.end(), 1);
   k->tabs_missing = 0;
   k->rec_dirty = true;
+  k->bounds_dirty = true;
   return SEISFAT_OK;
 }
 
@@ -1018,6 +1302,7 @@ int seisfat_kdm_set_table(seisfat_kdm_t k, int which, int index, const float* d_
     --k->tabs_missing;
   }
   if (which) k->rec_dirty = true;
+  k->bounds_dirty = true;
   return SEISFAT_OK;
 }
 
@@ -1028,6 +1313,42 @@ int ready(seisfat_kdm_s* k) {
   if (k->s_version != k->h->version)
     return kfail(SEISFAT_ESTATE, "the slowness changed since the tables were set (set them again)");
   if (k->tabs_missing) return kfail(SEISFAT_ESTATE, "tables not set (seisfat_kdm_set_tables / _set_table)");
+  return SEISFAT_OK;
+}
+
+// The forward operator's tile bounds and its choice between its two kernels,
+// once per tables and traces: it waits for two counts.  Where that cannot be
+// done (a stream under capture) the kernel that needs no bounds runs.  In units
+// of a wave's column and round (0.1 ns on the whole chip), a tile kernel's
+// workgroup costs FT_COST before its first round, and the trace kernel takes
+// 1.4 (tables that stay in the caches) to 3 units per column; either one needs
+// 512 workgroups to fill the chip.  The line lies at 1.6, so that the tiles are
+// taken only where they are surely no slower.  Measured, trace / tile kernel, ms:
+// 1001x1001, 3609 traces: nt 1001 0.25 / 0.67, 1401 0.55 / 0.99, 2001 1.44 / 1.33,
+// 4001 13.1 / 4.6, 8001 16.8 / 6.1; 501x701, 2424 traces of 1251 at 2 ms:
+// 1.68 / 1.05; 499x209, 820 traces of 425 at 4 ms: 0.163 / 0.210; 603x801 angle
+// domain, 2292 traces of 1501 at 2 ms: 6.2 / 3.2.
+constexpr double FT_COST = 400.0, FT_TRACE = 1.6;
+int derive_bounds(seisfat_kdm_s* k, hipStream_t st) {
+  if (!k->bounds_dirty) return SEISFAT_OK;
+  k->by_tiles = false;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  KHIP(hipStreamIsCapturing(st, &cap));
+  if (cap != hipStreamCaptureStatusNone) return SEISFAT_OK;
+  hipLaunchKernelGGL(k_kdm_tile_bounds, dim3((k->ntile + 3) / 4, std::min(k->nsrc + k->nrec, 65535)), dim3(256), 0, st,
+                     k->d_q, k->kq, k->nsrc + k->nrec, k->ntz, k->ntile, k->tile_cols, k->K, k->d_tlo, k->d_thi);
+  hipLaunchKernelGGL(k_kdm_clear, dim3(1), dim3(2), 0, st, k->d_cnt);
+  hipLaunchKernelGGL(k_kdm_tile_count, dim3(k->ntr), dim3(64), 0, st, k->d_tlo, k->d_thi, k->ntile, k->d_src, k->d_rec,
+                     k->nsrc, k->K, k->d_cnt);
+  KHIP(hipGetLastError());
+  unsigned long long n[2] = {0, 0};
+  KHIP(hipMemcpyAsync(n, k->d_cnt, sizeof(n), hipMemcpyDeviceToHost, st));
+  KHIP(hipStreamSynchronize(st));
+  const double wgs = (double)k->ntile * k->nb * k->nsplit;
+  const double by_tile = (k->tile_cols * (double)n[1] + FT_COST * wgs) / std::min(1.0, wgs / 512);
+  const double by_trace = FT_TRACE * k->tile_cols * (double)n[0] / std::min(1.0, k->ntr / 512.0);
+  k->by_tiles = by_tile < by_trace && k->ntile <= 8 * 65535 && 4096.0 * k->nb * k->nsplit < 0x1p32 && k->K.dt < 0x1p60f;
+  k->bounds_dirty = false;
   return SEISFAT_OK;
 }
 
@@ -1059,6 +1380,7 @@ int seisfat_kdm_set_traces(seisfat_kdm_t k, int ntr, const int* src, const int* 
   }
   KHIP(hipDeviceSynchronize());  // runs in flight may read the previous trace tables
   free_traces(k);
+  k->bounds_dirty = true;
   k->K.taper_rdiv = (k->taper_geom && std::all_of(cmp, cmp + ntr, cmp_ok)) ? 1 : 0;
   if (ntr == 0) return SEISFAT_OK;
   KHIP(hipMalloc((void**)&k->d_src, ntr * sizeof(int)));
@@ -1105,6 +1427,9 @@ int seisfat_kdm_set_traces(seisfat_kdm_t k, int ntr, const int* src, const int* 
   KHIP(hipMemcpy(k->d_bent, bent.data(), bent.size() * sizeof(int), hipMemcpyHostToDevice));
   KHIP(hipMemcpy(k->d_ent, ent.data(), ent.size() * sizeof(int), hipMemcpyHostToDevice));
   k->nb = nb;
+  // the forward's tiles: enough workgroups for the chip, at least 8 entries each
+  const long long wgs = (long long)k->ntile * nb, per_block = (long long)(ent.size() / (1 + KDM_SB)) / nb;
+  k->nsplit = (int)std::max<long long>(1, std::min((1024 + wgs - 1) / wgs, per_block / 8));
   // adjoint parts: up to KDM_PARTS, no more than the blocks; the image
   // domain's partial sums within 1 GiB
   int np = std::max(1, std::min(KDM_PARTS, nb));
@@ -1154,6 +1479,7 @@ int seisfat_kdm_forward(seisfat_kdm_t k, const float* d_model, float* d_data, vo
   if (const int rc = ready(k)) return rc;
   if (k->ntr == 0) return SEISFAT_OK;  // no traces to add into
   if (!d_data || !d_model) return kfail(SEISFAT_EINVAL, "null buffer");
+  if (const int rc = derive_bounds(k, st)) return rc;
   const bool rd = k->K.taper_rdiv != 0;
   if (k->p.domain == SEISFAT_KDM_IMAGE) {
     if (rd)
@@ -1178,6 +1504,9 @@ int seisfat_kdm_destroy(seisfat_kdm_t k) {
   kfree(k->d_tmin2);
   kfree(k->d_tmin3);
   kfree(k->d_nonneg);
+  kfree(k->d_tlo);
+  kfree(k->d_thi);
+  kfree(k->d_cnt);
   delete k;
   return SEISFAT_OK;
 }

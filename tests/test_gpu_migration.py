@@ -446,3 +446,47 @@ def test_convolution_block_edges(oracle, torch, adjoint, ntr, nt, nw):
                                                  C.c_void_p(out.data_ptr()),
                                                  C.c_void_p(torch.cuda.current_stream().cuda_stream)))
     assert np.array_equal(out.cpu().numpy(), oracle.trace_convolve(x, w, adjoint), equal_nan=True)
+
+
+# the forward's tile kernel at the edges of its tiles (64 rows, 16 or 8
+# columns), windows longer than its 1024 samples (several rounds), slices of a
+# block's entries, NaN and negative traveltimes (indices 0 and skipped), and the
+# trace kernel on the same survey under capture
+@pytest.mark.parametrize("domain", [mig.IMAGE, mig.ANGLE])
+@pytest.mark.parametrize("nz,nx,nt,dt,shift", [(63, 33, 400, 2e-3, 0.0), (64, 32, 400, 2e-3, 0.0), (65, 31, 16384, 2e-5, 0.0),
+                                               (130, 49, 3000, 2e-4, 0.0), (70, 40, 400, 1.5e-3, -0.05),
+                                               (70, 40, 500, 1.5e-3, np.nan)])
+def test_forward_tiles(oracle, torch, domain, nz, nx, nt, dt, shift):
+    m, xs, xr = survey(nz=nz, nx=nx, nsrc=9, nrec=60, seed=nz)
+    e = Eikonal(nz, nx, m.dz, m.dx)
+    e.set_slowness(m.s)
+    ts, tr = (e.traveltime_tables(x, np.full_like(x, 11.0)) for x in (xs, xr))
+    if np.isnan(shift):
+        ts[2, 20, 30], tr[5, 11, 40:43] = np.nan, np.nan
+    else:
+        tr += np.float32(shift)
+    K = make(e, m, xs, xr, domain, nt=nt, dt=dt, tables=(ts, tr), max_offset=1e4)
+    S = oracle.expand_boundary(m.s)
+    op = dict(dt=float(K.dt), dx=m.dx, dz=m.dz, aperture=30.0, da=float(K.da), nang=K.nang)
+    rng = np.random.default_rng(nz)
+    x = rng.standard_normal(K.model_shape).astype(np.float32)
+    d0 = (rng.standard_normal((K.ntr, nt)) * 1e-4).astype(np.float32)
+    cid = K.cmp_id if domain == mig.ANGLE else None
+    xd = torch.from_numpy(x).cuda()
+    K.adjoint(torch.zeros((K.ntr, nt), device="cuda"))
+    out = [torch.from_numpy(d0.copy()).cuda() for _ in range(2)]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        K.forward(xd, out[1])
+    K.forward(xd, out[0])
+    g.replay()
+    want = oracle.kdm(domain, False, S, ts, tr, K.src, K.rec, K.cmp, cid, d0.copy(), x, **op)
+    bound = oracle.kdm(domain, False, S, ts, tr, K.src, K.rec, K.cmp, cid, np.abs(d0), np.abs(x), **op)
+    fin = np.isfinite(want)
+    for got in out:
+        got = got.cpu().numpy()
+        assert np.array_equal(np.isfinite(got), fin)
+        bad = np.abs(got - want)[fin] > (1e-5 * bound + 1e-30)[fin]
+        assert bad.mean() <= (1e-3 if domain == mig.ANGLE else 0.0)
+    K.close()
+    e.close()
