@@ -65,10 +65,12 @@ struct KdmK {
   float zh_dt, zl_dt;  // two-word reciprocal of dt (fdiv)
   int fastdiv_dt;      // fdiv(x, zh_dt, zl_dt) == RN(x / dt) for every 2^-100 <= x < 2^100 (checked exhaustively)
   int taper_rdiv;      // (x - cmp) / sig_e needs no operand rescaling at any node and trace (kdm_weight)
-  float dx, dz, dt, da;
+  float dx, dz, dt;
   // k_kdm_prep's constant divisors and their reciprocals RN(1 / b)
   float dz2, dx2, dxz4, r_dz, r_dx, r_dz2, r_dx2, r_dxz4;
-  int prep_rdiv;        // they lie in [2^-44, 2^44]
+  int prep_rdiv;        // dz and dx lie in [2^-20, 2^20]
+  float da_m, r_da;     // da = da_m 2^da_e, da_m in [1, 2), and RN(1 / da_m)
+  int da_e;
   unsigned nz_recip;    // floor(2^32 / nz) (nz > 1)
   float ntf;     // (float)nt
   float tan_ap;  // tanf(aperture in radians), the reference's sigma / z
@@ -278,6 +280,10 @@ __device__ __forceinline__ void q_dir(const float* __restrict__ q, int tab, int 
   o.norm = b[(size_t)6 * npts];
 }
 
+// The index where every sum lies in [2^-100, 2^100) and the two-instruction
+// division by dt is proven.
+__device__ __forceinline__ int t_index_mid(float xs, const KdmK& K) { return (int)fdiv(xs, K.zh_dt, K.zl_dt); }
+
 // Time index of a node for a trace with traveltime sum xs, as far as the
 // kernels use it: the reference's tId = f2i_rd(RN(xs / dt)) where that lies in
 // [0, nt) or xs is NaN (0), a value >= nt or negative otherwise.  When every
@@ -290,13 +296,9 @@ __device__ __forceinline__ void q_dir(const float* __restrict__ q, int tab, int 
 __device__ __forceinline__ int t_index(float xs, const KdmK& K) {
   const bool mid = __float_as_uint(xs) - 0x0d800000u < 0x64000000u;  // 2^-100 <= xs < 2^100
   const uint64_t all_mid = __builtin_amdgcn_ballot_w64(mid);
-  if (K.fastdiv_dt && all_mid == __builtin_amdgcn_read_exec()) {
-    // min(RN(xs / dt), nt) of a positive finite quotient, nt from a scalar
-    // register (no NaN: the compiler's canonicalising fminf is not needed)
-    float v;
-    asm("v_min_f32 %0, %1, %2" : "=v"(v) : "s"(K.ntf), "v"(fdiv(xs, K.zh_dt, K.zl_dt)));
-    return (int)floorf(v);
-  }
+  // a positive finite quotient: truncation is the floor, and the conversion
+  // saturates (far beyond nt)
+  if (K.fastdiv_dt && all_mid == __builtin_amdgcn_read_exec()) return t_index_mid(xs, K);
   const float v = (K.fastdiv_dt && mid) ? fdiv(xs, K.zh_dt, K.zl_dt) : xs / K.dt;
   const int it = v != v ? 0 : (int)fminf(fmaxf(floorf(v), -1.0f), (float)K.nt);
   return xs >= K.thr ? K.nt : it;
@@ -314,31 +316,40 @@ __device__ __forceinline__ bool beyond(float a, float b, const KdmK& K) { return
 // the trace's CMP.  sS = S / (2 pi) and sig_e = sigma + EPS (with its refined
 // reciprocal r_sig) come in evaluated per node.  The taper is the reference's
 // expression and roundings: (x - cmp) / sig_e, by rdiv with the refined
-// reciprocal when the host found that no operand needs rescaling (RDIV, the
+// reciprocal and one correction when the host found that no operand needs
+// rescaling (RDIV, the
 // operator's taper_rdiv: every divisor in [EPS, 2^40), every dividend 0 or of
 // magnitude in [2^-59, 2^41)), then expf(-0.5 a a).
-// e^x for a finite x <= 0: 2^(x log2 e), x log2 e split into its rounded
-// product hi and the residual fma(x, L, -hi) + x Llo (L + Llo = log2 e), the
-// nearest integer n of hi applied by ldexp to the hardware 2^f of the
-// remaining f in [-0.5, 0.5].  The same instructions as the library's expf
-// without its overflow and non-finite handling: equal results for x >= -103.97;
-// below, x is clamped to -104 and the result is 0 or the least subnormals
-// (e^x < 2^-149 there).
-__device__ __forceinline__ float exp_nonpos(float x) {
+// e^(-y / 2) for a finite y >= 0: 2^(-y log2(e) / 2), the exponent split into
+// its rounded product hi and the residual fma(y, L, -hi) + y Llo (L + Llo =
+// -log2(e) / 2), the nearest integer n of hi applied by ldexp to the hardware
+// 2^f of the remaining f in [-0.5, 0.5].  (The factor -1/2 only scales: the
+// roundings are those of the exponential of x = -y / 2.)  y is clamped to 208,
+// where the result is 0 or the least subnormals.
+__device__ __forceinline__ float exp_mhalf(float y) {
 #pragma clang fp contract(off)  // hi - n must use the rounded hi: lo holds its residual
-  x = fmaxf(x, -104.0f);
-  const float hi = x * 0x1.715476p+0f;
-  const float lo = __builtin_fmaf(x, 0x1.4ae0bep-26f, __builtin_fmaf(x, 0x1.715476p+0f, -hi));
+  y = fminf(y, 208.0f);
+  const float hi = y * -0x1.715476p-1f;
+  const float lo = __builtin_fmaf(y, -0x1.4ae0bep-27f, __builtin_fmaf(y, -0x1.715476p-1f, -hi));
   const float n = __builtin_rintf(hi);
   return __builtin_ldexpf(__builtin_amdgcn_exp2f((hi - n) + lo), (int)n);
 }
 
+// The aperture taper of x about cmp: r_sig = RN(1 / sig_e).
 template <bool RDIV>
 __device__ __forceinline__ float kdm_taper(float x, float cmp, float sig_e, float r_sig) {
   const float n = x - cmp;
-  // RDIV: |a| < 2^61, so -0.5 a a is finite and <= 0
-  const float a = RDIV ? rdiv(n, sig_e, r_sig) : n / sig_e;
-  return RDIV ? exp_nonpos(-0.5f * a * a) : expf(-0.5f * a * a);
+  if (!RDIV) {
+    const float a = n / sig_e;
+    return expf(-0.5f * a * a);
+  }
+  // |a| < 2^61, so a a is finite and >= 0.  With r_sig the correctly rounded
+  // reciprocal one correction of q0 gives RN(n / sig_e) (see cdiv in
+  // eik_adjoint.hip; r_sig refined twice or not, the quotient is within
+  // 0.5 + 2^-22 ulp)
+  const float q0 = n * r_sig;
+  const float a = __builtin_fmaf(__builtin_fmaf(-sig_e, q0, n), r_sig, q0);
+  return exp_mhalf(a * a);
 }
 
 template <bool RDIV>
@@ -348,11 +359,34 @@ __device__ __forceinline__ float kdm_weight(const Q7& s, const Q7& r, float sS, 
   return sS * (s.amp * r.amp) * rf * kdm_taper<RDIV>(x, cmp, sig_e, r_sig);
 }
 
-// Reflection-angle bin of the node for the trace (the reference's aId).
+// The same with the factors of a node that do not depend on the receiver
+// already in the source's quantities (q_prefold): amp S / (2 pi), 0.2 ch and
+// -0.2 sh.
+__device__ __forceinline__ void q_prefold(Q7& s, float sS) {
+  s.amp *= sS;
+  s.ch *= 0.2f;
+  s.sh *= -0.2f;
+}
+template <bool RDIV>
+__device__ __forceinline__ float kdm_weight_pre(const Q7& s, const Q7& r, float x, float sig_e, float r_sig, float cmp) {
+  const float rf = __builtin_fmaf(s.ch, r.ch, __builtin_fmaf(s.sh, r.sh, 1.0f));
+  return (s.amp * r.amp) * rf * kdm_taper<RDIV>(x, cmp, sig_e, r_sig);
+}
+
+// Reflection-angle bin of the node for the trace (the reference's aId): the
+// bits of float division, float acosf, division by pi in double, float division
+// by da and rounding down (NaN -> 0), without the divisions' rescaling and
+// without branches.  The norms are at least EPS; v_div_fixup gives the quotient
+// of infinite and NaN operands.  The product with 1 / pi and one fma correction
+// is the double quotient (the FMA division theorem).  da = da_m 2^da_e, da_m in
+// [1, 2).
 __device__ __forceinline__ int kdm_angle_bin(const Q7& s, const Q7& r, const KdmK& K) {
-  const float ra = 0.5f * acosf((s.dx * r.dx + s.dz * r.dz) / (s.norm * r.norm));
-  const float ang = (float)((double)(180.0f * ra) / M_PI);
-  return f2i_rd(ang / K.da);
+  const float num = s.dx * r.dx + s.dz * r.dz, den = s.norm * r.norm;
+  const float c = __builtin_amdgcn_div_fixupf(rdiv(num, den, recip_refined(den)), den, num);
+  const double a = 180.0f * (0.5f * acosf(c)), q = a * (1.0 / M_PI);
+  const float ang = (float)__builtin_fma(__builtin_fma(-M_PI, q, a), 1.0 / M_PI, q);
+  const float v = __builtin_ldexpf(rdiv(ang, K.da_m, K.r_da), -K.da_e);
+  return (int)__builtin_amdgcn_fmed3f(v, 0.0f, 1e9f);  // (a NaN's median is the least of the others)
 }
 
 // Adjoint: thread per image point (a wave holds 64 consecutive points, one
@@ -410,7 +444,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
   const float z = (float)i * K.dz, x = (float)j * K.dx;
   const float sS = K.scale * S[(i + 3) + (size_t)(j + 3) * K.nzz];
   const float sig_e = K.tan_ap * z + KDM_EPS;
-  const float r_sig = recip_refined(sig_e);
+  const float r_sig = 1.0f / sig_e;
   float acc = (!ANGLE && live && nparts == 1) ? model[p] : 0.0f;
   for (int b = b_begin; b < b_end; ++b) {
     // slot k in use: bit k (one scalar register for the block)
@@ -446,6 +480,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
         const int sk = bsrc[b * SB + k];
         qs[k].t = q[(size_t)sk * KQ * K.npts + p];
         q_amp<KQ>(q, sk, p, K.npts, qs[k]);
+        q_prefold(qs[k], sS);
         if (ANGLE) q_dir<KQ>(q, sk, p, K.npts, qs[k]);
       }
     }
@@ -453,7 +488,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
       // lane l holds entry e0 + l (receiver, traces, receiver minimum) and
       // tests it: does any of its pairs pass the chunk test?  The entries that
       // pass are then taken one at a time, their words read from that lane.
-      int el_pass = 0;  // bit k: slot k holds a trace that passes the chunk test
+      // bit k: slot k holds a trace that passes the chunk test; bit 8 + k: with
+      // every sum of the chunk at least 2^-100 and no NaN
+      int el_pass = 0;
       int el_r = 0, el_t[SB], el_a[SB];
       float mr_l = 0.0f, el_c[SB];
 #pragma unroll
@@ -469,7 +506,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
         for (int k = 0; k < SB; ++k) el_t[k] = El[1 + k];
         mr_l = tmin[(size_t)el_r * K.nchunk + c];
 #pragma unroll
-        for (int k = 0; k < SB; ++k) el_pass |= (el_t[k] >= 0 && (use >> k & 1) && !beyond(ms[k], mr_l, K)) << k;
+        for (int k = 0; k < SB; ++k)
+          if (el_t[k] >= 0 && (use >> k & 1) && !beyond(ms[k], mr_l, K))
+            el_pass |= ((K.fastdiv_dt && ms[k] + mr_l >= 0x1p-100f) ? 257 : 1) << k;
         // the traces' CMP (and bin), read from this lane when the entry is taken
         if (el_pass) {
 #pragma unroll
@@ -516,7 +555,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
           tk[k] = __builtin_amdgcn_readlane(el_t[k], li);
           slots |= 1u << k;
           const float xs = qs[k].t + rt;
-          const int it = t_index(xs, K);
+          // (the clamp keeps the quotient finite; no sample lies beyond it, dt
+          // being at most 2^20 where the bit is used)
+          const int it = (pass >> k & 256) ? t_index_mid(fminf(xs, 0x1p99f), K) : t_index(xs, K);
           ok[k] = live && (unsigned)it < (unsigned)K.nt;
           // the trace's base (uniform) plus a 32-bit byte offset (it < nt <= 16384)
           const char* __restrict__ dk = (const char*)(data + (size_t)tk[k] * K.nt);
@@ -535,14 +576,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
         for (int k = 0; k < SB; ++k) {
           if (!(slots >> k & 1)) continue;
           const float cmp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(el_c[k]), li));
-          const float w = kdm_weight<RDIV>(qs[k], qr, sS, x, sig_e, r_sig, cmp);
+          const float w = kdm_weight_pre<RDIV>(qs[k], qr, x, sig_e, r_sig, cmp);
           if (ANGLE) {
             const int a = kdm_angle_bin(qs[k], qr, K);
             const int cb = __builtin_amdgcn_readlane(el_a[k], li);
             if (ok[k] && a >= 0 && a < K.nang)
               atomicAdd(model + i + (size_t)a * K.nz + (size_t)cb * K.nang * K.nz, w * dv[k]);
           } else {
-            acc += ok[k] ? w * dv[k] : 0.0f;
+            acc = __builtin_fmaf(ok[k] ? w : 0.0f, dv[k], acc);  // (dv is 0 where not ok)
           }
         }
       }
@@ -627,7 +668,7 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
         const float z = (float)i * K.dz, x = (float)j * K.dx;
         const float sS = K.scale * S[(i + 3) + (size_t)(j + 3) * K.nzz];
         const float sig_e = K.tan_ap * z + KDM_EPS;
-        const float w = kdm_weight<RDIV>(qs, qr, sS, x, sig_e, recip_refined(sig_e), cmp);
+        const float w = kdm_weight<RDIV>(qs, qr, sS, x, sig_e, 1.0f / sig_e, cmp);
         if (ANGLE) {
           const int a = kdm_angle_bin(qs, qr, K);
           if (a >= 0 && a < K.nang) atomicAdd(hist + it, (double)(w * model[moff + i + (size_t)a * K.nz]));
@@ -655,10 +696,10 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
 // and several hundred nodes to a sample, and double-buffered, so an entry needs
 // one barrier.  LDS sums are FP64: ds_add_f32 takes 169 cycles per wave
 // instruction on this chip whatever its addresses, ds_add_f64 8 to 20 (39 with
-// pairs of lanes on one address), and the sum is the more exact one.  Bound by
-// instruction issue (about 50 VALU per wave and pair).  1001 x 1001, 3609 traces
-// of 8001 samples: 6.1 ms, against 19.7 ms by trace with an FP32 histogram and
-// 16.8 with an FP64 one.
+// pairs of lanes on one address), and the sum is the more exact one.
+// 1001 x 1001, 3609 traces of 8001 samples: 5.7 ms (6.1 before the next entry's
+// receiver quantities were loaded one entry ahead), against 19.7 ms by trace
+// with an FP32 histogram and 16.8 with an FP64 one.
 constexpr int FT_WAVES = 8, FT_WIN = 1024, FT_LIST = 128;
 constexpr int ft_npt(bool angle) { return angle ? 1 : 2; }
 
@@ -749,7 +790,7 @@ __global__ __launch_bounds__(64 * FT_WAVES) void k_kdm_forward_tile(
   const int i = tile % ntz * 64 + lane, ic = min(i, K.nz - 1);
   const int j0 = tile / ntz * (FT_WAVES * NPT) + wave * NPT;
   const float sig_e = K.tan_ap * ((float)ic * K.dz) + KDM_EPS;
-  const float r_sig = recip_refined(sig_e);
+  const float r_sig = 1.0f / sig_e;
   int p[NPT];
   float x[NPT], sS[NPT];
 #pragma unroll
@@ -821,24 +862,32 @@ __global__ __launch_bounds__(64 * FT_WAVES) void k_kdm_forward_tile(
           const bool live = i < K.nz && j0 + n < K.nx;
           qs[n][k].t = live ? q[(size_t)sk * KQ * K.npts + p[n]] : FAR;
           q_amp<KQ>(q, sk, p[n], K.npts, qs[n][k]);
-          qs[n][k].amp *= sS[n];
-          qs[n][k].ch *= 0.2f;
-          qs[n][k].sh *= -0.2f;
+          q_prefold(qs[n][k], sS[n]);
           if (ANGLE) q_dir<KQ>(q, sk, p[n], K.npts, qs[n][k]);
         }
       }
       __syncthreads();
     }
-    for (int l = 0; l < n0 + n1; ++l) {
-      const FtEntry<SB>& E = list[l < n0 ? l : 64 + l - n0];
-      const int r = __builtin_amdgcn_readfirstlane(E.r), pass = __builtin_amdgcn_readfirstlane(E.pass);
-      Q7 qr[NPT];
+    // an entry's receiver quantities are loaded one entry ahead
+    const auto entry = [&](int l) { return l < n0 ? l : 64 + l - n0; };
+    Q7 qn[NPT];
+    const auto load = [&](int l) {
+      const int r = __builtin_amdgcn_readfirstlane(list[entry(min(l, n0 + n1 - 1))].r);
 #pragma unroll
       for (int n = 0; n < NPT; ++n) {
-        qr[n].t = q[(size_t)r * KQ * K.npts + p[n]];
-        q_amp<KQ>(q, r, p[n], K.npts, qr[n]);
-        if (ANGLE) q_dir<KQ>(q, r, p[n], K.npts, qr[n]);
+        qn[n].t = q[(size_t)r * KQ * K.npts + p[n]];
+        q_amp<KQ>(q, r, p[n], K.npts, qn[n]);
+        if (ANGLE) q_dir<KQ>(q, r, p[n], K.npts, qn[n]);
       }
+    };
+    if (n0 + n1) load(0);
+    for (int l = 0; l < n0 + n1; ++l) {
+      const FtEntry<SB>& E = list[entry(l)];
+      const int pass = __builtin_amdgcn_readfirstlane(E.pass);
+      Q7 qr[NPT];
+#pragma unroll
+      for (int n = 0; n < NPT; ++n) qr[n] = qn[n];
+      load(l + 1);
       bool more;
       int done = 0;  // samples of the windows already flushed
       do {
@@ -858,11 +907,10 @@ __global__ __launch_bounds__(64 * FT_WAVES) void k_kdm_forward_tile(
 #pragma unroll
           for (int n = 0; n < NPT; ++n) {
             const float xs = qs[n][k].t + qr[n].t;
-            const int it = (pass >> k & 256) ? (int)fdiv(xs, K.zh_dt, K.zl_dt) : t_index(xs, K);
+            const int it = (pass >> k & 256) ? t_index_mid(xs, K) : t_index(xs, K);
             const unsigned rel = (unsigned)(it - lo);
             if (rel >= lim) continue;
-            const float rf = __builtin_fmaf(qs[n][k].ch, qr[n].ch, __builtin_fmaf(qs[n][k].sh, qr[n].sh, 1.0f));
-            float w = (qs[n][k].amp * qr[n].amp) * rf * kdm_taper<RDIV>(x[n], cmp, sig_e, r_sig);
+            float w = kdm_weight_pre<RDIV>(qs[n][k], qr[n], x[n], sig_e, r_sig, cmp);
             if (ANGLE) {
               const int a = kdm_angle_bin(qs[n][k], qr[n], K);
               if ((unsigned)a >= (unsigned)K.nang) continue;
@@ -1218,7 +1266,9 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   K.zh_dt = 1.0f / p->dt;
   K.zl_dt = std::fma(-p->dt, K.zh_dt, 1.0f) / p->dt;
   K.fastdiv_dt = 0;
-  K.da = p->domain == SEISFAT_KDM_ANGLE ? p->da : 1.0f;
+  K.da_m = 2.0f * std::frexp(p->domain == SEISFAT_KDM_ANGLE ? p->da : 1.0f, &K.da_e);
+  K.da_e -= 1;
+  K.r_da = 1.0f / K.da_m;
   // sigma = tanf(aperture * pi / 180) * z, the angle rounded to float as the
   // reference's float argument takes it; 1 / (2 pi) rounded from double
   K.tan_ap = std::tan((float)((double)p->aperture * M_PI / 180.0));
@@ -1250,7 +1300,7 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
     }
     if (e == hipSuccess) e = hipMemcpy(&bad, d + 3, sizeof(int), hipMemcpyDeviceToHost);
     if (d) (void)hipFree(d);
-    K.fastdiv_dt = (e == hipSuccess && bad == 0) ? 1 : 0;
+    K.fastdiv_dt = (e == hipSuccess && bad == 0 && mid(K.dt)) ? 1 : 0;  // (and no quotient overflows)
   }
   if (e != hipSuccess) {
     kfree(k->d_q);
