@@ -61,8 +61,8 @@ void launch_fwd64_init(const AdjShot* shots, int nshots, int nzz, double dx, dou
 // walk_x: nshots * nstr * ldx exchange words (ldx >= 2 * nxx); tag: a value
 // no earlier launch on the same walk_x used
 void launch_fwd64_sweep(int sweep, const AdjShot* shots, int nshots, int nzz, int nstr, double dx, double dz,
-                        const double* Told, double* Tnew, int* walk_ctl, unsigned long long* walk_x, int ldx,
-                        unsigned tag, hipStream_t st);
+                        const SkewView& skew, const double* Told, double* Tnew, int* walk_ctl,
+                        unsigned long long* walk_x, int ldx, unsigned tag, hipStream_t st);
 // Picks of the fp64 trajectory's final traveltimes (rx, rz relative to each
 // receiver's shot grid).
 void launch_picks64(const AdjShot* shots, const int* rec_shot, const float* rx, const float* rz, int nrec, int nzz,

@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "eik_adjoint.h"
 
@@ -43,7 +44,7 @@ __global__ void k_adj_seed(const size_t* __restrict__ node, const int* __restric
 // the fp64 map (and finite differences of it) has.  Decisions and partials
 // are taken from the fp64 trajectory; the adjoint recurrence runs in fp32.
 struct ConstsD {
-  double dx, dz, dx2i, dz2i, sum, prod, hyp;
+  double dx, dz, dx2i, dz2i, sum, sum4, prod, hyp;
   double r_dx, r_dz, r_sum, r_hyp;  // RN(1/divisor), for cdiv
 };
 
@@ -75,29 +76,6 @@ __device__ __forceinline__ float dpp_shl1f(float old, float src) {
                                                     false));
 }
 
-// The local solver (src/modeling/modeling.cu:308-357) in fp64, operation for
-// operation as the fp64 oracle evaluates it.
-__device__ __forceinline__ double local_d(double tv, double te, double tev, double sref, double szo, double sxo,
-                                          const ConstsD& k) {
-  const double t1d1 = tv + k.dz * fmin(sref, szo);
-  const double t1d2 = te + k.dx * fmin(sref, sxo);
-  const double t1D = fmin(t1d1, t1d2);
-  double t2D = 1e6;
-  if ((tv <= te + k.dx * sref) && (te <= tv + k.dz * sref) && (te - tev >= 0.0) && (tv - tev >= 0.0)) {
-    const double ta = tev + te - tv;
-    const double tb = tev - te + tv;
-    t2D = cdiv((tb * k.dz2i + ta * k.dx2i) + sqrt(4.0 * sref * sref * k.sum - k.prod * (ta - tb) * (ta - tb)), k.sum,
-               k.r_sum);
-  } else if ((te - tev <= cdiv(sref * k.dz * k.dz, k.hyp, k.r_hyp)) && (te - tev > 0.0)) {
-    const double q = cdiv(te - tev, k.dz, k.r_dz);
-    t2D = te + k.dx * sqrt(sref * sref - q * q);
-  } else if ((tv - tev <= cdiv(sref * k.dx * k.dx, k.hyp, k.r_hyp)) && (tv - tev > 0.0)) {
-    const double p = cdiv(tv - tev, k.dx, k.r_dx);
-    t2D = tv + k.dz * sqrt(sref * sref - p * p);
-  }
-  return fmin(t1D, fmin(t2D, 1e6));
-}
-
 // time_set + time_init in fp64 (T0 holds 1e6 elsewhere for good).
 __global__ void k_fwd64_init(const AdjShot* __restrict__ shots, int nshots, int nzz, double dx, double dz,
                              double* __restrict__ T0) {
@@ -114,30 +92,118 @@ __global__ void k_fwd64_init(const AdjShot* __restrict__ shots, int nshots, int 
   T0[sh.toff + zi + (size_t)xi * nzz] = (double)s_at(sh.sd, nzz, zi, xi) * sqrt(ddx * ddx + ddz * ddz);
 }
 
+// Minimum of two doubles, neither a NaN (no quieting of loaded operands).
+__device__ __forceinline__ double vmin_d(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// sqrt(x) for a normal x whose root needs no rescaling: the hardware estimate
+// of 1 / sqrt(x) and the coupled iteration for the root and half its
+// reciprocal (Markstein), with two residual corrections: IEEE's root.
+__device__ __forceinline__ double sqrt_rn_d(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// What the local solver derives from the reference cell, evaluated when the
+// cell is first read (as the previous step's z-other cell).
+struct CellD {
+  double dzs, dxs, s2, s4, thrB, thrC;
+};
+
+__device__ __forceinline__ double thr_b(double s, const ConstsD& k) { return cdiv(k.dz * s * k.dz, k.hyp, k.r_hyp); }
+
+template <bool EQH>
+__device__ __forceinline__ CellD cell_d(double s, double thrB, const ConstsD& k) {
+  CellD c;
+  c.dzs = k.dz * s;
+  c.dxs = EQH ? c.dzs : k.dx * s;
+  c.s2 = s * s;
+  c.s4 = c.s2 * k.sum4;  // (4s s) sum: the factors of 4 only scale
+  c.thrB = thrB;
+  c.thrC = EQH ? thrB : cdiv(c.dxs * k.dx, k.hyp, k.r_hyp);
+  return c;
+}
+
+// The local solver (src/modeling/modeling.cu:308-357) in fp64, operation for
+// operation as the fp64 oracle evaluates it, and its minimum with told, without
+// branches: every lane evaluates all candidates and the values of branches not
+// taken are selected away; branches A, B and C share one square root.  Its radicand is positive wherever it is used (A: the
+// difference of the upwind times is at most a cell's edge time; B, C: the
+// threshold keeps q below s) and, with the validated slowness, far from the
+// range that needs rescaling.  h min(a, b) = min(h a, h b) for h > 0.
+template <bool EQH>
+__device__ __forceinline__ double local_sel_d(double tv, double te, double tev, const CellD& r, double dz_zo,
+                                              double dx_xo, double told, const ConstsD& k) {
+  const double t1d = vmin_d(tv + vmin_d(r.dzs, dz_zo), te + vmin_d(r.dxs, dx_xo));
+  const double de = te - tev, dv = tv - tev;
+  // Every condition is one compare whose mask goes straight to the selects (a
+  // mask combined on the scalar unit costs the step two crossings).  Branch A's
+  // four: a difference of doubles rounds to zero only when it is zero, so
+  // RN(a - b) >= 0 exactly when a >= b, and the minimum is >= 0 when all are.
+  const bool cA = vmin_d(vmin_d((te + r.dxs) - tv, (tv + r.dzs) - te), vmin_d(de, dv)) >= 0.0;
+  // 0 < d <= thr (thr > 0): positive doubles order as their bits, and zeros and
+  // negatives less one are at least as large as any positive double's
+  const bool cB = (unsigned long long)__double_as_longlong(de) - 1 < (unsigned long long)__double_as_longlong(r.thrB);
+  const bool cC = (unsigned long long)__double_as_longlong(dv) - 1 < (unsigned long long)__double_as_longlong(r.thrC);
+  const double ta = tev + te - tv, tb = tev - te + tv, dab = ta - tb;
+  const double dd = cB ? de : dv;
+  const double q = EQH ? cdiv(dd, k.dz, k.r_dz) : cdiv(dd, cB ? k.dz : k.dx, cB ? k.r_dz : k.r_dx);
+  double radA = r.s4 - k.prod * dab * dab, radBC = r.s2 - q * q;
+  asm("" : "+v"(radA), "+v"(radBC));  // both evaluated: no branch around either
+  const double root = sqrt_rn_d(cA ? radA : radBC);
+  double vA = cdiv((tb * k.dz2i + ta * k.dx2i) + root, k.sum, k.r_sum);
+  double vBC = (cB ? te : tv) + (EQH ? k.dz : cB ? k.dx : k.dz) * root;
+  asm("" : "+v"(vA), "+v"(vBC));
+  double two = cC ? vBC : 1e6;
+  two = cB ? vBC : two;
+  two = cA ? vA : two;
+  return vmin_d(vmin_d(t1d, told), two);  // (told <= 1e6 already)
+}
+
 // One fp64 sweep, Tnew = sweep(Told), out of place (ring nodes of Tnew hold
-// 1e6 for good).  A wave walks one strip of 64 sweep-local rows of one shot;
-// lane k holds row 64r + k and visits column t - k at step t: its z-upwind
-// and diagonal neighbours are lane k-1's results one and two steps back (DPP
-// shift), its x-upwind neighbour its own previous result, and lane 0 reads
-// the previous strip's last row from Tnew.  Inputs are loaded ADJ_PF steps
-// ahead.
+// 1e6 for good).  A workgroup walks one strip of 64 sweep-local rows of one
+// shot.  Its first wave computes: lane k holds row 64r + k and visits column
+// t - k at step t; its z-upwind and diagonal neighbours are lane k-1's results
+// one and two steps back (DPP shift), its x-upwind neighbour its own previous
+// result.  Traveltimes pass through an LDS ring of WK_R columns, which the
+// second and third wave fill and empty by whole columns (contiguous rows, as
+// global memory holds them): every step's 64 nodes lie in 64 different columns,
+// and a wave that loads and stores them itself touches 64 cache lines three
+// times a step (that version took 1.1 ms for 640 independent strips of 1207
+// columns against 0.47 ms for one alone, and 1.35 ms for 128 shots of 5
+// dependent strips).  In the ring the nodes of one step are 64 words of
+// different banks; results replace the old values in place.  Blocks of WK_B
+// steps end with one barrier; the column waves load two blocks ahead.
+// The first wave's step is bound by its instruction count (about 83, one in
+// four cycles) and the traveltime chain; a sweep of 128 shots of 307 x 1207
+// nodes takes 0.38 ms (1.20-1.36 before), one shot alone 0.29 (0.65), one strip
+// 0.23 (0.47).
 //
-// The strips of a shot run concurrently, each trailing the one above: lane
-// 0's upwind inputs are the upper strip's lane-63 results (its last row), which
-// that strip publishes as it computes them, column by column, each double as
-// two 64-bit words (one 32-bit half + the launch's tag in the high half),
-// written and read as single agent-scope atomics: a reader that sees the tag
-// in both words has the value, with no fence on either side.  The wave
-// fetches the words of a block of ADJ_PF steps in one load (lane u holds step
-// u's), one block ahead, takes step s's from its lane, and, while a tag is
-// stale, polls that column again (bounded: past the limit it sets the flag and
-// stops waiting for the rest of the strip, so a broken dependency cannot stall
-// the device).  Lane 0's diagonal input is
-// its previous step's upwind value (the ring column 0 holds 1e6).  Strips are
-// claimed from a ticket counter strip-major (every shot's strip r before any
-// strip r+1), so a strip's upper neighbour always holds a smaller ticket and
-// is running: the walk drains for any number of resident waves.
+// The strips of a shot run concurrently, each trailing the one above: lane 0's
+// upwind inputs are the upper strip's lane-63 results (its last row), which the
+// upper strip's column waves publish as they empty the ring, each double as two
+// 64-bit words (one 32-bit half + the launch's tag in the high half), written
+// and read as single agent-scope atomics: a reader that sees the tag in both
+// words has the value, with no fence on either side.  The fourth wave polls the
+// next block's words (bounded: past the limit it sets the flag and stops
+// waiting for the rest of the strip, so a broken dependency cannot stall the
+// device) and hands them to the first through LDS, with the slowness cells
+// below the strip's last row.  Strips are claimed from a ticket counter
+// strip-major (every shot's strip r before any strip r+1), so a strip's upper
+// neighbour always holds a smaller ticket and is running: the walk drains for
+// any number of resident workgroups.
 constexpr int WALK_SPIN = 1 << 16;
+constexpr int WK_B = 8;             // steps per block
+constexpr int WK_R = 64 + 2 * WK_B;  // ring columns: a step's 64, a block arriving, a block leaving
+constexpr int WK_C = WK_B / 2;       // columns per block and column wave
 
 __global__ void k_walk_begin(int* __restrict__ ctl) {
   if (threadIdx.x == 0) ctl[0] = 0;
@@ -147,150 +213,238 @@ __device__ __forceinline__ unsigned long long walk_word(unsigned half, unsigned 
   return ((unsigned long long)tag << 32) | half;
 }
 
+// Workgroup barrier after this wave's LDS operations (its global ones may stay
+// in flight).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The slowness cell that lane k of strip r (k = 64: the row below it) reads as
+// its z-other cell at local column c: s_at's row, and its column clamped to the
+// cells and to the shot's view in one median.  Byte offsets (below 2^32: at most
+// 2^30 padded nodes) from the uniform base.
 template <int SA, int SB>
-__global__ __launch_bounds__(64) void k_fwd64_sweep(const AdjShot* __restrict__ shots, int nshots, int nzz,
-                                                    int nstr, ConstsD K, const double* __restrict__ Told,
-                                                    double* __restrict__ Tnew, int* __restrict__ ctl,
-                                                    unsigned long long* __restrict__ xw, int ldx, unsigned tag) {
+struct ZoCell {
+  typedef __attribute__((address_space(1))) const char gchar;
+  gchar* base;
+  unsigned row, pitch;
+  int first, hi;
+  __device__ ZoCell(const ShotDev& sd, int nzz, int fi) {
+    const int f = min(max(fi, 1), nzz - 1);
+    base = (gchar*)sd.sbase;
+    row = 4u * (unsigned)((SA > 0 ? f : nzz - 1 - f) - (SA + 1) / 2);
+    pitch = 4u * (unsigned)nzz;
+    first = (SB > 0 ? 0 : sd.nxx - 2) - sd.sofs;
+    hi = min(max(sd.nxx - 2 - sd.sofs, 0), sd.smax);
+  }
+  __device__ unsigned offset(int c) const {
+    return row + (unsigned)min(max(SB > 0 ? first + c : first - c, 0), hi) * pitch;
+  }
+  __device__ float at_offset(unsigned o) const { return *(__attribute__((address_space(1))) const float*)(base + o); }
+  __device__ float at(int c) const { return at_offset(offset(c)); }
+  // no column from c0 to c1 is clamped
+  __device__ bool plain(int c0, int c1) const {
+    return SB > 0 ? first + c0 >= 0 && first + c1 <= hi : first - c1 >= 0 && first - c0 <= hi;
+  }
+};
+
+template <int SA, int SB, bool EQH>
+__global__ __launch_bounds__(256) void k_fwd64_sweep(const AdjShot* __restrict__ shots, int nshots, int nzz,
+                                                    int nstr, ConstsD K, SkewView sk,
+                                                    const double* __restrict__ Told, double* __restrict__ Tnew,
+                                                    int* __restrict__ ctl, unsigned long long* __restrict__ xw,
+                                                    int ldx, unsigned tag) {
   typedef __attribute__((address_space(1))) unsigned long long gword;
-  const int lane = threadIdx.x;
+  // column c, row k lies at ring[((c + k) mod WK_R) * 64 + k]: the nodes of step
+  // c + k are 64 consecutive words
+  __shared__ double ring[WK_R * 64];
+  __shared__ double thr_l[2][WK_B][64];  // a block's z-other cells: branch B's threshold
+  __shared__ float s_l[2][WK_B][66];     // and slowness (lane 64: the row below the strip)
+  __shared__ double xup_l[2][WK_B];      // upper strip's last row, columns of a block's steps
+  __shared__ int ticket;
+  const int lane = threadIdx.x & 63;
+  // (the hardware starts each workgroup of a CU on another SIMD, so the compute
+  // waves of up to four share none)
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (;;) {
-    int tk = 0;
-    if (lane == 0) tk = atomicAdd(ctl, 1);
-    tk = __builtin_amdgcn_readfirstlane(tk);
+    if (threadIdx.x == 0) ticket = atomicAdd(ctl, 1);
+    __syncthreads();
+    const int tk = __builtin_amdgcn_readfirstlane(ticket);
     if (tk >= nshots * nstr) break;
     const int r = tk / nshots, ks = tk - r * nshots;
     const AdjShot sh = shots[ks];
     const int nxx = sh.sd.nxx;
-    const double* __restrict__ To = Told + sh.toff;
-    double* __restrict__ Tn = Tnew + sh.toff;
-    const int NT = (nxx + 63 + 2 * ADJ_PF - 1) / (2 * ADJ_PF) * (2 * ADJ_PF);  // whole block pairs
+    const int NBLK = (nxx + 63 + WK_B - 1) / WK_B;
     // this strip's published last row, and the upper strip's
     gword* xme = (gword*)(xw + ((size_t)ks * nstr + r) * ldx);
     const gword* xup = (const gword*)(xw + ((size_t)ks * nstr + max(r - 1, 0)) * ldx);
-    const bool pub = lane == 63 && r + 1 < nstr;
-    // the upper strip's row (lane 0's upwind values): the loads, the tag test
-    // and the wait are wave-uniform
-    const bool up = r > 0;
     const int fi = 64 * r + lane;
     const bool row_int = fi >= 1 && fi <= nzz - 2;
-    const int fic = min(max(fi, 1), nzz - 2);
-    const int i = SA > 0 ? fic : nzz - 1 - fic;
-    double qto[ADJ_PF];
-    float qsz[ADJ_PF];
-    // Inputs of step t: the old value at clamped (always valid) coordinates
-    // and the z-other cell (i1, j1 + SB), one load per step.  The reference
-    // cell (i1, j1) is the previous step's z-other cell and the x-other cell
-    // (i1 + SA, j1) is lane k+1's z-other cell of the same step (one DPP
-    // move; lane 63's, in the next strip, arrives with the word blocks), so
-    // the z-other cell's row and column are clamped to the cell range only,
-    // keeping those identities for every interior node.
-    const int fis = min(max(fi, 1), nzz - 1);
-    const int is1 = (SA > 0 ? fis : nzz - 1 - fis) - (SA + 1) / 2;
-    auto load = [&](int t, double& to, float& sz) {
-      const int fjc = min(max(t - lane, 1), nxx - 2);
-      const int j = SB > 0 ? fjc : nxx - 1 - fjc;
-      to = To[i + (size_t)j * nzz];
-      const int fjs = min(max(t - lane, 0), nxx - 2);
-      sz = s_at(sh.sd, nzz, is1, (SB > 0 ? fjs : nxx - 1 - fjs) - (SB + 1) / 2 + SB);
-    };
-    // the upper strip's words of steps tb..tb+ADJ_PF-1, one block load: lane
-    // u (mod ADJ_PF) holds step tb+u's (column clamp(tb+u, 1, nxx-2)).
-    // Unconditional (strip 0 reads its own words and ignores them), so no
-    // branch forces a wait for it.
-    // With each block, lane 63's x-other cells: the z-other cells of a
-    // virtual lane 64 (row 64r+64, column t-64).
-    const int f64 = min(64 * r + 64, nzz - 1);
-    const int i64 = (SA > 0 ? f64 : nzz - 1 - f64) - (SA + 1) / 2;
-    auto xload = [&](int tb, unsigned long long& h, unsigned long long& l, float& x63) {
-      const int tt = tb + (lane & (ADJ_PF - 1));
-      const int fjx = min(max(tt, 1), nxx - 2);
-      h = __hip_atomic_load(xup + 2 * fjx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      l = __hip_atomic_load(xup + 2 * fjx + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const int fjs = min(max(tt - 64, 0), nxx - 2);
-      x63 = s_at(sh.sd, nzz, i64, (SB > 0 ? fjs : nxx - 1 - fjs) - (SB + 1) / 2 + SB);
-    };
+    // block n: the compute wave takes steps 8n .. 8n + 7; the others bring what
+    // block n + 1 reads.  (Blocks -1 and NBLK, NBLK + 1 only move data.)
+    if (wave == 0) {
+      double prev = 1e6, tev = 1e6;
+      CellD ref = cell_d<EQH>(1.0, 1.0, K);  // the previous step's z-other cell (unused at step 0)
+      const auto block = [&](int t0, int buf, auto edge) {
+        double* __restrict__ rg = ring + (t0 % WK_R) * 64 + lane;
+        unsigned zero = 0;
+        asm volatile("" : "+v"(zero));  // (one address register for the block's broadcasts)
+        // a step's operands are read one step ahead
+        double told = rg[0], gv = xup_l[buf][zero], thr = thr_l[buf][0][lane];
+        float szo = s_l[buf][0][lane], sxo = s_l[buf][0][lane + 1];
 #pragma unroll
-    for (int u = 0; u < ADJ_PF; ++u) load(u, qto[u], qsz[u]);
-    double prev = 1e6, prev2 = 1e6, gv_prev = 1e6;
-    float sref = 0.0f;  // the previous step's z-other cell (unused at step 0)
-    bool gave_up = false;
-    // ADJ_PF steps from t0 with the upper strip's words in (xh, xl).  Each
-    // step reloads its queue slot after its last use of the slot (and the
-    // caller each word block after its block), so a slot keeps its register
-    // across the loop and no copy waits for a load in flight.
-    auto block = [&](int t0, unsigned long long xh, unsigned long long xl, float x63) {
+        for (int u = 0; u < WK_B; ++u) {
+          const double told_u = told, thr_u = thr;
+          const float szo_u = szo, sxo_u = sxo;
+          // z-upwind: lane k-1's last result (lane 0: the upper strip's); the
+          // diagonal one was it a step ago
+          const double tv = dpp_shr1_d(gv, prev);
+          if (u + 1 < WK_B) {
+            told = rg[64 * (u + 1)];
+            gv = xup_l[buf][zero + u + 1];
+            thr = thr_l[buf][u + 1][lane];
+            szo = s_l[buf][u + 1][lane];
+            sxo = s_l[buf][u + 1][lane + 1];
+          }
+          const CellD next = cell_d<EQH>((double)szo_u, thr_u, K);
+          double out = local_sel_d<EQH>(tv, prev, tev, ref, next.dzs, K.dx * (double)sxo_u, told_u, K);
+          ref = next;
+          const int fj = t0 + u - lane;
+          if (!(row_int && (!edge.value || (fj >= 1 && fj <= nxx - 2)))) out = 1e6;
+          rg[64 * u] = out;
+          tev = tv;
+          prev = out;
+        }
+      };
+      lds_barrier();  // block -1
+      for (int n = 0; n < NBLK; ++n) {
+        const int t0 = n * WK_B;
+        if (t0 >= 64 && t0 + WK_B - 1 <= nxx - 2)
+          block(t0, n & 1, std::false_type());
+        else
+          block(t0, n & 1, std::true_type());
+        lds_barrier();
+      }
+      lds_barrier();
+      lds_barrier();
+    } else if (wave < 3) {
+      const double* __restrict__ To = Told + sh.toff;
+      double* __restrict__ Tn = Tnew + sh.toff;
+      const int fic = min(max(fi, 1), nzz - 2);
+      const int i = SA > 0 ? fic : nzz - 1 - fic;
+      const int c_off = (wave - 1) * WK_C;  // this wave's columns of a block
+      const auto col = [&](int fj) { return (size_t)(SB > 0 ? fj : nxx - 1 - fj) * nzz; };
+      const auto load = [&](int c, double& v) { v = (To + col(min(max(c, 1), nxx - 2)))[(unsigned)i]; };
+      double qa[WK_C], qb[WK_C];
 #pragma unroll
-      for (int u = 0; u < ADJ_PF; ++u) {
-        const int t = t0 + u;
-        double gv = 0.0, ge = 0.0;
-        if (up) {
-          // upper strip's value of column clamp(t, 1, nxx-2), published at its step t+63
-          const int fjc = min(max(t, 1), nxx - 2);
-          unsigned hw = __builtin_amdgcn_readlane((unsigned)xh, u);
-          unsigned ht = __builtin_amdgcn_readlane((unsigned)(xh >> 32), u);
-          unsigned lw = __builtin_amdgcn_readlane((unsigned)xl, u);
-          unsigned lt = __builtin_amdgcn_readlane((unsigned)(xl >> 32), u);
-          for (int it = 0; !gave_up && (ht != tag || lt != tag); ++it) {
+      for (int u = 0; u < WK_C; ++u) load(c_off + u, qa[u]);
+#pragma unroll
+      for (int u = 0; u < WK_C; ++u) load(WK_B + c_off + u, qb[u]);
+      const bool pub = lane == 63 && r + 1 < nstr;
+      // during block n: columns 8n + 8 .. 8n + 15 arrive in the words of columns
+      // 8n - 72 .. 8n - 65, whose last node block n - 1 computed
+      const auto move = [&](int n, double (&q)[WK_C]) {
+        const int c_in = (n + 1) * WK_B + c_off, c_out = c_in - WK_R;
+        double done[WK_C];
+        unsigned o[WK_C];
+#pragma unroll
+        for (int u = 0; u < WK_C; ++u) {
+          o[u] = (unsigned)(c_in % WK_R + u + lane);  // (WK_C divides WK_R: below 2 WK_R)
+          o[u] = min(o[u], o[u] - WK_R) * 64 + lane;
+          done[u] = ring[o[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < WK_C; ++u) ring[o[u]] = q[u];
+#pragma unroll
+        for (int u = 0; u < WK_C; ++u) {
+          const int fj = c_out + u;
+          if (pub && fj >= 1 && fj <= nxx - 2) {
+            __hip_atomic_store(xme + 2 * fj, walk_word((unsigned)__double2hiint(done[u]), tag), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(xme + 2 * fj + 1, walk_word((unsigned)__double2loint(done[u]), tag), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < WK_C; ++u) {
+          const int fj = c_out + u;
+          if (row_int && fj >= 1 && fj <= nxx - 2) (Tn + col(fj))[(unsigned)i] = done[u];
+        }
+#pragma unroll
+        for (int u = 0; u < WK_C; ++u) load(c_in + 2 * WK_B + u, q[u]);
+      };
+      // NBLK + 3 blocks, in pairs (a block past the last moves nothing of the grid)
+      for (int n = -1; n < NBLK + 2; n += 2) {
+        move(n, qa);
+        lds_barrier();
+        if (n + 1 < NBLK + 2) {
+          move(n + 1, qb);
+          lds_barrier();
+        }
+      }
+    } else {
+      const ZoCell<SA, SB> zo(sh.sd, nzz, fi), zo64(sh.sd, nzz, 64 * r + 64);
+      bool gave_up = false;
+      // the cells of steps 8(n + 1) .., one block ahead (lane u: the row below
+      // the strip at step u)
+      float q[WK_B], q64;
+      // Away from the clamped columns they come from the model's skewed copy
+      // (see SkewView): cell row kap = f - 1 of lane k >= 1 has kap mod 64 =
+      // k - 1, so the cells of one step share a skewed column; lane 0's (row
+      // 64r - 1) lie 64 columns further along the sweep (1 in strip 0, whose row
+      // 0 reads cell row 0).  64 lines a step without it: the strips of a shot
+      // then wait for one another (1.5 times the time of one strip alone with
+      // three workgroups on a CU).
+      const int kap = min(max(fi, 1), nzz - 1) - 1;
+      const int lead = lane > 0 ? 0 : r > 0 ? 64 : 1;
+      const unsigned lane_off = 4u * (unsigned)(kap + (SB > 0 ? lead : 64 - lead) * sk.KP);
+      const auto load = [&](int t0) {
+        if (sk.base && zo.plain(t0 - 64, t0 + WK_B - 1)) {
+          const int sig = sh.sd.x0 + sh.sd.sofs + (SB > 0 ? zo.first + t0 - 1 : zo.first - t0);
+          typedef __attribute__((address_space(1))) const char gchar;
+          gchar* b = (gchar*)(sk.base + (size_t)(sig + SK_OFF) * sk.KP);
+#pragma unroll
+          for (int u = 0; u < WK_B; ++u)
+            q[u] = *(__attribute__((address_space(1))) const float*)(b + (long long)(SB * u) * sk.KP * 4 + lane_off);
+        } else {
+#pragma unroll
+          for (int u = 0; u < WK_B; ++u) q[u] = zo.at(t0 + u - lane);
+        }
+        q64 = zo64.at(t0 + (lane & (WK_B - 1)) - 64);
+      };
+      load(0);
+      for (int n = -1; n < NBLK + 2; ++n) {
+        const int t = (n + 1) * WK_B + (lane & (WK_B - 1)), buf = (n + 1) & 1;
+        // the upper strip's value of column clamp(t, 1, nxx-2) (strip 0 has no
+        // upper strip: its first row is the ring)
+        const int fjc = min(max(t, 1), nxx - 2);
+        double v = 1e6;
+        if (r > 0 && n + 1 < NBLK) {
+          for (int it = 0;; ++it) {
+            const unsigned long long hw = __hip_atomic_load(xup + 2 * fjc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long lw =
+                __hip_atomic_load(xup + 2 * fjc + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v = __hiloint2double((int)(unsigned)hw, (int)(unsigned)lw);
+            if (gave_up || __all((unsigned)(hw >> 32) == tag && (unsigned)(lw >> 32) == tag)) break;
             if (it > WALK_SPIN) {
               if (lane == 0) atomicOr(ctl + 1, 1);
               gave_up = true;
               break;
             }
             __builtin_amdgcn_s_sleep(1);
-            const unsigned long long hi =
-                __hip_atomic_load(xup + 2 * fjc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long lo =
-                __hip_atomic_load(xup + 2 * fjc + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            hw = __builtin_amdgcn_readfirstlane((unsigned)hi);
-            ht = __builtin_amdgcn_readfirstlane((unsigned)(hi >> 32));
-            lw = __builtin_amdgcn_readfirstlane((unsigned)lo);
-            lt = __builtin_amdgcn_readfirstlane((unsigned)(lo >> 32));
           }
-          gv = __hiloint2double((int)hw, (int)lw);
-          ge = t >= 2 ? gv_prev : 1e6;  // column fjc-1: the previous step's, or the ring
-          gv_prev = gv;
         }
-        const double tv = dpp_shr1_d(gv, prev);
-        const double tev = dpp_shr1_d(ge, prev2);
-        const int fj = t - lane;
-        double out = 1e6;
-        const float szo = qsz[u];
-        const float sxo = dpp_shl1f(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x63), u)), szo);
-        const float sr = sref;
-        sref = szo;
-        if (row_int && fj >= 1 && fj <= nxx - 2) {
-          out = fmin(qto[u], local_d(tv, prev, tev, sr, szo, sxo, K));
-          const int j = SB > 0 ? fj : nxx - 1 - fj;
-          Tn[i + (size_t)j * nzz] = out;
+        // step 0's value is only step 1's diagonal one: the ring's
+        if (lane < WK_B) xup_l[buf][lane] = t == 0 ? 1e6 : v;
+        // (the cells after the words: the poll does not queue behind the next
+        // block's loads, which touch 64 lines each)
+#pragma unroll
+        for (int u = 0; u < WK_B; ++u) {
+          s_l[buf][u][lane] = q[u];
+          thr_l[buf][u][lane] = thr_b((double)q[u], K);
         }
-        if (pub && fj >= 1 && fj <= nxx - 2) {
-          __hip_atomic_store(xme + 2 * fj, walk_word((unsigned)__double2hiint(out), tag), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(xme + 2 * fj + 1, walk_word((unsigned)__double2loint(out), tag), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-        }
-        prev2 = prev;
-        prev = out;
-        load(min(t + ADJ_PF, NT - 1), qto[u], qsz[u]);
+        if (lane < WK_B) s_l[buf][lane][64] = q64;
+        load((n + 2) * WK_B);
+        lds_barrier();
       }
-    };
-    // word blocks ping-pong between (ah, al) and (bh, bl), each loaded one
-    // block before its use
-    unsigned long long ah, al, bh, bl;
-    float as, bs;
-    xload(0, ah, al, as);
-    // Drain once per strip: inside the loop every word block and queue slot
-    // was loaded a full block (over 63 memory operations) before its use,
-    // which needs no wait; the compiler's count merges the loop-entry path,
-    // where the first loads are recent, and would otherwise wait there at
-    // every block.
-    __builtin_amdgcn_s_waitcnt(0);
-    for (int t0 = 0; t0 < NT; t0 += 2 * ADJ_PF) {
-      xload(t0 + ADJ_PF, bh, bl, bs);
-      block(t0, ah, al, as);
-      xload(min(t0 + 2 * ADJ_PF, NT - ADJ_PF), ah, al, as);
-      block(t0 + ADJ_PF, bh, bl, bs);
     }
   }
 }
@@ -337,7 +491,7 @@ struct AdjCoef {
 };
 
 // The branch the fp64 forward took at a node (same expressions and
-// comparisons as local_d) and its partial derivatives.  Ties follow the
+// comparisons as local_sel_d) and its partial derivatives.  Ties follow the
 // oracle: T_old wins when T_old <= candidate; 1-D before 2-D when equal;
 // z-edge before x-edge when equal; min(S, S') of two equal cells splits dS
 // half and half (what central differences measure).
@@ -724,6 +878,7 @@ static ConstsD consts_d(double dx, double dz) {
   k.dz2i = 1.0 / (dz * dz);
   k.dx2i = 1.0 / (dx * dx);
   k.sum = k.dz2i + k.dx2i;
+  k.sum4 = 4.0 * k.sum;
   k.prod = k.dz2i * k.dx2i;
   k.hyp = std::sqrt(dx * dx + dz * dz);
   k.r_dx = 1.0 / k.dx;
@@ -739,19 +894,20 @@ void launch_fwd64_init(const AdjShot* shots, int nshots, int nzz, double dx, dou
 }
 
 void launch_fwd64_sweep(int sweep, const AdjShot* shots, int nshots, int nzz, int nstr, double dx, double dz,
-                        const double* Told, double* Tnew, int* walk_ctl, unsigned long long* walk_x, int ldx,
-                        unsigned tag, hipStream_t st) {
+                        const SkewView& skew, const double* Told, double* Tnew, int* walk_ctl,
+                        unsigned long long* walk_x, int ldx, unsigned tag, hipStream_t st) {
   const ConstsD k = consts_d(dx, dz);
   hipLaunchKernelGGL(k_walk_begin, dim3(1), dim3(64), 0, st, walk_ctl);
-  // one wave per strip, at most what is resident at once (the tickets keep
-  // any count correct)
-  const int grid = std::min(nshots * nstr, 4096);
-  switch (sweep) {
-    case 0: hipLaunchKernelGGL((k_fwd64_sweep<1, 1>), dim3(grid), dim3(64), 0, st, shots, nshots, nzz, nstr, k, Told, Tnew, walk_ctl, walk_x, ldx, tag); break;
-    case 1: hipLaunchKernelGGL((k_fwd64_sweep<-1, 1>), dim3(grid), dim3(64), 0, st, shots, nshots, nzz, nstr, k, Told, Tnew, walk_ctl, walk_x, ldx, tag); break;
-    case 2: hipLaunchKernelGGL((k_fwd64_sweep<1, -1>), dim3(grid), dim3(64), 0, st, shots, nshots, nzz, nstr, k, Told, Tnew, walk_ctl, walk_x, ldx, tag); break;
-    default: hipLaunchKernelGGL((k_fwd64_sweep<-1, -1>), dim3(grid), dim3(64), 0, st, shots, nshots, nzz, nstr, k, Told, Tnew, walk_ctl, walk_x, ldx, tag); break;
-  }
+  // a workgroup per strip, at most what is resident at once (three per CU;
+  // the tickets keep any count correct)
+  const int grid = std::min(nshots * nstr, 768);
+  auto* f = dx == dz ? (sweep == 0 ? k_fwd64_sweep<1, 1, true> : sweep == 1 ? k_fwd64_sweep<-1, 1, true>
+                        : sweep == 2 ? k_fwd64_sweep<1, -1, true> : k_fwd64_sweep<-1, -1, true>)
+                     : (sweep == 0 ? k_fwd64_sweep<1, 1, false> : sweep == 1 ? k_fwd64_sweep<-1, 1, false>
+                        : sweep == 2 ? k_fwd64_sweep<1, -1, false> : k_fwd64_sweep<-1, -1, false>);
+  hipLaunchKernelGGL(f, dim3(grid), dim3(256), 0, st, shots, nshots, nzz, nstr, k,
+                     skew.KP <= 1 << 20 ? skew : SkewView{nullptr, 0},  // (a lane's byte offset in 32 bits)
+                     Told, Tnew, walk_ctl, walk_x, ldx, tag);
 }
 
 void launch_picks64(const AdjShot* shots, const int* rec_shot, const float* rx, const float* rz, int nrec, int nzz,

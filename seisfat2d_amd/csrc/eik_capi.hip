@@ -908,7 +908,7 @@ int run_record(seisfat_batch_s* b, hipStream_t st) {
   const size_t ts = b->tsize;
   launch_fwd64_init(A.d_tab, b->nshots, h->nzz, h->dx, h->dz, A.d_T64, st);
   for (int s = 0; s < 4; ++s)
-    launch_fwd64_sweep(s, A.d_tab, b->nshots, h->nzz, A.nstr, h->dx, h->dz, A.d_T64 + s * ts,
+    launch_fwd64_sweep(s, A.d_tab, b->nshots, h->nzz, A.nstr, h->dx, h->dz, h->skew[s], A.d_T64 + s * ts,
                        A.d_T64 + (s + 1) * ts, A.d_walk_ctl, A.d_walk_x, A.walk_ldx,
                        A.walk_tag = A.walk_tag == 0xffffffffu ? 1 : A.walk_tag + 1, st);
   launch_picks64(A.d_tab, b->d_recshot, b->d_rx, b->d_rz, b->nrec, h->nzz, h->dx, h->dz, A.d_T64 + 4 * ts,

@@ -270,3 +270,32 @@ def test_ray_gradient_correlation(oracle, rng):
     assert corr > 0.9
     b.close()
     e.close()
+
+
+# the FP64 walk at the edges of its strips (64 rows), blocks (8 steps) and ring,
+# with skewed and clamped slowness columns (narrow windows, window edges) and
+# both spacings: the misfit and its gradient against the FP64 oracle
+@pytest.mark.parametrize("nz,nx,dz,dx,wins", [(8, 9, 10.0, 10.0, None), (57, 70, 10.0, 10.0, None),
+                                              (58, 131, 10.0, 7.0, None), (59, 150, 6.0, 9.0, [(0, 90), (41, 109), (60, 30)]),
+                                              (122, 200, 10.0, 10.0, [(0, 200), (3, 180), (100, 64), (150, 50)]),
+                                              (190, 77, 12.0, 5.0, None)])
+def test_walk_edges(oracle, nz, nx, dz, dx, wins):
+    w = models.rough(nz, nx, dz, dx, seed=nz + nx, sigma=4.0, vlo=2000.0, vhi=3000.0)
+    shots, rx, off = [], [], 0
+    for k, (x0, wd) in enumerate(wins or [(0, nx)] * 2):
+        r = np.linspace(x0 + 0.1, x0 + wd - 1.1, 7) * dx
+        shots.append((float(np.float32((x0 + (0.3 + 0.2 * k % 0.6) * (wd - 1)) * dx)), 0.0, x0, wd, off, len(r)))
+        rx.append(r)
+        off += len(r)
+    rx = np.concatenate(rx).astype(np.float32)
+    rz = np.full(len(rx), 0.3 * dz, np.float32)
+    obs = np.linspace(0.0, 0.3, len(rx)).astype(np.float32)
+    e = Eikonal(nz, nx, dz, dx)
+    e.set_slowness(w.s)
+    b = e.batch(shots, rx, rz)
+    J, g, _ = b.misfit_gradient(obs)
+    Jo, go, _ = oracle.batch_misfit(w.s.astype(np.float64), dx, dz, shots, rx, rz, obs.astype(np.float64))
+    assert np.isclose(J, Jo, rtol=1e-10)
+    assert np.abs(g - go).max() <= 1e-5 * np.abs(go).max()
+    b.close()
+    e.close()
