@@ -3,18 +3,16 @@
 //
 // The forward solve is init + four directional sweeps; node (i, j) of sweep s
 // becomes min(T_old, cand(tv, te, tev, S)) with tv, te, tev its upwind
-// neighbours after sweep s.  The adjoint walks the sweeps backwards; for each
-// sweep it
-//   1. re-derives, for every node in parallel, the branch the forward took
-//      and its local partials d(new)/d(tv, te, tev, S) from a recorded fp64
-//      trajectory of the solve (k_fwd64_sweep) — k_adj_coef;
-//   2. runs the linear recurrence
-//        mu(n) = lam_in(n) + sum over the three nodes m that read n of
-//                mu(m) * d(new_m)/d(n)
-//      in reverse dependency order — k_adj_sweep, one wave per 64-row strip;
-//   3. folds mu(n) * d(new_n)/dS into the per-shot slowness gradient — k_adj_fold.
-// The source initialisation T0 = S(node) * distance and the FP64 cross-shot
-// reduction onto the unpadded model close the chain.
+// neighbours after sweep s.  The adjoint walks the sweeps backwards
+// (k_adj_sweep): it re-derives the branch the forward took at every node and
+// its local partials d(new)/d(tv, te, tev, S) from a recorded fp64 trajectory of
+// the solve (k_fwd64_sweep), and runs the linear recurrence
+//   mu(n) = lam_in(n) + sum over the three nodes m that read n of
+//           mu(m) * d(new_m)/d(n)
+// in reverse dependency order, one workgroup per 64-row strip.  k_adj_fold
+// folds mu(n) * d(new_n)/dS onto the cells and adds the source initialisation's
+// T0 = S(node) * distance; k_adj_reduce sums the shots in FP64 onto the unpadded
+// model.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -24,14 +22,10 @@
 
 namespace seisfat {
 
-constexpr int ADJ_PF = 8;  // prefetch distance and word-block length of the strip walkers (steps)
-
 // A shot as the adjoint kernels see it.
 struct AdjShot {
   ShotDev sd;   // final traveltimes (sd.T), slowness view, width, source, window
-  size_t toff;  // offset of the shot in the natural-layout arrays (snapshots, gshot)
-  size_t koff;  // offset in the strip-skewed arrays
-  int NTP;      // steps per strip: nxx + 63 rounded up to ADJ_PF
+  size_t toff;  // offset of the shot's grid in every array below
 };
 
 // Forward sweep s runs rows in direction a and columns in direction b
@@ -42,14 +36,6 @@ __host__ __device__ inline int adj_a(int s) { return (s & 1) ? -1 : 1; }
 __host__ __device__ inline int adj_b(int s) { return (s & 2) ? -1 : 1; }
 __host__ __device__ inline int adj_ip(int i, int a, int nzz) { return a > 0 ? nzz - 1 - i : i; }
 __host__ __device__ inline int adj_jp(int j, int b, int nxx) { return b > 0 ? nxx - 1 - j : j; }
-
-// Strip-skewed layout: reverse-local node (ip, jp) is held by strip ip/64,
-// lane ip%64, at step jp + lane, so the 64 nodes one wave visits at one step
-// are 64 consecutive words.
-__host__ __device__ inline size_t adj_kidx(int ip, int jp, int NTP) {
-  const int lane = ip & 63;
-  return ((size_t)(ip >> 6) * NTP + (size_t)(jp + lane)) * 64 + lane;
-}
 
 // Pick seeds: lam[node[n]] = sum_{e in ptr[n]..ptr[n+1]} w[rec[e]] * wt[e].
 void launch_adj_seed(const size_t* node, const int* ptr, const int* rec, const float* wt, int nseed,
@@ -67,23 +53,22 @@ void launch_fwd64_sweep(int sweep, const AdjShot* shots, int nshots, int nzz, in
 // receiver's shot grid).
 void launch_picks64(const AdjShot* shots, const int* rec_shot, const float* rx, const float* rz, int nrec, int nzz,
                     double dx, double dz, const double* T4, double* out, hipStream_t st);
-// Local partials of sweep s from the fp64 trajectory (Tnew = T after sweep s,
-// Told = before); also moves lam_src (layout of sweep s+1) into lam_dst
-// (layout of sweep s) when lam_src is non-null.  nstr: 64-row strips per
-// shot; max_nxx: the widest shot's padded width.
-void launch_adj_coef(int sweep, const AdjShot* shots, int nshots, int nstr, int max_nxx, int nzz, double dx,
-                     double dz, const double* Tnew, const double* Told, const float* lam_src, float* lam_dst,
-                     float4* coef, uint8_t* code, hipStream_t st);
-void launch_adj_sweep(const AdjShot* shots, int nshots, int nstr, const float* lam_in, const float4* coef,
-                      float* lam_out, float* gc, int* walk_ctl, unsigned long long* walk_x, int ldx, unsigned tag,
+// Reverse sweep s from the fp64 trajectory (Tnew = T after sweep s, Told =
+// before): lam in place; g and code: every node's slowness contribution and the
+// cells it goes to.  skew_opposite: the skewed slowness copy of the opposite
+// orientation (sweep 3 - s).  walk_ctl, walk_x, tag as for the forward walk.
+void launch_adj_sweep(int sweep, const AdjShot* shots, int nshots, int nzz, int nstr, double dx, double dz,
+                      const SkewView& skew_opposite, const double* Tnew, const double* Told, float* lam, float* g,
+                      uint8_t* code, int* walk_ctl, unsigned long long* walk_x, int ldx, unsigned tag,
                       hipStream_t st);
-void launch_adj_fold(int sweep, const AdjShot* shots, int nshots, int nstr, int max_nxx, int nzz, const float* gc,
-                     const uint8_t* code, float* gshot, hipStream_t st);
-void launch_adj_source(const AdjShot* shots, int nshots, int nzz, double dx, double dz, const float* lam0,
-                       float* gshot, hipStream_t st);
+// Per-shot slowness gradient on padded cells from the four sweeps' g and code
+// (sweep s at [s * tsize]) and lam after sweep 0.
+void launch_adj_fold(const AdjShot* shots, int nshots, int max_nxx, int nzz, size_t tsize, double dx, double dz,
+                     const float* g, const uint8_t* code, const float* lam, float* gshot, hipStream_t st);
 // fixed_border: the model's border is not the replication of its edges (a
-// padded upload), so only interior nodes (and windows' replicated columns) fold
-void launch_adj_reduce(const AdjShot* shots, int nshots, int nz, int nx, int nzz, const float* gshot,
-                       double* grad, bool fixed_border, hipStream_t st);
+// padded upload), so only interior cells (and windows' replicated columns) fold
+// edge: scratch, nshots x 2 (max_w + nz), each shot's sums over the cells its model edges replicate to
+void launch_adj_reduce(const AdjShot* shots, int nshots, int nz, int nx, int nzz, int max_w, const float* gshot,
+                       double* edge, double* grad, bool fixed_border, hipStream_t st);
 
 }  // namespace seisfat

@@ -481,380 +481,539 @@ __global__ void k_picks64(const AdjShot* __restrict__ shots, const int* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Local partials of one node.  ds < 0 marks a node the sweep left unchanged
-// (T_old kept: the adjoint passes through); bit (di | dj << 1) of code marks
-// slowness cell (i - di, j - dj) as receiving ds, split evenly when two bits
-// are set.
+// 1 / b for a normal b whose reciprocal is normal (the refined reciprocal of
+// IEEE division) and, with it, RN(a / b).
+__device__ __forceinline__ double recip_d(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+}
+
+// Local partials of one node: (dT/dtv, dT/dte, dT/dtev, dT/dS), dT/dS < 0 at a
+// node the sweep left unchanged (T_old kept: the adjoint passes through).  Bit
+// (di | dj << 1) of code marks slowness cell (i - di, j - dj) as receiving
+// dT/dS, split evenly when two bits are set.
 struct AdjCoef {
-  float dtv, dte, dtev, ds;
-  int code;
+  float4 c;
+  unsigned code;
 };
 
-// The branch the fp64 forward took at a node (same expressions and
-// comparisons as local_sel_d) and its partial derivatives.  Ties follow the
-// oracle: T_old wins when T_old <= candidate; 1-D before 2-D when equal;
-// z-edge before x-edge when equal; min(S, S') of two equal cells splits dS
-// half and half (what central differences measure).
+// The partials of the branch the fp64 forward took at an updated node with
+// value tn (same expressions and comparisons as local_sel_d): a 1-D candidate
+// when one equals tn, else the 2-D branch whose conditions hold.  Ties follow
+// the oracle: 1-D before 2-D when equal; z-edge before x-edge when equal;
+// min(S, S') of two equal cells splits dS half and half (what central
+// differences measure).
 template <int SA, int SB>
-__device__ __forceinline__ AdjCoef adj_local(double tv, double te, double tev, double sref, double szo,
-                                             double sxo, double told, const ConstsD& k) {
+__device__ __forceinline__ AdjCoef adj_local(double tn, double tv, double te, double tev, double sref, double szo,
+                                             double sxo, bool upd, const ConstsD& k) {
   constexpr int di_ref = (SA + 1) / 2, dj_ref = (SB + 1) / 2;
-  constexpr int c_ref = di_ref | (dj_ref << 1);
-  constexpr int c_zo = di_ref | (((1 - SB) / 2) << 1);
-  constexpr int c_xo = ((1 - SA) / 2) | (dj_ref << 1);
-  const double t1d1 = tv + k.dz * fmin(sref, szo);
-  const double t1d2 = te + k.dx * fmin(sref, sxo);
-  const double t1D = fmin(t1d1, t1d2);
-  double tbr = 1e6;
-  bool taken = false;
-  double p_tv = 0.0, p_te = 0.0, p_tev = 0.0, p_s = 0.0;
-  if ((tv <= te + k.dx * sref) && (te <= tv + k.dz * sref) && (te - tev >= 0.0) && (tv - tev >= 0.0)) {
-    const double ta = tev + te - tv;
-    const double tb = tev - te + tv;
-    const double sq = sqrt(4.0 * sref * sref * k.sum - k.prod * (ta - tb) * (ta - tb));
-    tbr = cdiv((tb * k.dz2i + ta * k.dx2i) + sq, k.sum, k.r_sum);
-    taken = true;
+  constexpr unsigned c_ref = 1u << (di_ref | (dj_ref << 1));
+  constexpr unsigned c_zo = 1u << (di_ref | (((1 - SB) / 2) << 1));
+  constexpr unsigned c_xo = 1u << (((1 - SA) / 2) | (dj_ref << 1));
+  const double t1d1 = tv + k.dz * vmin_d(sref, szo);
+  const double t1d2 = te + k.dx * vmin_d(sref, sxo);
+  const bool one = vmin_d(t1d1, t1d2) == tn, z = t1d1 <= t1d2;
+  const double de = te - tev, dv = tv - tev;
+  const bool cA = (tv <= te + k.dx * sref) & (te <= tv + k.dz * sref) & (de >= 0.0) & (dv >= 0.0);
+  AdjCoef r{};
+  if (__any(upd & !one & cA)) {
     // t = ((tb dz2i + ta dx2i) + sqrt(4 S^2 D - dz2i dx2i (ta - tb)^2)) / D
-    const double kk = 2.0 * k.prod * (ta - tb) / sq;
-    p_te = cdiv(k.dx2i - k.dz2i - kk, k.sum, k.r_sum);
-    p_tv = cdiv(k.dz2i - k.dx2i + kk, k.sum, k.r_sum);
-    p_tev = 1.0;
-    p_s = 4.0 * sref / sq;
-  } else if ((te - tev <= cdiv(sref * k.dz * k.dz, k.hyp, k.r_hyp)) && (te - tev > 0.0)) {
-    // t = te + dx sqrt(S^2 - q^2), q = (te - tev) / dz
-    const double q = cdiv(te - tev, k.dz, k.r_dz);
-    const double Q = sqrt(sref * sref - q * q);
-    tbr = te + k.dx * Q;
-    taken = true;
-    const double r = k.dx * q / (k.dz * Q);
-    p_te = 1.0 - r;
-    p_tev = r;
-    p_s = k.dx * sref / Q;
-  } else if ((tv - tev <= cdiv(sref * k.dx * k.dx, k.hyp, k.r_hyp)) && (tv - tev > 0.0)) {
-    const double p = cdiv(tv - tev, k.dx, k.r_dx);
-    const double P = sqrt(sref * sref - p * p);
-    tbr = tv + k.dz * P;
-    taken = true;
-    const double r = k.dz * p / (k.dx * P);
-    p_tv = 1.0 - r;
-    p_tev = r;
-    p_s = k.dz * sref / P;
+    const double dab = (tev + te - tv) - (tev - te + tv);
+    const double sq = sqrt_rn_d(4.0 * sref * sref * k.sum - k.prod * dab * dab), y = recip_d(sq);
+    const double ak = 2.0 * k.prod * dab, as = 4.0 * sref, qk = ak * y, qs = as * y;
+    const double kk = __builtin_fma(__builtin_fma(-sq, qk, ak), y, qk);
+    const double te_d = cdiv(k.dx2i - k.dz2i - kk, k.sum, k.r_sum);  // (dT/dtv is its opposite)
+    r.c = make_float4((float)-te_d, (float)te_d, 1.0f, (float)__builtin_fma(__builtin_fma(-sq, qs, as), y, qs));
   }
-  const double t2D = fmin(tbr, 1e6);
-  const double cand = fmin(t1D, t2D);
-  AdjCoef c{0.0f, 0.0f, 0.0f, -1.0f, 0};
-  if (!(cand < told)) return c;
-  if (t1D <= t2D) {
-    if (t1d1 <= t1d2) {
-      c.dtv = 1.0f;
-      c.ds = (float)k.dz;
-      c.code = sref == szo ? (1 << c_ref) | (1 << c_zo) : sref < szo ? 1 << c_ref : 1 << c_zo;
-    } else {
-      c.dte = 1.0f;
-      c.ds = (float)k.dx;
-      c.code = sref == sxo ? (1 << c_ref) | (1 << c_xo) : sref < sxo ? 1 << c_ref : 1 << c_xo;
-    }
-    return c;
+  if (__any(upd & !one & !cA)) {
+    const bool cB = (de <= cdiv(sref * k.dz * k.dz, k.hyp, k.r_hyp)) & (de > 0.0);
+    // B: t = te + dx sqrt(S^2 - q^2), q = (te - tev) / dz; C: the same with the axes exchanged
+    const double h1 = cB ? k.dz : k.dx, h2 = cB ? k.dx : k.dz;
+    const double q = cdiv(cB ? de : dv, h1, cB ? k.r_dz : k.r_dx);
+    const double Q = sqrt_rn_d(sref * sref - q * q);
+    const double rr = h2 * q / (h1 * Q);
+    const float p = (float)(1.0 - rr);
+    if (!cA) r.c = make_float4(cB ? 0.0f : p, cB ? p : 0.0f, (float)rr, (float)(h2 * sref / Q));
   }
-  if (!taken || !(tbr < 1e6)) {  // the 1e6 constant won: no dependence
-    c.ds = 0.0f;
-    return c;
+  r.code = c_ref;
+  if (one) {
+    const double other = z ? szo : sxo;
+    const unsigned c_o = z ? c_zo : c_xo;
+    r.code = sref == other ? c_ref | c_o : sref < other ? c_ref : c_o;
+    r.c = make_float4(z ? 1.0f : 0.0f, z ? 0.0f : 1.0f, 0.0f, (float)(z ? k.dz : k.dx));
   }
-  c.dtv = (float)p_tv;
-  c.dte = (float)p_te;
-  c.dtev = (float)p_tev;
-  c.ds = (float)p_s;
-  c.code = 1 << c_ref;
-  return c;
+  if (!upd) {
+    r.c = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
+    r.code = 0;
+  }
+  return r;
 }
 
-// One workgroup per (strip rs, block of ADJ_CB reverse-local columns, shot):
-// first each wave takes whole columns of the block in natural order, lane =
-// row, so its loads of T and S are contiguous runs (a wave reading one step
-// of the strip-skewed layout reads a diagonal instead: 64 cache lines per
-// load, which bounded this kernel); the partials go to LDS by column, and
-// then the workgroup writes the skewed entries (lane k, step t) whose node
-// (64rs + k, t - k) lies in the block, each step a contiguous run of lanes.
-// Entries outside the grid are left untouched.
-constexpr int ADJ_CB = 32;
+// One reverse sweep: mu(n) = lam(n) + sum over the three nodes m that read n of
+// mu(m) d(new_m)/d(n), in reverse dependency order; a node the sweep updated
+// passes mu on through its partials and leaves 0 in lam, another keeps mu
+// there; g and code get mu dT/dS and the cells it goes to.  A workgroup walks
+// one strip of 64 reverse-local rows of one shot; step t holds row 64r + k at
+// column t - k, as the forward walk's.  Wave 0 runs the recurrence from LDS
+// (messages from lane k-1 by DPP, from its own previous step, and lane 0's from
+// the upper strip); wave 1 brings whole columns of lam, wave 2 those of the
+// traveltimes before and after the sweep, whose difference marks the nodes it
+// updated (the sign of the word); waves 4 and 5 store the finished columns of
+// lam, g and code; waves 6 to 13 evaluate the partials of a step of a block
+// each, one block ahead, and skip the steps no node of which was updated; wave 3
+// exchanges the last row's messages with the neighbouring strips (tagged words as
+// in the forward walk, bounded polls) and brings the row of traveltimes below
+// the strip.  The columns pass through skewed LDS rings ([step][lane], see k_fwd64_sweep), so
+// nothing skewed is stored: 16 B of traveltimes read, 8 B of lam, 5 B of g and
+// code per node.  The chain of a strip's steps is the bound while the strips are
+// fewer than the CUs, the partials' FP64 instructions beyond: one strip of
+// 58 x 1201 123 us a sweep, 301 x 1201 163 with 1 shot, 230 with 50 and 525 with
+// 128 (640 strips); as three kernels (partials, recurrence, contributions to the
+// cells, through skewed arrays of 37 B per node) it was 1.5 ms with 128.  Loads
+// and stores are kept in separate waves: with both in one, its loads wait for the
+// acknowledgement of its stores (730 us with 128 shots against 614).  8 waves for
+// the partials against 4: 123 / 163 / 230 / 525 against 155 / 201 / 258 / 557;
+// blocks of 16 steps with 4 waves 150 / 195 / 242 / 514; two workgroups a CU
+// (blocks of 4 steps) 621 with 128.
+constexpr int AB = 8;               // steps per block
+constexpr int AT = 64 + 3 * AB;     // ring steps.  Traveltimes: a step's columns, two blocks' lead (and one to
+                                    // round up); lam (the node's result replaces it): a block arriving, one leaving
+constexpr int ADJ_OUT = 2, ADJ_COEF = 8;    // waves that store and that evaluate partials
+constexpr int ADJ_THREADS = 64 * (4 + ADJ_OUT + ADJ_COEF);
+constexpr unsigned ADJ_UPD = 0x80;  // in the ring of codes: the node was updated
+
+// x mod n for 0 <= x < 2n
+__device__ __forceinline__ unsigned wrap(unsigned x, unsigned n) { return min(x, x - n); }
 
 template <int SA, int SB>
-__global__ __launch_bounds__(256) void k_adj_coef(const AdjShot* __restrict__ shots, int nzz, int nstr, ConstsD k,
-                                                  const double* __restrict__ Tnew, const double* __restrict__ Told,
-                                                  int pa, int pb, const float* __restrict__ lam_src,
-                                                  float* __restrict__ lam_dst, float4* __restrict__ coef,
-                                                  uint8_t* __restrict__ code) {
-  __shared__ float P[4][ADJ_CB][64];
-  __shared__ uint8_t Pc[ADJ_CB][64];
-  const AdjShot sh = shots[blockIdx.y];
-  const int nxx = sh.sd.nxx, NTP = sh.NTP;
-  const int rs = (int)(blockIdx.x % (unsigned)nstr), jp0 = (int)(blockIdx.x / (unsigned)nstr) * ADJ_CB;
-  if (jp0 >= nxx) return;  // whole workgroup: blocks past this shot's width
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int ip = 64 * rs + lane;
-  const double* __restrict__ Tn = Tnew + sh.toff;
-  for (int col = w; col < ADJ_CB; col += 4) {
-    const int jp = jp0 + col;
-    AdjCoef c{0.0f, 0.0f, 0.0f, -1.0f, 0};
-    if (ip < nzz && jp < nxx) {
-      const int i = adj_ip(ip, SA, nzz), j = adj_jp(jp, SB, nxx);  // (both maps are involutions)
-      if (i >= 1 && i <= nzz - 2 && j >= 1 && j <= nxx - 2) {
-        const double tv = Tn[(i - SA) + (size_t)j * nzz];
-        const double te = Tn[i + (size_t)(j - SB) * nzz];
-        const double tev = Tn[(i - SA) + (size_t)(j - SB) * nzz];
-        const double told = Told[sh.toff + i + (size_t)j * nzz];
-        const int i1 = i - (SA + 1) / 2, j1 = j - (SB + 1) / 2;
-        const double sref = s_at(sh.sd, nzz, i1, j1);
-        const double szo = s_at(sh.sd, nzz, i1, j1 + SB);
-        const double sxo = s_at(sh.sd, nzz, i1 + SA, j1);
-        c = adj_local<SA, SB>(tv, te, tev, sref, szo, sxo, told, k);
-      }
-    }
-    P[0][col][lane] = c.dtv;
-    P[1][col][lane] = c.dte;
-    P[2][col][lane] = c.dtev;
-    P[3][col][lane] = c.ds;
-    Pc[col][lane] = (uint8_t)c.code;
-  }
-  __syncthreads();
-  // step t = jp0 + e/64 of the skewed strip, lane e%64 (= this thread's lane)
-  const size_t sbase = sh.koff + (size_t)rs * NTP * 64;
-  for (int e = threadIdx.x; e < (ADJ_CB + 63) * 64; e += 256) {
-    const int t = jp0 + (e >> 6), jp = t - lane, col = jp - jp0;
-    if (col < 0 || col >= ADJ_CB || jp >= nxx || ip >= nzz) continue;
-    const size_t ko = sbase + (size_t)t * 64 + lane;
-    if (lam_src) {
-      const int i = adj_ip(ip, SA, nzz), j = adj_jp(jp, SB, nxx);
-      lam_dst[ko] = lam_src[sh.koff + adj_kidx(adj_ip(i, pa, nzz), adj_jp(j, pb, nxx), NTP)];
-    }
-    coef[ko] = make_float4(P[0][col][lane], P[1][col][lane], P[2][col][lane], P[3][col][lane]);
-    code[ko] = Pc[col][lane];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Reverse sweep: one wave per strip of 64 reverse-local rows; lane k holds
-// row 64r + k and visits column t - k at step t.  The z-upwind and diagonal
-// messages come from lane k-1 (DPP shift), the x message from the lane's own
-// previous step.  Lane 0's messages are the upper strip's lane-63 ones, which
-// that strip publishes column by column as tagged words (word 2jp = the launch's
-// tag and mv of column jp, word 2jp+1 the same for mev), written at its step
-// jp+63 and read with the forward walker's protocol: one block load per
-// ADJ_PF steps (lane u holds step u's words), one block ahead, and a bounded
-// poll of the column while a tag is stale.  Strip 0 and the columns no strip
-// publishes read zero messages.  Strips are claimed strip-major from the
-// ticket counter ctl[0], so every upper neighbour is already running.  Inputs
-// of ADJ_PF steps ahead are kept in flight; nodes outside the grid hold zero
-// inputs and produce zero outputs.
-__global__ __launch_bounds__(64) void k_adj_sweep(const AdjShot* __restrict__ shots, int nshots, int nstr,
-                                                  const float* __restrict__ lam_in,
-                                                  const float4* __restrict__ coef, float* __restrict__ lam_out,
-                                                  float* __restrict__ gc, int* __restrict__ ctl,
-                                                  unsigned long long* __restrict__ xw, int ldx, unsigned tag) {
+__global__ __launch_bounds__(ADJ_THREADS) void k_adj_sweep(const AdjShot* __restrict__ shots, int nshots, int nzz, int nstr,
+                                                  ConstsD K, SkewView sk, const double* __restrict__ Tnew,
+                                                  const double* __restrict__ Told, float* __restrict__ lam,
+                                                  float* __restrict__ g, uint8_t* __restrict__ code,
+                                                  int* __restrict__ ctl, unsigned long long* __restrict__ xw, int ldx,
+                                                  unsigned tag) {
   typedef __attribute__((address_space(1))) unsigned long long gword;
-  const int lane = threadIdx.x;
+  __shared__ double ringT[AT * 65];
+  __shared__ float ringV[AT * 64];
+  __shared__ uint8_t ringC[AT * 64];
+  __shared__ float4 cf[2][AB][64];
+  __shared__ float2 xin[2][AB];            // upper strip's messages (to the row below, to the diagonal)
+  __shared__ float2 pub[2][AB][2];         // this strip's last row's (second word: the other lanes' dummy)
+  __shared__ int ticket;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (;;) {
-    int tk = 0;
-    if (lane == 0) tk = atomicAdd(ctl, 1);
-    tk = __builtin_amdgcn_readfirstlane(tk);
+    if (threadIdx.x == 0) ticket = atomicAdd(ctl, 1);
+    __syncthreads();
+    const int tk = __builtin_amdgcn_readfirstlane(ticket);
     if (tk >= nshots * nstr) break;
     const int r = tk / nshots, ks = tk - r * nshots;
     const AdjShot sh = shots[ks];
-    const int NTP = sh.NTP, nxx = sh.sd.nxx;
-    const size_t base = sh.koff + (size_t)r * NTP * 64 + lane;
-    gword* xme = (gword*)(xw + ((size_t)ks * nstr + r) * ldx);
-    const gword* xup = (const gword*)(xw + ((size_t)ks * nstr + max(r - 1, 0)) * ldx);
-    const bool up = r > 0;
-    const bool pub = lane == 63 && r + 1 < nstr;
-    float ql[ADJ_PF];
-    float4 qc[ADJ_PF];
+    const int nxx = sh.sd.nxx;
+    const int NBLK = (nxx + 63 + AB - 1) / AB;
+    const int ip = 64 * r + lane;
+    const int ipc = min(ip, nzz - 1);
+    const int i = adj_ip(ipc, SA, nzz);
+    // column jp, clamped to the grid (its first and last columns are ring nodes,
+    // which no sweep updates), and the step from it to the next
+    const auto col = [&](int jp) { return (size_t)adj_jp(min(max(jp, 0), nxx - 1), SB, nxx) * nzz; };
+    const auto next = [&](int jp) { return jp >= 0 && jp + 1 < nxx ? (SB > 0 ? -nzz : nzz) : 0; };
+    // block n: wave 0 takes steps 8n .. 8n + 7 (for 0 <= n < NBLK)
+    const int n_first = -3, n_last = NBLK + 1;
+    if (wave == 0) {
+      float mv = 0.0f, me = 0.0f, mev = 0.0f, mevp = 0.0f;
+      for (int n = n_first; n <= n_last; ++n) {
+        if (n >= 0 && n < NBLK) {
+          const int buf = n & 1;
+          float* __restrict__ rv = ringV + (n * AB % AT) * 64 + lane;
+          float2* __restrict__ pb = &pub[buf][0][lane == 63 ? 0 : 1];
+          unsigned zero = 0;
+          asm volatile("" : "+v"(zero));  // (one address register for the block's broadcasts)
+          float ql = rv[0];
+          float4 c = cf[buf][0][lane];
+          float2 x = xin[buf][zero];
 #pragma unroll
-    for (int u = 0; u < ADJ_PF; ++u) {
-      ql[u] = lam_in[base + (size_t)u * 64];
-      qc[u] = coef[base + (size_t)u * 64];
-    }
-    // step t's words: mv of column t (word 2t) and mev of column t-1 (word
-    // 2t-1), at clamped addresses (the step ignores the columns out of range)
-    auto wv = [&](int t) { return xup + 2 * min(t, nxx - 1); };
-    auto we = [&](int t) { return xup + max(2 * min(t, nxx) - 1, 0); };
-    // unconditional (strip 0 reads its own words and ignores them)
-    auto xload = [&](int tb, unsigned long long& v, unsigned long long& e) {
-      const int t = tb + (lane & (ADJ_PF - 1));
-      v = __hip_atomic_load(wv(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      e = __hip_atomic_load(we(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    float mv = 0.0f, me = 0.0f, mev = 0.0f, mevp = 0.0f;
-    bool gave_up = false;
-    auto block = [&](int t0, unsigned long long bv, unsigned long long be) {
+          for (int u = 0; u < AB; ++u) {
+            const float qu = ql;
+            const float4 cu = c;
+            const float2 xu = x;
+            if (u + 1 < AB) {  // a step's operands are read one step ahead
+              ql = rv[64 * (u + 1)];
+              c = cf[buf][u + 1][lane];
+              x = xin[buf][zero + u + 1];
+            }
+            // messages into (ip, jp): from (ip-1, jp) [lane k-1, step t-1],
+            // (ip, jp-1) [own lane, step t-1], (ip-1, jp-1) [lane k-1, step t-2]
+            const float mu = ((qu + dpp_shr1(xu.x, mv)) + me) + dpp_shr1(xu.y, mevp);
+            mevp = mev;
+            const bool upd = cu.w >= 0.0f;
+            mv = upd ? mu * cu.x : 0.0f;
+            me = upd ? mu * cu.y : 0.0f;
+            mev = upd ? mu * cu.z : 0.0f;
+            rv[64 * u] = upd ? mu * cu.w : mu;
+            pb[2 * u] = make_float2(mv, mev);
+          }
+        }
+        lds_barrier();
+      }
+    } else if (wave == 1) {
+      // lam of columns 8n + 8 .. 8n + 15
+      const float* __restrict__ L = lam + sh.toff + col(0);  // the next column to load
+      int jl = 0;
+      const auto load = [&](float (&q)[AB]) {
 #pragma unroll
-      for (int u = 0; u < ADJ_PF; ++u) {
-        const int t = t0 + u;
-        float xv = 0.0f, xe = 0.0f;
-        if (up) {
+        for (int u = 0; u < AB; ++u) {
+          q[u] = L[(unsigned)i];
+          L += next(jl++);
+        }
+      };
+      float qa[AB], qb[AB];
+      load(qa);
+      load(qb);
+      const auto move = [&](int n, float (&q)[AB]) {
+        const int c_in = (n + 1) * AB;
+        if (c_in < 0) return;
+        const unsigned c = (unsigned)(c_in % AT) + lane;
+#pragma unroll
+        for (int u = 0; u < AB; ++u) ringV[wrap(c + u, AT) * 64 + lane] = q[u];
+        load(q);
+      };
+      for (int n = n_first; n <= n_last; n += 2) {
+        move(n, qa);
+        lds_barrier();
+        if (n + 1 <= n_last) {
+          move(n + 1, qb);
+          lds_barrier();
+        }
+      }
+    } else if (wave == 2) {
+      // traveltimes of columns 8n + 17 .. 8n + 24
+      const double* __restrict__ Tn = Tnew + sh.toff;
+      const double* __restrict__ To = Told + sh.toff;
+      int jl = (n_first + 2) * AB + 1;
+      const double* __restrict__ pn = Tn + col(jl);  // the next column to load
+      const double* __restrict__ po = To + col(jl);
+      const auto load = [&](double (&a)[AB], double (&b)[AB]) {
+#pragma unroll
+        for (int u = 0; u < AB; ++u) {
+          a[u] = pn[(unsigned)i];
+          b[u] = po[(unsigned)i];
+          const int d = next(jl++);
+          pn += d;
+          po += d;
+        }
+      };
+      double qa[2][AB], qb[2][AB];
+      load(qa[0], qa[1]);
+      load(qb[0], qb[1]);
+      const auto move = [&](int n, double (&q)[2][AB]) {
+        const int c_in = (n + 2) * AB + 1;
+        const unsigned c = (unsigned)((c_in + AT) % AT) + lane;
+#pragma unroll
+        for (int u = 0; u < AB; ++u)
+          ringT[wrap(c + u, AT) * 65 + lane] = __longlong_as_double(
+              __double_as_longlong(q[0][u]) | (q[0][u] < q[1][u] ? (long long)0x8000000000000000ull : 0));
+        load(q[0], q[1]);
+      };
+      for (int n = n_first; n <= n_last; n += 2) {
+        move(n, qa);
+        lds_barrier();
+        if (n + 1 <= n_last) {
+          move(n + 1, qb);
+          lds_barrier();
+        }
+      }
+    } else if (wave == 3) {
+      gword* xme = (gword*)(xw + ((size_t)ks * nstr + r) * ldx);
+      const gword* xup = (const gword*)(xw + ((size_t)ks * nstr + max(r - 1, 0)) * ldx);
+      const double* __restrict__ Tb = Tnew + sh.toff + adj_ip(min(64 * r + 64, nzz - 1), SA, nzz);
+      const int u = lane & (AB - 1);
+      bool gave_up = false;
+      double below = Tb[col((n_first + 2) * AB + 1 + u)];
+      for (int n = n_first; n <= n_last; ++n) {
+        // publish block n - 1's last row: column 8(n - 1) + u - 63
+        if (n >= 1 && n <= NBLK && r + 1 < nstr) {
+          const int jp = (n - 1) * AB + u - 63;
+          const float2 m = pub[(n - 1) & 1][u][0];
+          if (lane < AB && jp >= 0 && jp < nxx) {
+            __hip_atomic_store(xme + 2 * jp, walk_word(__float_as_uint(m.x), tag), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(xme + 2 * jp + 1, walk_word(__float_as_uint(m.y), tag), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+        // the upper strip's messages of step t = 8(n + 1) + u: to the row below
+        // of column t (word 2t), to the diagonal of column t - 1 (word 2t - 1);
+        // strip 0 and the columns no strip publishes read zero
+        const int t = (n + 1) * AB + u;
+        float2 x = make_float2(0.0f, 0.0f);
+        if (r > 0 && n >= -1 && n + 1 < NBLK) {
           const bool nv = t < nxx, ne = t >= 1 && t <= nxx;
-          unsigned vw = __builtin_amdgcn_readlane((unsigned)bv, u);
-          unsigned vt = __builtin_amdgcn_readlane((unsigned)(bv >> 32), u);
-          unsigned ew = __builtin_amdgcn_readlane((unsigned)be, u);
-          unsigned et = __builtin_amdgcn_readlane((unsigned)(be >> 32), u);
-          for (int it = 0; !gave_up && ((nv && vt != tag) || (ne && et != tag)); ++it) {
+          const gword* pv = xup + 2 * min(t, nxx - 1);
+          const gword* pe = xup + max(2 * min(t, nxx) - 1, 0);
+          for (int it = 0;; ++it) {
+            const unsigned long long v = __hip_atomic_load(pv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long e = __hip_atomic_load(pe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            x = make_float2(nv ? __uint_as_float((unsigned)v) : 0.0f, ne ? __uint_as_float((unsigned)e) : 0.0f);
+            if (gave_up ||
+                __all((!nv || (unsigned)(v >> 32) == tag) && (!ne || (unsigned)(e >> 32) == tag)))
+              break;
             if (it > WALK_SPIN) {
               if (lane == 0) atomicOr(ctl + 1, 1);
               gave_up = true;
               break;
             }
             __builtin_amdgcn_s_sleep(1);
-            const unsigned long long v = __hip_atomic_load(wv(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long e = __hip_atomic_load(we(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            vw = __builtin_amdgcn_readfirstlane((unsigned)v);
-            vt = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-            ew = __builtin_amdgcn_readfirstlane((unsigned)e);
-            et = __builtin_amdgcn_readfirstlane((unsigned)(e >> 32));
           }
-          xv = nv ? __uint_as_float(vw) : 0.0f;
-          xe = ne ? __uint_as_float(ew) : 0.0f;
         }
-        // messages into (ip, jp): from (ip-1, jp) [lane k-1, step t-1],
-        // (ip, jp-1) [own lane, step t-1], (ip-1, jp-1) [lane k-1, step t-2]
-        const float in_v = dpp_shr1(xv, mv);
-        const float in_ev = dpp_shr1(xe, mevp);
-        const float mu = ((ql[u] + in_v) + me) + in_ev;
-        mevp = mev;
-        const float4 cf = qc[u];
-        const bool upd = cf.w >= 0.0f;
-        mv = upd ? mu * cf.x : 0.0f;
-        me = upd ? mu * cf.y : 0.0f;
-        mev = upd ? mu * cf.z : 0.0f;
-        lam_out[base + (size_t)t * 64] = upd ? 0.0f : mu;
-        gc[base + (size_t)t * 64] = upd ? mu * cf.w : 0.0f;
-        const int jp = t - 63;
-        if (pub && jp >= 0 && jp < nxx) {
-          __hip_atomic_store(xme + 2 * jp, walk_word(__float_as_uint(mv), tag), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(xme + 2 * jp + 1, walk_word(__float_as_uint(mev), tag), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
+        if (lane < AB) {
+          xin[(n + 1) & 1][u] = x;
+          const int jp = (n + 2) * AB + 1 + u;
+          if (jp >= 0) ringT[wrap((unsigned)(jp % AT + 64), AT) * 65 + 64] = below;
         }
-        // reload the slot after its last use (it keeps its register)
-        const int tn = min(t + ADJ_PF, NTP - 1);
-        ql[u] = lam_in[base + (size_t)tn * 64];
-        qc[u] = coef[base + (size_t)tn * 64];
+        below = Tb[col((n + 3) * AB + 1 + u)];
+        lds_barrier();
       }
-    };
-    unsigned long long av, ae, bv, be;
-    xload(0, av, ae);
-    __builtin_amdgcn_s_waitcnt(0);  // once per strip (see k_fwd64_sweep)
-    for (int t0 = 0; t0 < NTP; t0 += 2 * ADJ_PF) {
-      xload(t0 + ADJ_PF, bv, be);
-      block(t0, av, ae);
-      if (t0 + ADJ_PF >= NTP) break;  // NTP is a multiple of ADJ_PF only
-      xload(t0 + 2 * ADJ_PF, av, ae);
-      block(t0 + ADJ_PF, bv, be);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Slowness contributions of sweep s onto padded cell (i, j): the nodes
-// (i + di, j + dj) whose code marks offset (di, dj), in a fixed order.  One
-// workgroup per (strip rs, block of ADJ_CB reverse-local columns, shot) owns
-// the cells whose nodes lie in the block: it first copies the block's
-// entries, with one row and one column of halo on each side, from the
-// strip-skewed layout into LDS by column (each step a contiguous run of
-// lanes), then sums each cell's contributions from LDS, a wave per column
-// with lane = row, so the cell updates are contiguous.
-template <int SA, int SB>
-__global__ __launch_bounds__(256) void k_adj_fold(const AdjShot* __restrict__ shots, int nzz, int nstr,
-                                                  const float* __restrict__ gc, const uint8_t* __restrict__ code,
-                                                  float* __restrict__ gshot) {
-  constexpr int W = ADJ_CB + 2, H = 66;  // columns jp0-1 .. jp0+ADJ_CB, rows 64rs-1 .. 64rs+64
-  __shared__ float G[W][H];
-  __shared__ uint8_t C[W][H];
-  const AdjShot sh = shots[blockIdx.y];
-  const int nxx = sh.sd.nxx, NTP = sh.NTP;
-  const int rs = (int)(blockIdx.x % (unsigned)nstr), jp0 = (int)(blockIdx.x / (unsigned)nstr) * ADJ_CB;
-  if (jp0 >= nxx) return;  // whole workgroup: blocks past this shot's width
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int ip = 64 * rs + lane;
-  // the strip's own rows: step t = jp0 - 1 + e/64, lane e%64
-  const size_t sbase = sh.koff + (size_t)rs * NTP * 64;
-  for (int e = threadIdx.x; e < (W + 63) * 64; e += 256) {
-    const int t = jp0 - 1 + (e >> 6), jp = t - lane;
-    if (jp < max(jp0 - 1, 0) || jp > jp0 + ADJ_CB || jp >= nxx || ip >= nzz) continue;
-    const size_t ko = sbase + (size_t)t * 64 + lane;
-    G[jp - jp0 + 1][lane + 1] = gc[ko];
-    C[jp - jp0 + 1][lane + 1] = code[ko];
-  }
-  // halo rows: the last row of strip rs-1 and the first of strip rs+1
-  if (threadIdx.x < 2 * W) {
-    const int h = threadIdx.x / W, jp = jp0 - 1 + threadIdx.x % W;
-    const int iph = h == 0 ? 64 * rs - 1 : 64 * rs + 64;
-    if (iph >= 0 && iph < nzz && jp >= 0 && jp < nxx) {
-      const size_t ko = sh.koff + adj_kidx(iph, jp, NTP);
-      G[jp - jp0 + 1][h == 0 ? 0 : H - 1] = gc[ko];
-      C[jp - jp0 + 1][h == 0 ? 0 : H - 1] = code[ko];
-    }
-  }
-  __syncthreads();
-  for (int col = w; col < ADJ_CB; col += 4) {
-    const int jp = jp0 + col;
-    if (ip >= nzz || jp >= nxx) continue;
-    const int i = adj_ip(ip, SA, nzz), j = adj_jp(jp, SB, nxx);
-    float acc = 0.0f;
+    } else if (wave < 4 + ADJ_OUT) {
+      // the block of columns whose last node block n - 1 took (8n - 72 .. 8n - 65) leaves (these
+      // waves load nothing from memory, so they never wait for a store)
+      constexpr int C = AB / ADJ_OUT;
+      const int u0 = (wave - 4) * C;
+      const bool row = ip < nzz;
+      for (int n = n_first; n <= n_last; ++n) {
+        const int c_out = (n - 1) * AB - 64 + u0;
+        if (c_out + C > 0 && c_out < nxx) {
+          float v[C];
+          unsigned cd[C];
+          const unsigned c = (unsigned)((c_out + AT) % AT) + lane;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int di = c & 1, dj = c >> 1;
-      const int ni = i + di, nj = j + dj;
-      if (ni >= 1 && ni <= nzz - 2 && nj >= 1 && nj <= nxx - 2) {
-        // node (ni, nj) in reverse-local coordinates, within the LDS window
-        const int r = adj_ip(ni, SA, nzz) - 64 * rs + 1, q = adj_jp(nj, SB, nxx) - jp0 + 1;
-        const int m = C[q][r];
-        if (m & (1 << c)) acc += (m & (m - 1)) ? 0.5f * G[q][r] : G[q][r];
+          for (int u = 0; u < C; ++u) {
+            const unsigned o = wrap(c + u, AT) * 64 + lane;
+            v[u] = ringV[o];
+            cd[u] = ringC[o];
+          }
+          const size_t o = sh.toff + col(c_out);
+          float* __restrict__ L = lam + o;
+          float* __restrict__ G = g + o;
+          uint8_t* __restrict__ Cd = code + o;
+          if (row) {
+#pragma unroll
+            for (int u = 0; u < C; ++u) {
+              if (c_out + u >= 0 && c_out + u < nxx) {
+                const bool upd = (cd[u] & ADJ_UPD) != 0;
+                L[(unsigned)i] = upd ? 0.0f : v[u];
+                G[(unsigned)i] = upd ? v[u] : 0.0f;
+                Cd[(unsigned)i] = (uint8_t)(cd[u] & 15u);
+              }
+              const int d = next(c_out + u);
+              L += d;
+              G += d;
+              Cd += d;
+            }
+          }
+        }
+        lds_barrier();
+      }
+    } else {
+      // slowness of step t: the reference cell of (ip, jp) is cell row ip of the
+      // opposite orientation, so step t's are consecutive in its skewed copy
+      // (column sig); the z-other cell is the previous step's; the x-other cell
+      // lane k-1's previous step's (lane 0: the upper strip's last row, 63 steps on).
+      // Where a column is clamped, by s_at.
+      constexpr int C = AB / ADJ_COEF;
+      const int u0 = (wave - 4 - ADJ_OUT) * C;
+      const int pitch = (SB > 0 ? -1 : 1) * sk.KP;  // words from one step's column to the next's
+      const unsigned rowk = (unsigned)min(64 * r + lane, sk.KP - 1);
+      // the x-other cell relative to the lowest of the lanes' columns
+      const int lead = lane == 0 && r > 0 ? 64 : 0;
+      const unsigned up_off = rowk - (lane == 0 && r == 0 ? 0u : 1u) + (unsigned)((SB > 0 ? 64 - lead : lead) * sk.KP);
+      const int i1 = i - (SA + 1) / 2;
+      typedef __attribute__((address_space(1))) const float cfloat;
+      // step u0's column (the pointers advance a block at a time)
+      cfloat* bp = (cfloat*)sk.base + (long long)(sh.sd.x0 + (SB > 0 ? nxx - 2 + 63 : 0) + SK_OFF) * sk.KP + (long long)u0 * pitch;
+      const int jbase = (SB > 0 ? nxx - 2 : 0) - sh.sd.sofs;
+      float sr[C], sz[C], sx[C];
+      const auto load = [&](int v, int t) {
+        // columns t - 64 .. t unclamped
+        if (sk.base && (SB > 0 ? jbase - t >= 0 && jbase - t + 64 <= sh.sd.smax
+                               : jbase + t - 64 >= 0 && jbase + t <= sh.sd.smax)) {
+          cfloat* b = bp + (long long)v * pitch;
+          cfloat* z = b - pitch;
+          sr[v] = b[rowk];
+          sz[v] = z[rowk];
+          sx[v] = (SB > 0 ? z + 64 * (long long)pitch : z)[up_off];
+        } else {
+          const int jp = min(max(t - lane, 1), nxx - 2);
+          const int j1 = adj_jp(jp, SB, nxx) - (SB + 1) / 2;
+          const int i1c = min(max(i1, 0), nzz - 1), i2c = min(max(i1 + SA, 0), nzz - 1);
+          sr[v] = s_at(sh.sd, nzz, i1c, j1);
+          sz[v] = s_at(sh.sd, nzz, i1c, j1 + SB);
+          sx[v] = s_at(sh.sd, nzz, i2c, j1);
+        }
+      };
+#pragma unroll
+      for (int v = 0; v < C; ++v) load(v, u0 + v);
+      for (int n = n_first; n <= n_last; ++n) {
+        if (n >= -1 && n + 1 < NBLK) {
+          bp += AB * (long long)pitch;
+#pragma unroll
+          for (int v = 0; v < C; ++v) {
+            const int t = (n + 1) * AB + u0 + v;
+            const double sref = (double)sr[v], szo = (double)sz[v], sxo = (double)sx[v];
+            const unsigned o0 = (unsigned)(t % AT), o1 = wrap(o0 + 1, AT), o2 = wrap(o0 + 2, AT);
+            const double tn = ringT[o0 * 65 + lane], te = ringT[o1 * 65 + lane], tv = ringT[o1 * 65 + lane + 1],
+                         tev = ringT[o2 * 65 + lane + 1];
+            // (a column before the grid holds another step's or nothing)
+            const bool upd = t >= lane && __double2hiint(tn) < 0;
+            AdjCoef a{make_float4(0.0f, 0.0f, 0.0f, -1.0f), 0};
+            if (__any(upd)) {
+              a = adj_local<SA, SB>(fabs(tn), fabs(tv), fabs(te), fabs(tev), sref, szo, sxo, upd, K);
+              if (upd) a.code |= ADJ_UPD;
+            }
+            load(v, t + AB);
+            cf[(n + 1) & 1][u0 + v][lane] = a.c;
+            ringC[o0 * 64 + lane] = (uint8_t)a.code;
+          }
+        }
+        lds_barrier();
       }
     }
-    gshot[sh.toff + i + (size_t)j * nzz] += acc;
   }
 }
 
-// T0 = S(node) * distance on the source stencil: dT0/dS(node) = distance.
-__global__ void k_adj_source(const AdjShot* __restrict__ shots, int nshots, int nzz, double dx, double dz,
-                             const float* __restrict__ lam0, float* __restrict__ gshot) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nshots * 9) return;
-  const AdjShot sh = shots[t / 9];
-  const int ii = (t % 9) % 3, jj = (t % 9) / 3;
+// Per-shot slowness gradient on padded cells: cell (i, j) receives, sweep 3
+// first, the contributions g of the nodes (i + di, j + dj) whose code marks
+// offset (di, dj), in a fixed order, then the source initialisation's (T0 =
+// S(node) * distance on the source stencil).  A wave takes 64 rows of ADJ_FC
+// consecutive columns, so a node column is read once for the two cell columns
+// it contributes to, and adds all four sweeps in one pass: 0.29 ms for 128 shots
+// of 301 x 1201 (28 B per node), against 4 x 0.30 with a pass per sweep.
+constexpr int ADJ_FC = 8;
+
+__global__ __launch_bounds__(256) void k_adj_fold(const AdjShot* __restrict__ shots, int nzz, size_t tsize, double dx,
+                                                  double dz, const float* __restrict__ g,
+                                                  const uint8_t* __restrict__ code, const float* __restrict__ lam,
+                                                  float* __restrict__ gshot) {
+  const AdjShot sh = shots[blockIdx.z];
+  const int nxx = sh.sd.nxx;
+  const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int j0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * ADJ_FC;
+  if (j0 >= nxx || i >= nzz) return;
+  const bool r0 = i >= 1 && i <= nzz - 2, r1 = i + 1 <= nzz - 2;  // rows i, i + 1 interior
+  const size_t row1 = i + 1 < nzz ? 1 : 0;
+  // the previous node column's contributions to this cell column: nodes (i, j)
+  // and (i + 1, j), per sweep
+  float pa[4], pb[4];
   const int sIdx = (int)(((double)sh.sd.sx + 0.5 * dx) / dx) + NB;
   const int sIdz = (int)(((double)sh.sd.sz + 0.5 * dz) / dz) + NB;
-  const int zi = sIdz + (ii - 1), xi = sIdx + (jj - 1);
-  const double ddx = (double)(xi - NB) * dx - (double)sh.sd.sx;
-  const double ddz = (double)(zi - NB) * dz - (double)sh.sd.sz;
-  const float lam = lam0[sh.koff + adj_kidx(adj_ip(zi, 1, nzz), adj_jp(xi, 1, sh.sd.nxx), sh.NTP)];
-  gshot[sh.toff + zi + (size_t)xi * nzz] += lam * (float)sqrt(ddx * ddx + ddz * ddz);
+#pragma unroll
+  for (int q = 0; q <= ADJ_FC; ++q) {
+    const int nj = j0 + q;
+    const bool in = nj >= 1 && nj <= nxx - 2;
+    float ga[4], gb[4];
+    unsigned ma[4], mb[4];
+    const size_t o = sh.toff + i + (size_t)min(nj, nxx - 1) * nzz;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      ga[s] = g[s * tsize + o];
+      gb[s] = g[s * tsize + o + row1];
+      ma[s] = code[s * tsize + o];
+      mb[s] = code[s * tsize + o + row1];
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for (int s = 3; s >= 0; --s) {
+      const unsigned a = in && r0 ? ma[s] : 0u, b = in && r1 ? mb[s] : 0u;
+      const float fa = (a & (a - 1)) ? 0.5f * ga[s] : ga[s], fb = (b & (b - 1)) ? 0.5f * gb[s] : gb[s];
+      if (q > 0) {
+        float acc = pa[s] + pb[s];
+        acc += (a & 4u) ? fa : 0.0f;
+        acc += (b & 8u) ? fb : 0.0f;
+        sum += acc;
+      }
+      pa[s] = (a & 1u) ? fa : 0.0f;
+      pb[s] = (b & 2u) ? fb : 0.0f;
+    }
+    const int j = nj - 1;  // the cell column that is complete
+    if (q > 0 && j < nxx) {
+      const size_t c = sh.toff + i + (size_t)j * nzz;
+      if (abs(i - sIdz) <= 1 && abs(j - sIdx) <= 1) {
+        const double ddx = (double)(j - NB) * dx - (double)sh.sd.sx;
+        const double ddz = (double)(i - NB) * dz - (double)sh.sd.sz;
+        sum += lam[c] * (float)sqrt(ddx * ddx + ddz * ddz);
+      }
+      gshot[c] = sum;
+    }
+  }
 }
 
-// d/ds of the unpadded model: every padded node of every shot maps to the
+// d/ds of the unpadded model: every padded cell of every shot maps to the
 // model cell it replicates (rows clamped to the model, columns clamped to the
 // shot's window); sums in fp64, shots in order.  fixed_border: the model's
 // border was uploaded as given (not the replication of its edges), so its
 // rows, and the border columns of shots on the whole model, are constants
 // with no derivative; a window's own replicated columns still fold.
+//
+// A cell on an edge takes 4 padded cells of each shot and a corner 16, one
+// away from the edges a single one; with a loop over them in the cell's own thread,
+// no two shots' loads are in flight together.  So k_adj_border first sums each
+// shot's edge cells, and k_adj_reduce adds one value a shot and cell, those of
+// ADJ_RS shots loaded together (128 shots of 301 x 1201: 0.42 ms in one kernel, 0.027 + 0.095 now).
+// edge: [shot][row 0: w][row nz-1: w][column 0: nz][column w-1: nz]; where the
+// rows have a border, their corners are read from the rows' part.
+constexpr int ADJ_RS = 16;
+
+struct EdgeRange {
+  int lo, hi;  // padded indices of the cells that map to cell c of n
+};
+__device__ __forceinline__ EdgeRange edge_range(int c, int n, bool fixed) {
+  return {c == 0 && !fixed ? 0 : c + NB, c == n - 1 && !fixed ? n - 1 + 2 * NB : c + NB};
+}
+
+__global__ __launch_bounds__(256) void k_adj_border(const AdjShot* __restrict__ shots, int nz, int nzz,
+                                                    const float* __restrict__ gshot, double* __restrict__ edge,
+                                                    int pitch, int fixed_border) {
+  const AdjShot& sh = shots[blockIdx.y];
+  const int w = sh.sd.w, e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= 2 * (w + nz)) return;
+  const bool cfix = fixed_border && sh.sd.sofs == 0;  // a whole-model shot reads the border as given
+  const int c = e < 2 * w ? e : e - 2 * w;
+  const int iz = e < 2 * w ? (c < w ? 0 : nz - 1) : c < nz ? c : c - nz;
+  const int lq = e < 2 * w ? (c < w ? c : c - w) : c < nz ? 0 : w - 1;
+  const EdgeRange p = edge_range(iz, nz, fixed_border), q = edge_range(lq, w, cfix);
+  const float* __restrict__ gs = gshot + sh.toff;
+  double acc = 0.0;
+  for (int j = q.lo; j <= q.hi; ++j)
+    for (int i = p.lo; i <= p.hi; ++i) acc += (double)gs[i + (size_t)j * nzz];
+  edge[(size_t)blockIdx.y * pitch + e] = acc;
+}
+
 __global__ __launch_bounds__(256) void k_adj_reduce(const AdjShot* __restrict__ shots, int nshots, int nz,
                                                     int nx, int nzz, const float* __restrict__ gshot,
+                                                    const double* __restrict__ edge, int pitch,
                                                     double* __restrict__ grad, int fixed_border) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= nz * nx) return;
   const int iz = idx % nz, ix = idx / nz;
-  const int plo = (iz == 0 && !fixed_border) ? 0 : iz + NB;
-  const int phi = (iz == nz - 1 && !fixed_border) ? nz - 1 + 2 * NB : iz + NB;
+  const bool redge = !fixed_border && (iz == 0 || iz == nz - 1);
   double acc = 0.0;
-  for (int s = 0; s < nshots; ++s) {
-    const int x0 = shots[s].sd.x0, w = shots[s].sd.w;
-    if (ix < x0 || ix >= x0 + w) continue;
-    const int lq = ix - x0;
-    const bool cfix = fixed_border && shots[s].sd.sofs == 0;  // a whole-model shot reads the border as given
-    const int qlo = (lq == 0 && !cfix) ? 0 : lq + NB;
-    const int qhi = (lq == w - 1 && !cfix) ? w - 1 + 2 * NB : lq + NB;
-    const float* __restrict__ g = gshot + shots[s].toff;
-    for (int q = qlo; q <= qhi; ++q)
-      for (int p = plo; p <= phi; ++p) acc += (double)g[p + (size_t)q * nzz];
+  for (int s0 = 0; s0 < nshots; s0 += ADJ_RS) {
+    double v[ADJ_RS];
+#pragma unroll
+    for (int u = 0; u < ADJ_RS; ++u) {
+      const int s = min(s0 + u, nshots - 1);
+      const AdjShot& sh = shots[s];
+      const int lq = ix - sh.sd.x0, w = sh.sd.w;
+      const bool in = s0 + u < nshots && lq >= 0 && lq < w;
+      const bool cedge = (lq == 0 || lq == w - 1) && !(fixed_border && sh.sd.sofs == 0);
+      v[u] = (gshot + sh.toff)[(unsigned)(iz + NB) + (unsigned)(min(max(lq, 0), w - 1) + NB) * (unsigned)nzz];
+      if (in && (redge || cedge))
+        v[u] = edge[(size_t)s * pitch + (redge ? (iz == 0 ? 0 : w) + lq : 2 * w + (lq == 0 ? 0 : nz) + iz)];
+      if (!in) v[u] = 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < ADJ_RS; ++u) acc += v[u];
   }
   grad[idx] = acc;
 }
@@ -917,52 +1076,32 @@ void launch_picks64(const AdjShot* shots, const int* rec_shot, const float* rx, 
                      dz, T4, out);
 }
 
-void launch_adj_coef(int sweep, const AdjShot* shots, int nshots, int nstr, int max_nxx, int nzz, double dx,
-                     double dz, const double* Tnew, const double* Told, const float* lam_src, float* lam_dst,
-                     float4* coef, uint8_t* code, hipStream_t st) {
-  const dim3 grid(nstr * ((max_nxx + ADJ_CB - 1) / ADJ_CB), nshots);
-  const int pa = adj_a(sweep + 1), pb = adj_b(sweep + 1);
-  const ConstsD k = consts_d(dx, dz);
-  switch (sweep) {
-    case 0: hipLaunchKernelGGL((k_adj_coef<1, 1>), grid, dim3(256), 0, st, shots, nzz, nstr, k, Tnew, Told, pa, pb, lam_src, lam_dst, coef, code); break;
-    case 1: hipLaunchKernelGGL((k_adj_coef<-1, 1>), grid, dim3(256), 0, st, shots, nzz, nstr, k, Tnew, Told, pa, pb, lam_src, lam_dst, coef, code); break;
-    case 2: hipLaunchKernelGGL((k_adj_coef<1, -1>), grid, dim3(256), 0, st, shots, nzz, nstr, k, Tnew, Told, pa, pb, lam_src, lam_dst, coef, code); break;
-    default: hipLaunchKernelGGL((k_adj_coef<-1, -1>), grid, dim3(256), 0, st, shots, nzz, nstr, k, Tnew, Told, pa, pb, lam_src, lam_dst, coef, code); break;
-  }
-}
-
-void launch_adj_sweep(const AdjShot* shots, int nshots, int nstr, const float* lam_in, const float4* coef,
-                      float* lam_out, float* gc, int* walk_ctl, unsigned long long* walk_x, int ldx, unsigned tag,
+void launch_adj_sweep(int sweep, const AdjShot* shots, int nshots, int nzz, int nstr, double dx, double dz,
+                      const SkewView& skew_opposite, const double* Tnew, const double* Told, float* lam, float* g,
+                      uint8_t* code, int* walk_ctl, unsigned long long* walk_x, int ldx, unsigned tag,
                       hipStream_t st) {
+  const ConstsD k = consts_d(dx, dz);
   hipLaunchKernelGGL(k_walk_begin, dim3(1), dim3(64), 0, st, walk_ctl);
-  const int grid = std::min(nshots * nstr, 4096);
-  hipLaunchKernelGGL(k_adj_sweep, dim3(grid), dim3(64), 0, st, shots, nshots, nstr, lam_in, coef, lam_out, gc,
-                     walk_ctl, walk_x, ldx, tag);
+  const int grid = std::min(nshots * nstr, 256);  // one workgroup per CU (LDS)
+  auto* f = sweep == 0 ? k_adj_sweep<1, 1> : sweep == 1 ? k_adj_sweep<-1, 1> : sweep == 2 ? k_adj_sweep<1, -1>
+                                                                                        : k_adj_sweep<-1, -1>;
+  hipLaunchKernelGGL(f, dim3(grid), dim3(ADJ_THREADS), 0, st, shots, nshots, nzz, nstr, k, skew_opposite, Tnew, Told, lam, g,
+                     code, walk_ctl, walk_x, ldx, tag);
 }
 
-void launch_adj_fold(int sweep, const AdjShot* shots, int nshots, int nstr, int max_nxx, int nzz, const float* gc,
-                     const uint8_t* code, float* gshot, hipStream_t st) {
-  const dim3 grid(nstr * ((max_nxx + ADJ_CB - 1) / ADJ_CB), nshots);
-  switch (sweep) {
-    case 0: hipLaunchKernelGGL((k_adj_fold<1, 1>), grid, dim3(256), 0, st, shots, nzz, nstr, gc, code, gshot); break;
-    case 1: hipLaunchKernelGGL((k_adj_fold<-1, 1>), grid, dim3(256), 0, st, shots, nzz, nstr, gc, code, gshot); break;
-    case 2: hipLaunchKernelGGL((k_adj_fold<1, -1>), grid, dim3(256), 0, st, shots, nzz, nstr, gc, code, gshot); break;
-    default: hipLaunchKernelGGL((k_adj_fold<-1, -1>), grid, dim3(256), 0, st, shots, nzz, nstr, gc, code, gshot); break;
-  }
+void launch_adj_fold(const AdjShot* shots, int nshots, int max_nxx, int nzz, size_t tsize, double dx, double dz,
+                     const float* g, const uint8_t* code, const float* lam, float* gshot, hipStream_t st) {
+  const dim3 grid((nzz + 63) / 64, (max_nxx + 4 * ADJ_FC - 1) / (4 * ADJ_FC), nshots);
+  hipLaunchKernelGGL(k_adj_fold, grid, dim3(256), 0, st, shots, nzz, tsize, dx, dz, g, code, lam, gshot);
 }
 
-void launch_adj_source(const AdjShot* shots, int nshots, int nzz, double dx, double dz, const float* lam0,
-                       float* gshot, hipStream_t st) {
-  const int n = nshots * 9;
-  hipLaunchKernelGGL(k_adj_source, dim3((n + 255) / 256), dim3(256), 0, st, shots, nshots, nzz, dx, dz, lam0,
-                     gshot);
-}
-
-void launch_adj_reduce(const AdjShot* shots, int nshots, int nz, int nx, int nzz, const float* gshot,
-                       double* grad, bool fixed_border, hipStream_t st) {
-  const int n = nz * nx;
+void launch_adj_reduce(const AdjShot* shots, int nshots, int nz, int nx, int nzz, int max_w, const float* gshot,
+                       double* edge, double* grad, bool fixed_border, hipStream_t st) {
+  const int n = nz * nx, pitch = 2 * (max_w + nz);
+  const dim3 grid((pitch + 255) / 256, nshots);
+  hipLaunchKernelGGL(k_adj_border, grid, dim3(256), 0, st, shots, nz, nzz, gshot, edge, pitch, fixed_border ? 1 : 0);
   hipLaunchKernelGGL(k_adj_reduce, dim3((n + 255) / 256), dim3(256), 0, st, shots, nshots, nz, nx, nzz, gshot,
-                     grad, fixed_border ? 1 : 0);
+                     edge, pitch, grad, fixed_border ? 1 : 0);
 }
 
 }  // namespace seisfat

@@ -141,12 +141,11 @@ void free_batch(seisfat_batch_s* b) {
   AdjState& a = b->adj;
   dfree(a.d_tab);
   dfree(a.d_T64);
-  dfree(a.d_lamA);
-  dfree(a.d_lamB);
-  dfree(a.d_coef);
+  dfree(a.d_lam);
+  dfree(a.d_g);
   dfree(a.d_code);
-  dfree(a.d_gc);
   dfree(a.d_gshot);
+  dfree(a.d_edge);
   dfree(a.d_seed_node);
   dfree(a.d_seed_ptr);
   dfree(a.d_seed_rec);
@@ -796,20 +795,14 @@ int adj_prepare(seisfat_batch_s* b) {
   const int nzz = h->nzz, nshots = b->nshots;
   A.nstr = (nzz + 63) / 64;
   A.tab.resize(nshots);
-  size_t koff = 0;
   A.max_nxx = 0;
   for (int k = 0; k < nshots; ++k) {
     AdjShot& s = A.tab[k];
     s.sd = b->iso[k];
     s.toff = b->toff[k];
-    const int nxx = s.sd.nxx;
-    s.NTP = (nxx + 63 + ADJ_PF - 1) / ADJ_PF * ADJ_PF;
-    s.koff = koff;
-    koff += (size_t)A.nstr * s.NTP * 64;
-    A.max_nxx = std::max(A.max_nxx, nxx);
+    A.max_nxx = std::max(A.max_nxx, s.sd.nxx);
   }
-  A.ksize = koff;
-  // pick seeds: (skewed node of the last reverse sweep, receiver, weight),
+  // pick seeds: (node, receiver, weight),
   // grouped by node with receivers in order
   struct Seed {
     size_t node;
@@ -837,8 +830,7 @@ int adj_prepare(seisfat_batch_s* b) {
     for (int pIdx = 0; pIdx < 4; ++pIdx)
       for (int pIdz = 0; pIdz < 4; ++pIdz) {
         const int ni = i + pIdz - 1, nj = j + pIdx - 1;
-        const size_t node =
-            s.koff + adj_kidx(adj_ip(ni, adj_a(3), nzz), adj_jp(nj, adj_b(3), s.sd.nxx), s.NTP);
+        const size_t node = s.toff + ni + (size_t)nj * nzz;
         es.push_back(Seed{node, r, (float)(wx[pIdx] * wz[pIdz])});
       }
   }
@@ -860,8 +852,9 @@ int adj_prepare(seisfat_batch_s* b) {
   int rc;
   const size_t tsize = b->tsize;
   if ((rc = dalloc(&A.d_tab, (size_t)nshots)) || (rc = dalloc(&A.d_T64, 5 * tsize)) ||
-      (rc = dalloc(&A.d_lamA, A.ksize)) || (rc = dalloc(&A.d_lamB, A.ksize)) || (rc = dalloc(&A.d_coef, A.ksize)) ||
-      (rc = dalloc(&A.d_code, A.ksize)) || (rc = dalloc(&A.d_gc, A.ksize)) || (rc = dalloc(&A.d_gshot, tsize)) ||
+      (rc = dalloc(&A.d_lam, tsize)) || (rc = dalloc(&A.d_g, 4 * tsize)) ||
+      (rc = dalloc(&A.d_code, 4 * tsize)) || (rc = dalloc(&A.d_gshot, tsize)) ||
+      (rc = dalloc(&A.d_edge, (size_t)nshots * 2 * (A.max_nxx - 2 * NB + h->nz))) ||
       (rc = dalloc(&A.d_seed_node, snode.size())) ||
       (rc = dalloc(&A.d_seed_ptr, sptr.size())) || (rc = dalloc(&A.d_seed_rec, srec.size())) ||
       (rc = dalloc(&A.d_seed_w, sw.size())) || (rc = dalloc(&A.d_w, (size_t)b->nrec)) || (rc = dalloc(&A.d_picks64, (size_t)b->nrec)) ||
@@ -880,13 +873,6 @@ int adj_prepare(seisfat_batch_s* b) {
     HIPCHK(hipMemcpyAsync(A.d_seed_rec, srec.data(), srec.size() * sizeof(int), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(A.d_seed_w, sw.data(), sw.size() * sizeof(float), hipMemcpyHostToDevice, st));
   }
-  // Entries of the skewed arrays outside every grid are never written and
-  // must read as zero.
-  HIPCHK(hipMemsetAsync(A.d_lamA, 0, A.ksize * sizeof(float), st));
-  HIPCHK(hipMemsetAsync(A.d_lamB, 0, A.ksize * sizeof(float), st));
-  HIPCHK(hipMemsetAsync(A.d_coef, 0, A.ksize * sizeof(float4), st));
-  HIPCHK(hipMemsetAsync(A.d_code, 0, A.ksize, st));
-  HIPCHK(hipMemsetAsync(A.d_gc, 0, A.ksize * sizeof(float), st));
   // ring nodes of every trajectory grid, and T0 off the source stencil, stay 1e6
   launch_fill_d(A.d_T64, 5 * tsize, 1e6, st);
   HIPCHK(hipGetLastError());
@@ -929,19 +915,18 @@ int enqueue_vjp(seisfat_batch_s* b, const float* d_w, double* d_grad, hipStream_
   if (!d_grad) return fail(SEISFAT_EINVAL, "null gradient pointer");
   if (b->nrec > 0 && !d_w) return fail(SEISFAT_EINVAL, "null cotangent pointer");
   const int nzz = h->nzz, ns = b->nshots;
-  launch_fill(A.d_lamB, A.ksize, 0.0f, st);
-  launch_adj_seed(A.d_seed_node, A.d_seed_ptr, A.d_seed_rec, A.d_seed_w, A.nseed, d_w, A.d_lamB, st);
-  launch_fill(A.d_gshot, b->tsize, 0.0f, st);
   const size_t ts = b->tsize;
+  launch_fill(A.d_lam, ts, 0.0f, st);
+  launch_adj_seed(A.d_seed_node, A.d_seed_ptr, A.d_seed_rec, A.d_seed_w, A.nseed, d_w, A.d_lam, st);
   for (int s = 3; s >= 0; --s) {
-    launch_adj_coef(s, A.d_tab, ns, A.nstr, A.max_nxx, nzz, h->dx, h->dz, A.d_T64 + (s + 1) * ts,
-                    A.d_T64 + s * ts, s == 3 ? nullptr : A.d_lamA, A.d_lamB, A.d_coef, A.d_code, st);
-    launch_adj_sweep(A.d_tab, ns, A.nstr, A.d_lamB, A.d_coef, A.d_lamA, A.d_gc, A.d_walk_ctl, A.d_walk_x,
-                     A.walk_ldx, A.walk_tag = A.walk_tag == 0xffffffffu ? 1 : A.walk_tag + 1, st);
-    launch_adj_fold(s, A.d_tab, ns, A.nstr, A.max_nxx, nzz, A.d_gc, A.d_code, A.d_gshot, st);
+    const SkewView skew = h->skew[3 - s].KP <= 1 << 20 ? h->skew[3 - s] : SkewView{nullptr, 0};
+    launch_adj_sweep(s, A.d_tab, ns, nzz, A.nstr, h->dx, h->dz, skew, A.d_T64 + (s + 1) * ts, A.d_T64 + s * ts, A.d_lam,
+                     A.d_g + s * ts, A.d_code + s * ts, A.d_walk_ctl, A.d_walk_x, A.walk_ldx,
+                     A.walk_tag = A.walk_tag == 0xffffffffu ? 1 : A.walk_tag + 1, st);
   }
-  launch_adj_source(A.d_tab, ns, nzz, h->dx, h->dz, A.d_lamA, A.d_gshot, st);
-  launch_adj_reduce(A.d_tab, ns, h->nz, h->nx, nzz, A.d_gshot, d_grad, !A.pad_replicated, st);
+  launch_adj_fold(A.d_tab, ns, A.max_nxx, nzz, ts, h->dx, h->dz, A.d_g, A.d_code, A.d_lam, A.d_gshot, st);
+  launch_adj_reduce(A.d_tab, ns, h->nz, h->nx, nzz, A.max_nxx - 2 * NB, A.d_gshot, A.d_edge, d_grad, !A.pad_replicated,
+                    st);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(b->ev_done, st));
   return SEISFAT_OK;

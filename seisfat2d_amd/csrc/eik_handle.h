@@ -60,14 +60,12 @@ struct AdjState {
   std::vector<AdjShot> tab;
   AdjShot* d_tab = nullptr;
   int nstr = 0, max_nxx = 0;
-  size_t ksize = 0;
   double* d_T64 = nullptr;  // fp64 trajectory: T0 (initial field) .. T4, tsize each
-  float* d_lamA = nullptr;
-  float* d_lamB = nullptr;
-  float4* d_coef = nullptr;
-  uint8_t* d_code = nullptr;
-  float* d_gc = nullptr;
-  float* d_gshot = nullptr;
+  float* d_lam = nullptr;   // adjoint of the traveltimes, tsize
+  float* d_g = nullptr;     // slowness contributions of every node, 4 sweeps x tsize
+  uint8_t* d_code = nullptr;  // the cells they go to
+  float* d_gshot = nullptr;  // per-shot gradient on padded cells, tsize
+  double* d_edge = nullptr;  // its sums onto the edge cells of each shot's window
   size_t* d_seed_node = nullptr;
   int* d_seed_ptr = nullptr;
   int* d_seed_rec = nullptr;
