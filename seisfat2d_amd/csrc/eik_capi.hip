@@ -986,20 +986,21 @@ int seisfat_eik_create(int nz, int nx, float dz, float dx, seisfat_eik_t* out) {
     const float divs[12] = {c.sum,    c.hyp,    c.dz,    c.dx,    c.zh_sum, c.zh_hyp,
                             c.zh_dz,  c.zh_dx,  c.zl_sum, c.zl_hyp, c.zl_dz,  c.zl_dx};
     float rec[4] = {};
-    int bad[4] = {1, 1, 1, 1};
+    int bad[5] = {1, 1, 1, 1, 1};  // the divisors, the square root
     float* d = nullptr;
-    hipError_t e2 = hipMalloc((void**)&d, 20 * sizeof(float));
+    hipError_t e2 = hipMalloc((void**)&d, 21 * sizeof(float));
     if (e2 == hipSuccess) e2 = hipMemcpy(d, divs, sizeof(divs), hipMemcpyHostToDevice);
-    if (e2 == hipSuccess) e2 = hipMemset(d + 16, 0, 4 * sizeof(int));
+    if (e2 == hipSuccess) e2 = hipMemset(d + 16, 0, 5 * sizeof(int));
     if (e2 == hipSuccess) {
       launch_recip(d, d + 12, 4, h->stream);
       launch_fastdiv_check(d, d + 4, d + 8, 4, (int*)(d + 16), h->stream);
+      launch_sqrt_check((int*)(d + 20), h->stream);
       e2 = hipStreamSynchronize(h->stream);
     }
     if (e2 == hipSuccess) e2 = hipMemcpy(rec, d + 12, sizeof(rec), hipMemcpyDeviceToHost);
     if (e2 == hipSuccess) e2 = hipMemcpy(bad, d + 16, sizeof(bad), hipMemcpyDeviceToHost);
     if (d) (void)hipFree(d);
-    h->kc.fastdiv = (bad[0] | bad[1] | bad[2] | bad[3]) == 0;
+    h->kc.fastdiv = (bad[0] | bad[1] | bad[2] | bad[3] | bad[4]) == 0;
     if (e2 != hipSuccess) {
       seisfat_eik_destroy(h);
       return fail(SEISFAT_EHIP, std::string("reciprocal setup: ") + hipGetErrorString(e2));

@@ -33,7 +33,8 @@ struct EikConsts {
   // divisors (see fdiv below)
   float zh_sum, zl_sum, zh_hyp, zl_hyp, zh_dz, zl_dz, zh_dx, zl_dx;
   // host-side: fdiv reproduces the correctly rounded quotient for all four
-  // divisors (checked exhaustively when the geometry is created)
+  // divisors, and sqrt_short the square root (checked exhaustively when the
+  // geometry is created)
   int fastdiv;
   // a node whose old traveltime and upwind neighbours are all TINF keeps
   // TINF: its 1-D candidates are >= TINF, branches B and C are not taken
@@ -89,11 +90,34 @@ __device__ __forceinline__ float rsqrt_rn(float x) {
   return (r2 > 0.0f) ? sup : t;
 }
 
+// The correctly rounded square root in six instructions instead of rsqrt_rn's
+// nine: one Newton step from the hardware's reciprocal root, whose residual is
+// exact.  By itself the step only has an error just above half a unit; that it
+// rounds right for every fraction with this hardware's estimate is checked
+// over two binades (k_sqrt_check), which the others repeat at a power of 4.
+// (With the other savings of eik_local_sel 64 -> 56 vector instructions a step:
+// one shot of 201 x 1001 902 -> 836 us, 256 shots 9.81 -> 9.70 ms.)
+// The estimate is bounded so that 0 gives 0; a negative radicand (estimate NaN,
+// bounded to -2^100) gives at least 2^100, which the minima that follow discard
+// like rsqrt_rn's NaN.
+__device__ __forceinline__ float sqrt_short(float x) {
+  // (radicands are above 2^-90 or 0)
+  const float y = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(x), -0x1p100f, 0x1p100f);
+  const float g = x * y;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+}
+
 // IEEE minNum of two non-NaN values without the sNaN-quieting canonicalise
 // the compiler would add for loaded operands (no operand here is a NaN).
 __device__ __forceinline__ float vmin(float a, float b) {
   float r;
   asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+__device__ __forceinline__ float vmax(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
   return r;
 }
 
@@ -242,7 +266,8 @@ __device__ __forceinline__ CellQ cell_q(float s, const EikConsts& k) {
 // h > 0, RN(h * min(a, b)) = min(RN(h * a), RN(h * b)), so the 1-D candidates
 // can use the cells' precomputed products.  Bit-identical to eik_local: the
 // selected lanes evaluate the same operations in the same order; the others
-// compute values that the selects discard.  FD: divisions by fdiv.  Returns
+// compute values that the selects discard.  FD: divisions by fdiv, the root by
+// sqrt_short.  Returns
 // min(told, eik_local): the minimum of told, both 1-D candidates, the 2-D
 // candidate and TINF (no operand is a NaN, so two three-way minima give the
 // same value as the nested pairwise ones).
@@ -258,14 +283,22 @@ __device__ __forceinline__ float eik_local_sel(float tv, float te, float tev, co
   // Branch A's four conditions as one test: for finite floats a, b,
   // RN(a - b) >= 0 exactly when a >= b (a difference of floats rounds to
   // zero only when it is zero), and a minimum is >= 0 exactly when every
-  // operand is.  B and C: with thr > 0 finite, 0 < d <= thr exactly when
-  // bits(d) - 1 < bits(thr) as unsigned words (positive floats order as their
-  // bit patterns; +0, -0 and negatives wrap to at least 0x7fffffff).
-  const bool cA = vmin3(te + r.dxs - tv, tv + r.dzs - te, vmin(de, dv)) >= 0.0f;
-  const bool cB = __float_as_uint(de) - 1u < __float_as_uint(r.thrB);
-  const bool cC = __float_as_uint(dv) - 1u < __float_as_uint(r.thrC);
+  // operand is.  B and C: with thr > 0 finite, 0 <= d <= thr exactly when
+  // bits(d) <= bits(thr) as unsigned words (floats order as their bit patterns,
+  // negatives above all; a difference is never -0).  The conditions exclude
+  // d = 0, which changes nothing: its candidate is t0 + h2 RN(sqrt(RN(s^2))) =
+  // t0 + h2 s, not below that axis' 1-D candidate, and where it takes C's place
+  // (de = 0 < dv <= thrC < s dx) branch A holds.
+  // EQH: dx s = dz s, so of the first two only the one for the larger of tv and
+  // te can fail.
+  const bool cA = EQH ? vmin3(vmin(te, tv) + r.dzs - vmax(te, tv), de, dv) >= 0.0f
+                      : vmin3(te + r.dxs - tv, tv + r.dzs - te, vmin(de, dv)) >= 0.0f;
+  const bool cB = __float_as_uint(de) <= __float_as_uint(r.thrB);
   // branch B precedes C (the reference's else-if order)
   const float dd = cB ? de : dv;
+  // EQH: the thresholds are equal, and dd, where cB holds, is below it
+  const bool cBC = EQH ? __float_as_uint(dd) <= __float_as_uint(r.thrB)
+                       : cB | (__float_as_uint(dv) <= __float_as_uint(r.thrC));
   const float h1 = EQH ? k.dz : (cB ? k.dz : k.dx);
   const float r1 = EQH ? k.r_dz : (cB ? k.r_dz : k.r_dx);
   const float zh1 = EQH ? k.zh_dz : (cB ? k.zh_dz : k.zh_dx);
@@ -274,17 +307,17 @@ __device__ __forceinline__ float eik_local_sel(float tv, float te, float tev, co
   const float t0 = cB ? te : tv;
   const float q = FD ? fdiv(dd, zh1, zl1) : rdiv(dd, h1, r1);
   const float ta = tev + te - tv;
-  const float tb = tev - te + tv;
+  const float tb = tv - de;  // RN(tev - te) = -de
   const float dab = ta - tb;
   // radicand a - b * c: A: 4 s^2 (dz2i + dx2i) - (dz2i dx2i dab) dab; B/C: s^2 - q q
   const float ra = cA ? r.s4 : r.s2;
   const float rb = cA ? k.prod * dab : q;
   const float rc = cA ? dab : q;
-  const float sq = rsqrt_rn(ra - rb * rc);
+  const float sq = FD ? sqrt_short(ra - rb * rc) : rsqrt_rn(ra - rb * rc);
   const float num = (tb * k.dz2i + ta * k.dx2i) + sq;
   const float tA = FD ? fdiv(num, k.zh_sum, k.zl_sum) : rdiv(num, k.sum, k.r_sum);
   const float tBC = t0 + h2 * sq;
-  const float t2D = cA ? tA : ((cB | cC) ? tBC : TINF);
+  const float t2D = cA ? tA : (cBC ? tBC : TINF);
   return vmin3(t1D, t2D, told);
 }
 

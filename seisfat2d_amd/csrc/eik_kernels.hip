@@ -218,8 +218,9 @@ __device__ __forceinline__ int skew_addr(const ShotDev& sd, int nxx, int NC, int
 // One step of a tile: lane k updates sweep-local node (kg, c0 + t - k).  The
 // step's old traveltime, upwind-row value and slowness cells are loaded by the
 // caller ahead of time (software pipelining across the solver's branches).
-// ALLCOLS: every column the tile visits is an interior node column, so only
-// the row test remains.
+// ALLCOLS: every column the tile visits is an interior node column; no test
+// remains then, since a row past the last only feeds others past it, and
+// neither the write-back nor another tile reads them.
 template <bool EQH, bool FD, bool ALLCOLS, bool XDPP = false, bool CONV = false>
 __device__ __forceinline__ void tile_step(float* __restrict__ sT, int tab, int t, int lane, bool row_ok, int c0,
                                           int NC,
@@ -228,13 +229,13 @@ __device__ __forceinline__ void tile_step(float* __restrict__ sT, int tab, int t
   const CellQ zo = cell_q<EQH, FD>(szo, k);  // this step's z-other cell, next step's reference cell
   const float tv = dpp_shr1(h, te);
   const int c = c0 + t - lane;
-  const bool act = ALLCOLS ? row_ok : (row_ok && (unsigned)c < (unsigned)NC);
+  const bool act = ALLCOLS || (row_ok && (unsigned)c < (unsigned)NC);
   // XDPP: lane k's x-other cell is lane k+1's z-other cell of this step; sxo
   // is then only lane 63's (times dx when EQH, where zo.dzs = dz*s = dx*s)
   const float dxs_xo = !XDPP ? k.dx * sxo : (EQH ? dpp_shl1(sxo, zo.dzs) : k.dx * dpp_shl1(sxo, szo));
   const float m = eik_local_sel<EQH, FD>(tv, te, tev, sref, zo.dzs, dxs_xo, k, told);  // min(told, candidates)
   const float res = act ? m : told;
-  if constexpr (CONV) chg = chg | (res < told);  // converged mode: did this lane lower a traveltime
+  if constexpr (CONV) chg = chg | (row_ok & (res < told));  // converged mode: did this lane lower a traveltime
   ring_at(sT, tab) = res;
   tev = tv;
   te = res;
@@ -1033,6 +1034,19 @@ __global__ void k_fastdiv_check(const float* __restrict__ b, const float* __rest
   if (flag) atomicOr(bad + d, 1);
 }
 
+// Exhaustive check of sqrt_short over the radicands of two binades, and 0,
+// against the IEEE square root: any other normal
+// radicand x 4^k gives the same root x 2^k (no operation of the step leaves the
+// normal range above 2^-90).
+__global__ void k_sqrt_check(int* __restrict__ bad) {
+  const unsigned u = (127u << 23) + blockIdx.x * blockDim.x + threadIdx.x;
+  const float x = u == 127u << 23 ? 0.0f : __uint_as_float(u);
+  const float y = __uint_as_float(u);
+  if (__float_as_uint(sqrt_short(x)) != __float_as_uint(sqrtf(x)) ||
+      __float_as_uint(sqrt_short(y)) != __float_as_uint(sqrtf(y)))
+    atomicOr(bad, 1);
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launchers.
 void launch_recip(const float* b, float* r, int n, hipStream_t st) {
@@ -1041,6 +1055,10 @@ void launch_recip(const float* b, float* r, int n, hipStream_t st) {
 
 void launch_fastdiv_check(const float* b, const float* zh, const float* zl, int n, int* bad, hipStream_t st) {
   hipLaunchKernelGGL(k_fastdiv_check, dim3(4096, n), dim3(256), 0, st, b, zh, zl, bad);
+}
+
+void launch_sqrt_check(int* bad, hipStream_t st) {
+  hipLaunchKernelGGL(k_sqrt_check, dim3((2u << 23) / 256), dim3(256), 0, st, bad);
 }
 
 void launch_fill(float* p, size_t n, float v, hipStream_t st) {
