@@ -138,6 +138,8 @@ void free_batch(seisfat_batch_s* b) {
   dfree(b->d_qp_b);
   dfree(b->d_ptiles);
   dfree(b->d_qoff);
+  dfree(b->d_strips);
+  dfree(b->d_soff);
   AdjState& a = b->adj;
   dfree(a.d_tab);
   dfree(a.d_T64);
@@ -178,9 +180,12 @@ int enqueue_solve(seisfat_batch_s* b, hipStream_t st, const Mark& mark) {
     if (sweeps == 0)
       if (int rc = mark(0)) return rc;
     int n = 0;
-    if (b->schedule == SEISFAT_SCHED_TILED && b->pairs && d_tab_b) {
-      n = launch_sweeps_pairs(d_tab, d_tab_b, b->d_ptiles, b->d_qoff, b->nstrips, nzz, b->kc, h->eqh, skew, b->pr,
-                              solve, st);
+    if (b->schedule == SEISFAT_SCHED_TILED && b->pairs && skew) {
+      n = launch_sweeps_strips(d_tab, d_tab_b, b->d_strips, b->d_soff, b->strips_most, b->nstrips, nzz, b->kc, h->eqh,
+                               skew, b->pr, solve, st);
+    } else if (b->schedule == SEISFAT_SCHED_TILED && b->pairs) {
+      n = launch_sweeps_pairs(d_tab, d_tab_b, b->d_ptiles, b->d_qoff, b->nstrips, nzz, b->kc, h->eqh, b->pr, solve,
+                              st);
     } else if (b->schedule == SEISFAT_SCHED_TILED) {
       n = launch_sweeps_persist(d_tab, b->d_tiles, b->ntiles, b->nstrips, nzz, b->kc, h->eqh, skew, true, b->pr,
                                 solve, st);
@@ -331,6 +336,35 @@ void build_pair_tiles(seisfat_batch_s* b, std::vector<int4>& pt, std::vector<int
     });
     for (const E& e : per[x]) pt.push_back(make_int4(e.k, e.r, e.bb, prio[e.k] | (e.which << 2)));
     qoff.push_back((int)pt.size());
+  }
+}
+
+// Strips of both sweeps of a fused pair, shots spread over the 8 XCDs by their
+// columns; an XCD's strips in the order of their place in their shot's chain
+// (first sweep's strips, then the second's), the widest shots' first, so every
+// strip follows those it waits for.
+void build_strips(seisfat_batch_s* b) {
+  const int n = b->nshots, NRS = b->nstrips;
+  std::vector<int> order(n);
+  for (int k = 0; k < n; ++k) order[k] = k;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return b->iso[a].nxx > b->iso[c].nxx; });
+  long long load[8] = {};
+  std::vector<std::vector<int>> per(8);
+  b->strip_blocks = 0;
+  for (int k : order) {
+    const int x = (int)(std::min_element(load, load + 8) - load);
+    per[x].push_back(k);
+    load[x] += b->iso[k].nxx;
+    b->strip_blocks += 2LL * NRS * ((b->iso[k].nxx - 2 + 63 + STRIP_BLOCK - 1) / STRIP_BLOCK);
+  }
+  b->strips.clear();
+  b->strip_qoff.assign(1, 0);
+  b->strips_most = 0;
+  for (int x = 0; x < 8; ++x) {
+    for (int p = 0; p < 2 * NRS; ++p)
+      for (int k : per[x]) b->strips.push_back(make_int4(k, p % NRS, p / NRS, 0));
+    b->strip_qoff.push_back((int)b->strips.size());
+    b->strips_most = std::max(b->strips_most, b->strip_qoff[x + 1] - b->strip_qoff[x]);
   }
 }
 
@@ -548,19 +582,25 @@ int create_batch(seisfat_eik_t h, int type, int schedule, int nshots, const seis
         b->iso_b[k].xh = b->iso[k].xh + words;
         b->iso_b[k].xc = b->iso[k].xc + words;
       }
-      std::vector<int4> pt;
-      std::vector<int> qoff;
-      build_pair_tiles(b, pt, qoff);
       TRY(dalloc(&b->d_iso_b, nshots));
-      TRY(dalloc(&b->d_ptiles, pt.size()));
-      TRY(dalloc(&b->d_qoff, qoff.size()));
       HIPCHK_B(hipMemcpyAsync(b->d_iso_b, b->iso_b.data(), nshots * sizeof(ShotDev), hipMemcpyHostToDevice,
                               h->stream));
-      HIPCHK_B(hipMemcpyAsync(b->d_ptiles, pt.data(), pt.size() * sizeof(int4), hipMemcpyHostToDevice, h->stream));
-      HIPCHK_B(hipMemcpyAsync(b->d_qoff, qoff.data(), qoff.size() * sizeof(int), hipMemcpyHostToDevice, h->stream));
-      // the host copies are read back only after the stream synchronises below
-      b->pair_tiles = std::move(pt);
-      b->pair_qoff = std::move(qoff);
+      if (type == SEISFAT_ANI) {
+        build_pair_tiles(b, b->pair_tiles, b->pair_qoff);
+        TRY(dalloc(&b->d_ptiles, b->pair_tiles.size()));
+        TRY(dalloc(&b->d_qoff, b->pair_qoff.size()));
+        HIPCHK_B(hipMemcpyAsync(b->d_ptiles, b->pair_tiles.data(), b->pair_tiles.size() * sizeof(int4),
+                                hipMemcpyHostToDevice, h->stream));
+        HIPCHK_B(hipMemcpyAsync(b->d_qoff, b->pair_qoff.data(), b->pair_qoff.size() * sizeof(int),
+                                hipMemcpyHostToDevice, h->stream));
+      }
+      build_strips(b);
+      TRY(dalloc(&b->d_strips, b->strips.size()));
+      TRY(dalloc(&b->d_soff, b->strip_qoff.size()));
+      HIPCHK_B(hipMemcpyAsync(b->d_strips, b->strips.data(), b->strips.size() * sizeof(int4), hipMemcpyHostToDevice,
+                              h->stream));
+      HIPCHK_B(hipMemcpyAsync(b->d_soff, b->strip_qoff.data(), b->strip_qoff.size() * sizeof(int),
+                              hipMemcpyHostToDevice, h->stream));
     }
     // the qP solve (anisotropic batches) runs after the isotropic one and
     // reuses its exchange and done words under its own sweep ids
@@ -666,22 +706,24 @@ int batch_status(seisfat_batch_s* b) {
   // stream could take an XCD's whole share).  A queue's ticket counter ends
   // at its length plus the workgroups that drained it, or at 0 if none did.
   int cnt[NUM_COUNTERS] = {};
-  const bool queues = b->pairs && b->last_run_plain && b->d_ctl && b->pair_qoff.size() == 9;
+  const bool queues = b->pairs && b->last_run_plain && b->d_ctl && b->strip_qoff.size() == 9;
   if (queues) HIPCHK(hipMemcpyAsync(cnt, b->d_ctl, sizeof(cnt), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if (err[0]) return fail(SEISFAT_EHIP, "persistent sweep: a tile dependency did not arrive within the spin limit");
+  if (err[0]) return fail(SEISFAT_EHIP, "persistent sweep: a dependency did not arrive within the spin limit");
   if (err[1])
     return fail(SEISFAT_EHIP, "adjoint strip walk (fp64 trajectory or reverse sweep): a strip's upper "
                               "neighbour did not arrive within the spin limit");
   if (queues) {
     const int solves = b->type == SEISFAT_ANI ? 2 : 1;
-    for (int s = 0; s < solves; ++s)
+    for (int s = 0; s < solves; ++s) {
+      const std::vector<int>& q = s == 0 ? b->strip_qoff : b->pair_qoff;
       for (int p = 0; p < 2; ++p)
         for (int x = 0; x < 8; ++x)
-          if (cnt[PAIR_COUNTERS + 16 * s + 8 * p + x] < b->pair_qoff[x + 1] - b->pair_qoff[x])
+          if (cnt[PAIR_COUNTERS + 16 * s + 8 * p + x] < q[x + 1] - q[x])
             return fail(SEISFAT_EHIP, "fused sweep pairs: XCD " + std::to_string(x) +
                                           " received no workgroup, its tiles were not solved (another kernel "
                                           "running at the same time?); use schedule option pairs = 0");
+    }
   }
   return SEISFAT_OK;
 }
@@ -1319,8 +1361,8 @@ int seisfat_batch_status(seisfat_batch_t b) {
 int seisfat_batch_tile_counts(seisfat_batch_t b, long long* total, long long* skipped) {
   if (!b || !total || !skipped) return fail(SEISFAT_EINVAL, "null batch or output");
   if (!b->d_ctl) return fail(SEISFAT_EINVAL, "tile counts exist for the persistent tiled schedule only");
-  const long long solves = b->type == SEISFAT_ANI ? 2 : 1;
-  *total = solves * (b->pairs ? 2LL * (long long)b->pair_tiles.size() : 4LL * b->ntiles);
+  const long long tiles = b->pairs ? 2LL * (long long)b->pair_tiles.size() : 4LL * b->ntiles;
+  *total = (b->pairs ? 2 * b->strip_blocks : tiles) + (b->type == SEISFAT_ANI ? tiles : 0);
   int n = 0;
   HIPCHK(hipEventSynchronize(b->ev_done));
   HIPCHK(hipMemcpyAsync(&n, b->d_ctl + CTL_SKIP, sizeof(int), hipMemcpyDeviceToHost, b->h->stream));

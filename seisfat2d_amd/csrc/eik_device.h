@@ -271,11 +271,12 @@ __device__ __forceinline__ CellQ cell_q(float s, const EikConsts& k) {
 // min(told, eik_local): the minimum of told, both 1-D candidates, the 2-D
 // candidate and TINF (no operand is a NaN, so two three-way minima give the
 // same value as the nested pairwise ones).
+// m1, m2: min(dz s_ref, dz s_zo) and min(dx s_ref, dx s_xo).
 template <bool EQH, bool FD>
-__device__ __forceinline__ float eik_local_sel(float tv, float te, float tev, const CellQ& r, float dzs_zo,
-                                               float dxs_xo, const EikConsts& k, float told) {
-  const float t1d1 = tv + vmin(r.dzs, dzs_zo);
-  const float t1d2 = te + vmin(r.dxs, dxs_xo);
+__device__ __forceinline__ float eik_local_sel(float tv, float te, float tev, const CellQ& r, float m1,
+                                               float m2, const EikConsts& k, float told) {
+  const float t1d1 = tv + m1;
+  const float t1d2 = te + m2;
   const float t1D = vmin3(t1d1, t1d2, TINF);
   const float de = te - tev;
   const float dv = tv - tev;

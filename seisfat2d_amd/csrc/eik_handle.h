@@ -117,10 +117,18 @@ struct seisfat_batch_s {
   std::vector<ShotDev> iso_b, qp_b;  // iso / qp with the pairs' second-sweep exchange buffers
   ShotDev* d_iso_b = nullptr;
   ShotDev* d_qp_b = nullptr;
+  // tiles of the qP solve (anisotropic batches)
   int4* d_ptiles = nullptr;
   int* d_qoff = nullptr;
   std::vector<int4> pair_tiles;  // host copies of the queues' contents
   std::vector<int> pair_qoff;
+  // strips of the isotropic solve
+  int4* d_strips = nullptr;
+  int* d_soff = nullptr;
+  std::vector<int4> strips;
+  std::vector<int> strip_qoff;
+  int strips_most = 0;        // of an XCD
+  long long strip_blocks = 0;  // blocks of all strips
   // the last run was a plain pass (run / recorded run), whose fused-pair
   // queues batch_status checks were drained
   bool last_run_plain = false;

@@ -56,12 +56,20 @@ struct PersistRun {
 // Both sweeps of each pair (0,1) and (2,3) in one launch each, shots
 // partitioned over the 8 XCDs: ptiles holds each XCD's tiles of both sweeps
 // (w bit 2 = second sweep, bits 0-1 = priority) at [qoff[x], qoff[x+1]);
-// shots_b differs from shots_a only in its exchange buffers.  skew: the
-// skewed slowness copies, or null for slowness staged from the shots' own
-// grids (the qP solve); solve (0 or 1) selects sweep ids and queue counters.
+// shots_b differs from shots_a only in its exchange buffers.  Slowness comes
+// from the shots' own grids (the qP solve); solve (0 or 1) selects sweep ids and
+// queue counters.
 int launch_sweeps_pairs(const ShotDev* shots_a, const ShotDev* shots_b, const int4* ptiles, const int* qoff,
-                        int nstrips, int nzz, const EikConsts& k, bool eqh, const SkewView* skew,
-                        const PersistRun& pr, int solve, hipStream_t st);
+                        int nstrips, int nzz, const EikConsts& k, bool eqh, const PersistRun& pr, int solve,
+                        hipStream_t st);
+// The same pairs by strips, slowness from the skewed copies: strips holds each XCD's
+// strips (x = shot, y = strip, z = second sweep) at [qoff[x], qoff[x+1]), at
+// most `most` an XCD.
+constexpr int STRIP_BLOCK = 8;    // steps of a strip's block (the unit of its skips)
+constexpr int STRIPS_PER_CU = 3;  // workgroups a CU holds
+int launch_sweeps_strips(const ShotDev* shots_a, const ShotDev* shots_b, const int4* strips, const int* qoff,
+                         int most, int nstrips, int nzz, const EikConsts& k, bool eqh, const SkewView* skew,
+                         const PersistRun& pr, int solve, hipStream_t st);
 // out[i] = XCC id of workgroup i (i < n)
 void launch_xcc_ids(int* out, int n, hipStream_t st);
 // changed / skip (converged mode, skewed slowness only): every tile that

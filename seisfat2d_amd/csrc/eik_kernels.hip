@@ -6,6 +6,8 @@
 //                     reference schedule (src/modeling/modeling.cu:123-159)
 //   k_sweep_tiles     the same sweep as 64x64 skewed tiles staged in LDS,
 //                     one launch per tile diagonal over every shot of a batch
+//   k_strip_pair      two sweeps of a solve in one launch, a workgroup a strip
+//   k_sweep_pair      the same by tiles (the qP solve)
 //   k_picks           compute_seismogram's Catmull-Rom picks
 //                     (src/modeling/modeling.cu:161-194, src/admin/admin.cpp:121-134)
 //   k_quasi_slowness  get_quasi_slowness   (src/modeling/eikonal_ani.cu:47-111)
@@ -233,7 +235,8 @@ __device__ __forceinline__ void tile_step(float* __restrict__ sT, int tab, int t
   // XDPP: lane k's x-other cell is lane k+1's z-other cell of this step; sxo
   // is then only lane 63's (times dx when EQH, where zo.dzs = dz*s = dx*s)
   const float dxs_xo = !XDPP ? k.dx * sxo : (EQH ? dpp_shl1(sxo, zo.dzs) : k.dx * dpp_shl1(sxo, szo));
-  const float m = eik_local_sel<EQH, FD>(tv, te, tev, sref, zo.dzs, dxs_xo, k, told);  // min(told, candidates)
+  const float m = eik_local_sel<EQH, FD>(tv, te, tev, sref, vmin(sref.dzs, zo.dzs), vmin(sref.dxs, dxs_xo), k,
+                                         told);  // min(told, candidates)
   const float res = act ? m : told;
   if constexpr (CONV) chg = chg | (row_ok & (res < told));  // converged mode: did this lane lower a traveltime
   ring_at(sT, tab) = res;
@@ -777,15 +780,15 @@ __global__ __launch_bounds__(64) void k_sweep_persist(const ShotDev* __restrict_
 // it waits for, so a second-sweep tile starts as soon as the first-sweep
 // tiles under it are written back, not when the whole first sweep is done.
 // Per-XCD queues drain for the same reason a single queue does.
-template <int SB, bool EQH, bool FD, bool FIRST_A, bool SKEW>
+template <int SB, bool EQH, bool FD, bool FIRST_A>
 __global__ __launch_bounds__(64) void k_sweep_pair(const ShotDev* __restrict__ shots_a,
                                                    const ShotDev* __restrict__ shots_b,
                                                    const int4* __restrict__ tiles, const int* __restrict__ qoff,
-                                                   int nzz, EikConsts k, SkewView sv_a, SkewView sv_b,
-                                                   PersistCtl ctl_a, PersistCtl ctl_b) {
+                                                   int nzz, EikConsts k, PersistCtl ctl_a, PersistCtl ctl_b) {
   __shared__ float sT[64 * RING_LD];
-  __shared__ float sS[SKEW ? 1 : SS_STEPS * 64];
+  __shared__ float sS[SS_STEPS * 64];
   __shared__ __attribute__((aligned(8))) float sHX[HX_WORDS];
+  const SkewView none{nullptr, 0};
   const int xcd = __builtin_amdgcn_s_getreg((15 << 11) | 20) & 7;  // hwreg(HW_REG_XCC_ID, 0, 16)
   const unsigned tag_a = (*ctl_a.epoch << 11) | (ctl_a.sweep_id << 8);
   const unsigned tag_b = (*ctl_b.epoch << 11) | (ctl_b.sweep_id << 8);
@@ -809,14 +812,364 @@ __global__ __launch_bounds__(64) void k_sweep_pair(const ShotDev* __restrict__ s
     }
     int raw = 0, next = 0;
     if (tl.w & 4)
-      tile_process<-1, SB, EQH, FD, SKEW, false, true, 2, false>(
-          tl, shots_b, nzz, k, sv_b, cb, tag_b, sT, sS, sHX, [&] { raw = claim_issue(); },
+      tile_process<-1, SB, EQH, FD, false, false, true, 2, false>(
+          tl, shots_b, nzz, k, none, cb, tag_b, sT, sS, sHX, [&] { raw = claim_issue(); },
           [&] { next = __builtin_amdgcn_readfirstlane(raw); });
     else
-      tile_process<1, SB, EQH, FD, SKEW, FIRST_A, true, 1, false>(
-          tl, shots_a, nzz, k, sv_a, ctl_a, tag_a, sT, sS, sHX, [&] { raw = claim_issue(); },
+      tile_process<1, SB, EQH, FD, false, FIRST_A, true, 1, false>(
+          tl, shots_a, nzz, k, none, ctl_a, tag_a, sT, sS, sHX, [&] { raw = claim_issue(); },
           [&] { next = __builtin_amdgcn_readfirstlane(raw); });
     tk = next;
+  }
+}
+
+// Fused sweep pair by strips: a workgroup walks one strip of 64 rows of one
+// sweep from its first column to its last (step t: lane k on column t - k, as a
+// tile's steps, without the tiles' restarts), with the work around the steps in
+// waves of their own:
+//   wave 0  the steps.  Traveltimes and the slowness quantities come from LDS.
+//   wave 1  old traveltimes: whole columns into the ring, WP_D blocks ahead (a
+//           second sweep's once the first one's strips have stored them)
+//   wave 2  publishes the strip's last row, then stores finished columns
+//   wave 3  the quantities that depend on slowness alone
+//   wave 4  the upper strip's last row (tagged words, polled a block ahead)
+// The ring holds column c, row k at [(c + k) mod WP_R][k], so a step's nodes are
+// 64 consecutive words and a result replaces its old value.  The waves meet at a
+// barrier every WP_B steps.  Shots belong to XCDs as in k_sweep_pair; tickets
+// are strips, all shots' first ones first, so a workgroup only waits for
+// smaller tickets.  A block whose inputs are all TINF is not run (k.tinf_fixed).
+//
+// What bounds it: a wave issues one instruction in four cycles, and the steps are
+// a chain, so a strip takes (columns + 63) x 60 instructions; beside them a step
+// costs 35 cycles of its block's barrier and first LDS reads (125 ns a step).  The
+// next strip starts 88 steps later (64 columns, a block, the words' way).  A 64 x
+// 64 tile, staged, run and written back by one wave, took twice that for its
+// hand-over.  With 256 shots three workgroups fit a CU (LDS; five waves) and a
+// strip's step takes 180 ns; two thirds of the vector instructions are wave 0's.
+// One shot of 201 x 1001: 313 + 376 us the two pairs by tiles, 205 + 224 by
+// strips; 1001 x 4001: 1305 + 1535 against 785 + 865; 24 windows of 403 x 1777:
+// 790 + 805 against 346 + 390; a solve of 256 windows of 1001 x 4001: 9.7 ms
+// against 9.0.  Blocks of 12 steps (two workgroups a CU): the same for one shot,
+// 20 % more for 256; of 16 (one): 4 % less for one shot, twice the time for 256.
+// Four waves, wave 3 polling as well (four workgroups a CU): 5 to 15 % more.
+constexpr int WP_B = STRIP_BLOCK;
+constexpr int WP_R = (64 + 4 * WP_B - 1) / WP_B * WP_B;  // ring steps: a step's 64, a block arriving, one leaving
+constexpr int WP_D = 3;                 // blocks of loads in flight
+constexpr int WP_P = 4;                 // blocks between a first sweep's progress words
+constexpr int WP_THREADS = 320;
+
+// Workgroup barrier after this wave's LDS operations (its global ones may stay
+// in flight).
+__device__ __forceinline__ void wp_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// x mod WP_R for 0 <= x < 2 WP_R
+__device__ __forceinline__ unsigned wp_wrap(unsigned x) { return min(x, x - WP_R); }
+
+struct StripLds {
+  float ring[WP_R * 64];
+  float4 cell[2][WP_B][64];  // m1, m2 (see eik_local_sel), s and thrB of the reference cell
+  __attribute__((aligned(16))) float up[2][WP_B];  // upper strip's last row at the columns of a block's steps
+  int tinf[2][2];            // the block's old traveltimes, and its upper row, are all TINF
+  int ticket;
+};
+
+// One strip.  XMODE 1: the pair's first sweep (FIRST: of the solve), 2: its second.
+template <int SA, int SB, bool EQH, bool FD, bool FIRST, int XMODE>
+__device__ __forceinline__ void strip_walk(StripLds& L, const ShotDev sd, int r, int nzz, const EikConsts& k,
+                                           const SkewView& sv, const PersistCtl& ctl, unsigned tagb) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int nxx = sd.nxx, NR = nzz - 2, NC = nxx - 2;
+  const int kg = 64 * r + lane;
+  const bool row_ok = kg < NR;
+  const int nblk = (NC + 63 + WP_B - 1) / WP_B;
+  // block n: wave 0 takes steps n WP_B .. n WP_B + WP_B - 1 (0 <= n < nblk), the others bring
+  // what block n + 1 reads and take away what block n - 1 left
+  if (wave == 0) {
+    float te = TINF, tev = TINF;
+    const auto block = [&](int t0, int buf, auto edge) {
+      float* __restrict__ rg = L.ring + (t0 % WP_R) * 64 + lane;
+      unsigned zero = 0;
+      asm volatile("" : "+v"(zero));  // (one address register for the block's broadcasts)
+      // a step's operands are read one step ahead, old values two steps', the
+      // upper row's four steps' at a time
+      float told[2], done = 0.0f;
+      float4 up, c = L.cell[buf][0][lane];
+#pragma unroll
+      for (int u = 0; u < WP_B; ++u) {
+        if (u == 0) {
+          told[0] = rg[0];
+          told[1] = rg[64];
+          up = *reinterpret_cast<const float4*>(&L.up[buf][zero]);
+        }
+        const float told_u = told[u & 1], up_u = u & 2 ? (u & 1 ? up.w : up.z) : (u & 1 ? up.y : up.x);
+        const float4 cu = c;
+        const float tv = dpp_shr1(up_u, te);
+        if (u + 1 < WP_B) c = L.cell[buf][u + 1][lane];
+        if ((u & 1) && u + 1 < WP_B) {
+          told[0] = rg[64 * (u + 1)];
+          told[1] = rg[64 * (u + 2)];
+        }
+        if ((u & 3) == 3 && u + 1 < WP_B) up = *reinterpret_cast<const float4*>(&L.up[buf][zero + u + 1]);
+        __builtin_amdgcn_sched_barrier(0);  // (left alone the compiler reads them just before their use)
+        CellQ q;
+        q.dzs = cu.z * k.dz;
+        q.dxs = EQH ? q.dzs : cu.z * k.dx;
+        q.s2 = cu.z * cu.z;
+        q.s4 = q.s2 * k.sum4;
+        q.thrB = cu.w;
+        q.thrC = EQH ? q.thrB : (FD ? fdiv(q.dxs * k.dx, k.zh_hyp, k.zl_hyp) : rdiv(q.dxs * k.dx, k.hyp, k.r_hyp));
+        float res = eik_local_sel<EQH, FD>(tv, te, tev, q, cu.x, cu.y, k, told_u);
+        // outside the grid: the ring's value (past the last row nothing reads it)
+        if (edge.value && !(row_ok && (unsigned)(t0 + u - lane) < (unsigned)NC)) res = TINF;
+        if (u & 1) {
+          rg[64 * (u - 1)] = done;
+          rg[64 * u] = res;
+        }
+        done = res;
+        tev = tv;
+        te = res;
+      }
+    };
+    wp_barrier();  // block -1
+    int nskip = 0;
+    for (int n = 0; n < nblk; ++n) {
+      const int t0 = n * WP_B, buf = n & 1;
+      const bool still = k.tinf_fixed && __builtin_amdgcn_readfirstlane(L.tinf[buf][0] & L.tinf[buf][1]) &&
+                         __all((te == TINF) & (tev == TINF));
+      if (still)
+        ++nskip;
+      else if (t0 >= 64 && t0 + WP_B <= NC)
+        block(t0, buf, std::false_type());
+      else
+        block(t0, buf, std::true_type());
+      wp_barrier();
+    }
+    if (nskip && lane == 0) atomicAdd(ctl.nskip, nskip);
+    wp_barrier();
+    wp_barrier();
+  } else if (wave == 1) {
+    gfloat* __restrict__ T = gptr(sd.T);
+    const unsigned row = (unsigned)prow<SA>(min(kg, NR), nzz);
+    const auto col = [&](int c) {  // (uniform address, the lane's offset in one register)
+      gfloat* p = T + (size_t)pcol<SB>(min(max(c, -1), NC), nxx) * nzz;
+      asm volatile("" : "+s"(p));
+      return p + row;
+    };
+    // second sweep: columns the first one has stored in this strip's rows (its
+    // strips r0, r0 + 1)
+    int seen = XMODE == 2 ? 0 : 1 << 30;
+    const int r0 = (NR - 1 - min(64 * r + 63, NR - 1)) >> 6, r1 = (NR - 1 - 64 * r) >> 6;
+    const auto wait_for = [&](int c) {  // column c and those before it
+      const int want = min(c + 1, NC);
+      for (int it = 0; seen < want; ++it) {
+        const unsigned long long w = __hip_atomic_load((const gword*)(sd.xd + (size_t)(lane & 1 ? r1 : r0) * sd.nb),
+                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int cols = (unsigned)(w >> 32) == ctl.xtag ? (int)(unsigned)w : 0;
+        seen = min(__builtin_amdgcn_readlane(cols, 0), __builtin_amdgcn_readlane(cols, 1));
+        if (it > SPIN_LIMIT) {
+          if (lane == 0) atomicOr(ctl.err, 1);
+          seen = 1 << 30;
+        }
+        if (seen < want) __builtin_amdgcn_s_sleep(2);
+      }
+      asm volatile("" ::: "memory");
+    };
+    const int sIdx = (int)((sd.sx + 0.5f * k.dx) / k.dx) + NB;
+    const int sIdz = (int)((sd.sz + 0.5f * k.dz) / k.dz) + NB;
+    const auto load = [&](int c0, float (&q)[WP_B]) {
+      if (XMODE == 2) wait_for(c0 + WP_B - 1);
+#pragma unroll
+      for (int u = 0; u < WP_B; ++u) {
+        if (FIRST) {
+          // time_set + time_init
+          q[u] = TINF;
+          const int j = pcol<SB>(c0 + u, nxx), i = prow<SA>(kg, nzz);
+          if (abs(j - sIdx) <= 1 && c0 + u >= 0 && c0 + u < NC) {
+            if (row_ok && abs(i - sIdz) <= 1) {
+              const float ddx = (float)(j - NB) * k.dx - sd.sx;
+              const float ddz = (float)(i - NB) * k.dz - sd.sz;
+              q[u] = s_at(sd, nzz, i, j) * sqrtf(ddx * ddx + ddz * ddz);
+            }
+          }
+        } else if (XMODE == 2) {
+          q[u] = __hip_atomic_load(col(c0 + u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+          q[u] = *col(c0 + u);
+        }
+      }
+    };
+    float q[WP_D][WP_B];
+#pragma unroll
+    for (int d = 0; d < WP_D; ++d) load(d * WP_B, q[d]);
+    int run = 1 << 20;  // the last `run` columns are all TINF (those before the grid count)
+    for (int n = -1; n < nblk + 2; n += WP_D)
+#pragma unroll
+      for (int d = 0; d < WP_D; ++d)
+        if (n + d < nblk + 2) {
+          const int c_in = (n + d + 1) * WP_B;
+          const unsigned s0 = (unsigned)(c_in % WP_R) + lane;
+#pragma unroll
+          for (int u = 0; u < WP_B; ++u) {
+            L.ring[wp_wrap(s0 + u) * 64 + lane] = q[d][u];
+            run = __all(q[d][u] == TINF) ? run + 1 : 0;
+          }
+          if (lane == 0) L.tinf[(n + d + 1) & 1][0] = run >= 64 + WP_B;
+          load(c_in + WP_D * WP_B, q[d]);
+          wp_barrier();
+        }
+  } else if (wave == 2) {
+    gfloat* __restrict__ T = gptr(sd.T);
+    const unsigned row = (unsigned)prow<SA>(min(kg, NR), nzz);
+    const bool pub = r + 1 < ctl.nstrips;
+    const auto progress = [&](int cols) {  // the columns before `cols` are in T
+      __builtin_amdgcn_s_waitcnt(0);       // (their stores have reached L2)
+      asm volatile("" ::: "memory");
+      if (lane == 0)
+        __hip_atomic_store((gword*)(sd.xd + (size_t)r * sd.nb),
+                           ((unsigned long long)tagb << 32) | (unsigned)min(cols, NC), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    };
+    for (int n = -1; n < nblk + 2; ++n) {
+      const int c_out = (n - 1) * WP_B - 64;
+      if (XMODE == 1 && c_out > 0 && (n - 1) % WP_P == 0) progress(c_out);  // (those of earlier blocks)
+      // the last row's results of block n - 1
+      if (pub && lane < WP_B) {
+        const int t = (n - 1) * WP_B + lane, c = t - 63;
+        if (c >= 0 && c < NC) xstore(sd.xh + (size_t)r * sd.ldh + c, L.ring[(t % WP_R) * 64 + 63], tagb);
+      }
+      // columns that lane 63 finished by the end of block n - 1
+      if (c_out + WP_B > 0) {
+        const unsigned s0 = (unsigned)((c_out + WP_R) % WP_R) + lane;
+        float v[WP_B];
+#pragma unroll
+        for (int u = 0; u < WP_B; ++u) v[u] = L.ring[wp_wrap(s0 + u) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < WP_B; ++u)
+          if (row_ok && c_out + u >= 0 && c_out + u < NC) {
+            gfloat* p = T + (size_t)pcol<SB>(c_out + u, nxx) * nzz;
+            asm volatile("" : "+s"(p));
+            p[row] = v[u];
+          }
+      }
+      wp_barrier();
+    }
+    if (XMODE == 1) progress(NC);
+  } else if (wave == 3) {
+    // Cell (kap, lam) of step t: the z-other cell of lane k at lam = t - k + 1
+    // (reference cell of step t + 1); lane 63's x-other cell is (64r + 64, t - 63).
+    const int kap = 64 * r + lane;
+    const int lam_lo = SB > 0 ? 3 : 2, lam_hi = SB > 0 ? sd.w + 2 : sd.w + 1;  // unreplicated cell columns
+    typedef __attribute__((address_space(1))) const float cfloat;
+    cfloat* base = (cfloat*)sv.base + (long long)((SB > 0 ? sd.x0 + 1 : sd.x0 + sd.w + 66) + SK_OFF) * sv.KP;
+    const long long pitch = (long long)SB * sv.KP;
+    const auto load = [&](int t0, float (&q)[WP_B], float& x63) {
+      const int tx = t0 + min(lane, WP_B - 1);
+      if (t0 - 63 >= lam_lo && t0 + WP_B <= lam_hi) {
+        cfloat* b = base + t0 * pitch;
+#pragma unroll
+        for (int u = 0; u < WP_B; ++u) {
+          asm volatile("" : "+s"(b));  // (uniform address, the lane's offset in one register)
+          q[u] = b[(unsigned)kap];
+          b += pitch;
+        }
+        x63 = base[(long long)(64 * r + 64) + (tx - 64) * pitch];
+      } else {
+        int lam = t0 - lane;
+#pragma unroll
+        for (int u = 0; u < WP_B; ++u) {
+          ++lam;
+          asm volatile("" : "+v"(lam));  // (one address at a time in registers)
+          q[u] = gptr(sv.base)[skew_addr<SB>(sd, nxx, NC, sv.KP, kap, lam)];
+        }
+        x63 = gptr(sv.base)[skew_addr<SB>(sd, nxx, NC, sv.KP, 64 * r + 64, tx - 63)];
+      }
+    };
+    const auto thr = [&](float dzs) {
+      return FD ? fdiv(dzs * k.dz, k.zh_hyp, k.zl_hyp) : rdiv(dzs * k.dz, k.hyp, k.r_hyp);
+    };
+    float q[WP_D][WP_B], x63[WP_D];
+    float s = gptr(sv.base)[skew_addr<SB>(sd, nxx, NC, sv.KP, kap, -lane)];
+#pragma unroll
+    for (int d = 0; d < WP_D; ++d) load(d * WP_B, q[d], x63[d]);
+    float dzs = s * k.dz, dxs = EQH ? dzs : s * k.dx, th = thr(dzs);
+    for (int n = -1; n < nblk + 2; n += WP_D)
+#pragma unroll
+      for (int d = 0; d < WP_D; ++d)
+        if (n + d < nblk + 2) {
+          const int buf = (n + d + 1) & 1;
+          const int xb = __float_as_int(x63[d] * k.dx);
+#pragma unroll
+          for (int u = 0; u < WP_B; ++u) {
+            const float s_zo = q[d][u], dzs_zo = s_zo * k.dz, dxs_zo = EQH ? dzs_zo : s_zo * k.dx;
+            // lane k's x-other cell is lane k + 1's z-other cell of the same step
+            const float dxs_xo = dpp_shl1(__int_as_float(__builtin_amdgcn_readlane(xb, u)), dxs_zo);
+            asm volatile("" : "+v"(s));  // (a copy: the loads keep single registers, not the vector's)
+            L.cell[buf][u][lane] = make_float4(vmin(dzs, dzs_zo), vmin(dxs, dxs_xo), s, th);
+            s = s_zo;
+            dzs = dzs_zo;
+            dxs = dxs_zo;
+            th = thr(dzs);
+          }
+          if (n + d + 1 + WP_D < nblk) load((n + d + 1 + WP_D) * WP_B, q[d], x63[d]);
+          wp_barrier();
+        }
+  } else {
+    const unsigned long long* xup = sd.xh + (size_t)max(r - 1, 0) * sd.ldh;
+    bool gave_up = false;
+    const int u = min(lane, WP_B - 1);
+    const auto word = [&](int n) {  // of block n's steps
+      return __hip_atomic_load((const gword*)(xup + min(n * WP_B + u, NC - 1)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    };
+    unsigned long long w = r > 0 ? word(0) : 0ull;
+    for (int n = -1; n < nblk + 2; ++n) {
+      float v = TINF;
+      if (r > 0 && n + 1 < nblk) {
+        for (int it = 0; !gave_up && !__all((unsigned)(w >> 32) == tagb); ++it) {
+          if (it > SPIN_LIMIT) {
+            if (lane == 0) atomicOr(ctl.err, 1);
+            gave_up = true;
+          }
+          __builtin_amdgcn_s_sleep(1);
+          w = word(n + 1);
+        }
+        if ((n + 1) * WP_B + u < NC) v = __uint_as_float((unsigned)w);
+        w = word(n + 2);
+      }
+      const int buf = (n + 1) & 1;
+      if (lane < WP_B) L.up[buf][lane] = v;
+      const bool none = __all(v == TINF);
+      if (lane == 0) L.tinf[buf][1] = none;
+      wp_barrier();
+    }
+  }
+}
+
+template <int SB, bool EQH, bool FD, bool FIRST_A>
+__global__ __launch_bounds__(WP_THREADS) void k_strip_pair(const ShotDev* __restrict__ shots_a,
+                                                           const ShotDev* __restrict__ shots_b,
+                                                           const int4* __restrict__ strips,
+                                                           const int* __restrict__ qoff, int nzz, EikConsts k,
+                                                           SkewView sv_a, SkewView sv_b, PersistCtl ctl_a,
+                                                           PersistCtl ctl_b) {
+  __shared__ StripLds L;
+  const int xcd = __builtin_amdgcn_s_getreg((15 << 11) | 20) & 7;  // hwreg(HW_REG_XCC_ID, 0, 16)
+  const unsigned tag_a = (*ctl_a.epoch << 11) | (ctl_a.sweep_id << 8);
+  const unsigned tag_b = (*ctl_b.epoch << 11) | (ctl_b.sweep_id << 8);
+  PersistCtl cb = ctl_b;
+  cb.xtag = tag_a;
+  const int base = qoff[xcd], n = qoff[xcd + 1] - base;
+  for (;;) {
+    if (threadIdx.x == 0) L.ticket = atomicAdd(ctl_a.counter + xcd, 1);
+    __syncthreads();
+    const int tk = __builtin_amdgcn_readfirstlane(L.ticket);
+    if (tk >= n) break;
+    const int4 e = strips[base + tk];  // shot, strip, second sweep
+    if (e.z)
+      strip_walk<-1, SB, EQH, FD, false, 2>(L, shots_b[e.x], e.y, nzz, k, sv_b, cb, tag_b);
+    else
+      strip_walk<1, SB, EQH, FD, FIRST_A, 1>(L, shots_a[e.x], e.y, nzz, k, sv_a, ctl_a, tag_a);
   }
 }
 
@@ -1233,14 +1586,13 @@ int launch_sweeps_persist(const ShotDev* shots, const int4* tiles, int ntiles, i
   return 4;
 }
 
-template <int SB, bool EQH, bool FD, bool FIRST_A, bool SKEW>
+template <int SB, bool EQH, bool FD, bool FIRST_A>
 static void pair_launch(const ShotDev* shots_a, const ShotDev* shots_b, const int4* tiles, const int* qoff,
-                        int nzz, const EikConsts& k, const SkewView& sv_a, const SkewView& sv_b,
-                        const PersistCtl& ca, const PersistCtl& cb, hipStream_t st) {
+                        int nzz, const EikConsts& k, const PersistCtl& ca, const PersistCtl& cb, hipStream_t st) {
   static int per_cu = 0, cus = 0;
   if (per_cu == 0) {
     int dev = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_sweep_pair<SB, EQH, FD, FIRST_A, SKEW>, 64, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_sweep_pair<SB, EQH, FD, FIRST_A>, 64, 0) !=
             hipSuccess ||
         per_cu <= 0)
       per_cu = 4;
@@ -1249,40 +1601,25 @@ static void pair_launch(const ShotDev* shots_a, const ShotDev* shots_b, const in
       cus = 256;
   }
   const int grid = (ca.wpcu > 0 ? std::min(ca.wpcu, per_cu) : per_cu) * cus;
-  hipLaunchKernelGGL((k_sweep_pair<SB, EQH, FD, FIRST_A, SKEW>), dim3(grid), dim3(64), 0, st, shots_a, shots_b, tiles,
-                     qoff, nzz, k, sv_a, sv_b, ca, cb);
+  hipLaunchKernelGGL((k_sweep_pair<SB, EQH, FD, FIRST_A>), dim3(grid), dim3(64), 0, st, shots_a, shots_b, tiles,
+                     qoff, nzz, k, ca, cb);
 }
 
-template <int SB, bool FIRST_A>
-static void pair_dispatch(bool eqh, bool fd, bool skew, const ShotDev* shots_a, const ShotDev* shots_b,
-                          const int4* tiles, const int* qoff, int nzz, const EikConsts& k, const SkewView& sv_a,
-                          const SkewView& sv_b, const PersistCtl& ca, const PersistCtl& cb, hipStream_t st) {
-#define SEIS_PAIR(E, F, S) pair_launch<SB, E, F, FIRST_A, S>(shots_a, shots_b, tiles, qoff, nzz, k, sv_a, sv_b, ca, cb, st)
-  // the known-divisor division where it is exact
-  if (skew) {
-    if (eqh) {
-      if (fd) SEIS_PAIR(true, true, true);
-      else SEIS_PAIR(true, false, true);
-    } else {
-      if (fd) SEIS_PAIR(false, true, true);
-      else SEIS_PAIR(false, false, true);
-    }
-  } else {
-    if (eqh) {
-      if (fd) SEIS_PAIR(true, true, false);
-      else SEIS_PAIR(true, false, false);
-    } else {
-      if (fd) SEIS_PAIR(false, true, false);
-      else SEIS_PAIR(false, false, false);
-    }
-  }
-#undef SEIS_PAIR
+template <int SB, bool EQH, bool FD, bool FIRST_A>
+static void strip_launch(const ShotDev* shots_a, const ShotDev* shots_b, const int4* strips, const int* qoff,
+                         int most, int nzz, const EikConsts& k, const SkewView& sv_a, const SkewView& sv_b,
+                         const PersistCtl& ca, const PersistCtl& cb, hipStream_t st) {
+  // workgroups go round robin over the 8 XCDs (check_xcc)
+  const int per_cu = std::min(ca.wpcu > 0 ? ca.wpcu : STRIPS_PER_CU, STRIPS_PER_CU);
+  const int grid = 8 * std::min(most, 32 * per_cu);
+  hipLaunchKernelGGL((k_strip_pair<SB, EQH, FD, FIRST_A>), dim3(grid), dim3(WP_THREADS), 0, st, shots_a, shots_b,
+                     strips, qoff, nzz, k, sv_a, sv_b, ca, cb);
 }
 
-int launch_sweeps_pairs(const ShotDev* shots_a, const ShotDev* shots_b, const int4* ptiles, const int* qoff,
-                        int nstrips, int nzz, const EikConsts& k, bool eqh, const SkewView* skew,
-                        const PersistRun& pr, int solve, hipStream_t st) {
-  const SkewView none{nullptr, 0};
+// The two pairs of a solve: first and second sweeps' control blocks, counters
+// and ids.
+template <class Launch>
+static void for_pairs(int nstrips, const PersistRun& pr, int solve, const Launch& launch) {
   for (int p = 0; p < 2; ++p) {
     PersistCtl ca{}, cb{};
     ca.wpcu = cb.wpcu = pr.wpcu;
@@ -1296,15 +1633,45 @@ int launch_sweeps_pairs(const ShotDev* shots_a, const ShotDev* shots_b, const in
     cb.sweep_id = (unsigned)(4 * solve + 2 * p + 1);
     ca.xtag = cb.xtag = 0u;
     cb.counter = ca.counter;
-    const SkewView& sa = skew ? skew[2 * p] : none;
-    const SkewView& sb = skew ? skew[2 * p + 1] : none;
-    if (p == 0)
-      pair_dispatch<1, true>(eqh, k.fastdiv != 0, skew != nullptr, shots_a, shots_b, ptiles, qoff, nzz, k, sa, sb,
-                             ca, cb, st);
-    else
-      pair_dispatch<-1, false>(eqh, k.fastdiv != 0, skew != nullptr, shots_a, shots_b, ptiles, qoff, nzz, k, sa, sb,
-                               ca, cb, st);
+    launch(p, ca, cb);
   }
+}
+
+int launch_sweeps_strips(const ShotDev* shots_a, const ShotDev* shots_b, const int4* strips, const int* qoff,
+                         int most, int nstrips, int nzz, const EikConsts& k, bool eqh, const SkewView* skew,
+                         const PersistRun& pr, int solve, hipStream_t st) {
+  for_pairs(nstrips, pr, solve, [&](int p, const PersistCtl& ca, const PersistCtl& cb) {
+#define SEIS_STRIPS(E, F)                                                                                       \
+  (p == 0 ? strip_launch<1, E, F, true> : strip_launch<-1, E, F, false>)(shots_a, shots_b, strips, qoff, most, nzz, \
+                                                                         k, skew[2 * p], skew[2 * p + 1], ca, cb, st)
+    if (eqh) {
+      if (k.fastdiv) SEIS_STRIPS(true, true);
+      else SEIS_STRIPS(true, false);
+    } else {
+      if (k.fastdiv) SEIS_STRIPS(false, true);
+      else SEIS_STRIPS(false, false);
+    }
+#undef SEIS_STRIPS
+  });
+  return 2;
+}
+
+int launch_sweeps_pairs(const ShotDev* shots_a, const ShotDev* shots_b, const int4* ptiles, const int* qoff,
+                        int nstrips, int nzz, const EikConsts& k, bool eqh, const PersistRun& pr, int solve,
+                        hipStream_t st) {
+  for_pairs(nstrips, pr, solve, [&](int p, const PersistCtl& ca, const PersistCtl& cb) {
+#define SEIS_PAIR(E, F) \
+  (p == 0 ? pair_launch<1, E, F, true> : pair_launch<-1, E, F, false>)(shots_a, shots_b, ptiles, qoff, nzz, k, ca, cb, st)
+    // the known-divisor division where it is exact
+    if (eqh) {
+      if (k.fastdiv) SEIS_PAIR(true, true);
+      else SEIS_PAIR(true, false);
+    } else {
+      if (k.fastdiv) SEIS_PAIR(false, true);
+      else SEIS_PAIR(false, false);
+    }
+#undef SEIS_PAIR
+  });
   return 2;
 }
 

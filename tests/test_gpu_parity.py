@@ -535,6 +535,32 @@ def test_unreached_tiles_skipped_only_where_the_geometry_keeps_1e6(oracle, monke
     e.close()
 
 
+@pytest.mark.parametrize("dz,dx", [(5.0, 5.0), (6.3, 9.7)])
+@pytest.mark.parametrize("nz,nx", [(2, 2), (3, 70), (59, 9), (60, 64), (61, 65), (124, 131), (125, 129), (190, 257)])
+def test_strip_walk_edges(oracle, nz, nx, dz, dx):
+    """Rows around multiples of the 64 of a strip, columns around its 8-step
+    blocks and its ring, narrow windows and windows at both ends of the model,
+    sources near corners: the fused pairs bit-exact, also on a second run."""
+    s = smooth_slowness(np.random.default_rng(nz + nx), nz, nx, min(dz, dx))
+    wins = [(0, nx), (0, max(nx // 2, 1)), (nx - max(nx // 3, 1), max(nx // 3, 1)), (nx // 3, max(nx // 2, 1))]
+    shots = []
+    for k, (x0, w) in enumerate(wins):
+        fx, fz = [(0.0, 0.0), (0.98, 0.98), (0.5, 0.0), (0.25, 0.7)][k]
+        shots.append((float(np.float32((x0 + fx * (w - 1)) * dx)), float(np.float32(fz * (nz - 1) * dz)), x0, w, 0, 0))
+    e = Eikonal(nz, nx, dz, dx)
+    e.set_slowness(s)
+    b = e.batch(shots, schedule=SCHED_TILED)
+    Trefs = oracle.solve_windows(s, dx, dz, [x[0] for x in shots], [x[1] for x in shots],
+                                 [x[2] for x in shots], [x[3] for x in shots], nthreads=4)
+    for _ in range(2):
+        b.run()
+        b.status()
+        for k, Tr in enumerate(Trefs):
+            assert np.array_equal(b.T(k), Tr), k
+    b.close()
+    e.close()
+
+
 def test_window_at_the_far_end_of_a_model_with_skewed_copies_over_2_gib(oracle, monkeypatch):
     """A 8000 x 70000 model, whose skewed slowness copies (one per sweep
     orientation) each exceed 2^31 bytes: a narrow window at the model's right
