@@ -66,7 +66,7 @@ int launch_sweeps_pairs(const ShotDev* shots_a, const ShotDev* shots_b, const in
 // strips (x = shot, y = strip, z = second sweep) at [qoff[x], qoff[x+1]), at
 // most `most` an XCD.
 constexpr int STRIP_BLOCK = 8;    // steps of a strip's block (the unit of its skips)
-constexpr int STRIPS_PER_CU = 3;  // workgroups a CU holds
+constexpr int STRIPS_PER_CU = 4;  // workgroups a CU holds
 int launch_sweeps_strips(const ShotDev* shots_a, const ShotDev* shots_b, const int4* strips, const int* qoff,
                          int most, int nstrips, int nzz, const EikConsts& k, bool eqh, const SkewView* skew,
                          const PersistRun& pr, int solve, hipStream_t st);

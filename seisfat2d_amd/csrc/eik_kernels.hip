@@ -829,10 +829,10 @@ __global__ __launch_bounds__(64) void k_sweep_pair(const ShotDev* __restrict__ s
 // waves of their own:
 //   wave 0  the steps.  Traveltimes and the slowness quantities come from LDS.
 //   wave 1  old traveltimes: whole columns into the ring, WP_D blocks ahead (a
-//           second sweep's once the first one's strips have stored them)
+//           second sweep's once the first one's strips have stored them), and the
+//           upper strip's last row (tagged words, polled a block ahead)
 //   wave 2  publishes the strip's last row, then stores finished columns
 //   wave 3  the quantities that depend on slowness alone
-//   wave 4  the upper strip's last row (tagged words, polled a block ahead)
 // The ring holds column c, row k at [(c + k) mod WP_R][k], so a step's nodes are
 // 64 consecutive words and a result replaces its old value.  The waves meet at a
 // barrier every WP_B steps.  Shots belong to XCDs as in k_sweep_pair; tickets
@@ -840,30 +840,40 @@ __global__ __launch_bounds__(64) void k_sweep_pair(const ShotDev* __restrict__ s
 // smaller tickets.  A block whose inputs are all TINF is not run (k.tinf_fixed).
 //
 // What bounds it: a wave issues one instruction in four cycles, and the steps are
-// a chain, so a strip takes (columns + 63) x 60 instructions; beside them a step
-// costs 35 cycles of its block's barrier and first LDS reads (125 ns a step).  The
+// a chain, so a strip takes (columns + 63) x 57 instructions; beside them a step
+// costs 20 cycles of its block's barrier and first LDS reads (115 ns a step).  The
 // next strip starts 88 steps later (64 columns, a block, the words' way).  A 64 x
 // 64 tile, staged, run and written back by one wave, took twice that for its
-// hand-over.  With 256 shots three workgroups fit a CU (LDS; five waves) and a
-// strip's step takes 180 ns; two thirds of the vector instructions are wave 0's.
-// One shot of 201 x 1001: 313 + 376 us the two pairs by tiles, 205 + 224 by
-// strips; 1001 x 4001: 1305 + 1535 against 785 + 865; 24 windows of 403 x 1777:
-// 790 + 805 against 346 + 390; a solve of 256 windows of 1001 x 4001: 9.7 ms
-// against 9.0.  Blocks of 12 steps (two workgroups a CU): the same for one shot,
+// hand-over.  With 256 shots four workgroups fit a CU (LDS), one wave 0 a SIMD; the
+// clock is lower then (1.9 GHz) and a step takes 190 ns.
+// One shot of 201 x 1001: 313 + 376 us the two pairs by tiles, 194 + 210 by
+// strips; 1001 x 4001: 1305 + 1535 against 740 + 810; 24 windows of 403 x 1777:
+// 790 + 805 against 325 + 363; a solve of 256 windows of 1001 x 4001: 9.7 ms
+// against 8.1.  Blocks of 12 steps (two workgroups a CU): the same for one shot,
 // 20 % more for 256; of 16 (one): 4 % less for one shot, twice the time for 256.
-// Four waves, wave 3 polling as well (four workgroups a CU): 5 to 15 % more.
+// A fifth wave for the upper strip's words: the same for one shot, but workgroups
+// of 320 threads fit a CU three times (256 shots 9.0 ms); wave 3 reading them: 5 to
+// 15 % more, its loads being the latest.
 constexpr int WP_B = STRIP_BLOCK;
 constexpr int WP_R = (64 + 4 * WP_B - 1) / WP_B * WP_B;  // ring steps: a step's 64, a block arriving, one leaving
 constexpr int WP_D = 3;                 // blocks of loads in flight
 constexpr int WP_P = 4;                 // blocks between a first sweep's progress words
-constexpr int WP_THREADS = 320;
+constexpr int WP_THREADS = 256;
 
 // Workgroup barrier after this wave's LDS operations (its global ones may stay
 // in flight).
 __device__ __forceinline__ void wp_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// x mod WP_R for 0 <= x < 2 WP_R
-__device__ __forceinline__ unsigned wp_wrap(unsigned x) { return min(x, x - WP_R); }
+// The ring's word of column c (0 <= c mod WP_R), row `lane`: byte offset, for the
+// columns c + u of a block with wp_word's wrap.
+__device__ __forceinline__ unsigned wp_column(int c, int lane) {
+  return (unsigned)((c + WP_R) % WP_R + lane) * 256u + 4u * (unsigned)lane;
+}
+template <class F>
+__device__ __forceinline__ F& wp_word(F* ring, unsigned column, int u) {
+  const unsigned x = column + 256u * u;
+  return *reinterpret_cast<F*>(reinterpret_cast<char*>(ring) + min(x, x - 256u * WP_R));
+}
 
 struct StripLds {
   float ring[WP_R * 64];
@@ -932,30 +942,29 @@ __device__ __forceinline__ void strip_walk(StripLds& L, const ShotDev sd, int r,
       }
     };
     wp_barrier();  // block -1
-    int nskip = 0;
-    for (int n = 0; n < nblk; ++n) {
-      const int t0 = n * WP_B, buf = n & 1;
-      const bool still = k.tinf_fixed && __builtin_amdgcn_readfirstlane(L.tinf[buf][0] & L.tinf[buf][1]) &&
-                         __all((te == TINF) & (tev == TINF));
-      if (still)
-        ++nskip;
-      else if (t0 >= 64 && t0 + WP_B <= NC)
-        block(t0, buf, std::false_type());
+    int n = 0;
+    // the blocks before the front: te and tev are still TINF (beyond its first
+    // block the test would cost 10 cycles a step and find nothing)
+    if (SB > 0 && k.tinf_fixed) {
+      for (; n < nblk && __builtin_amdgcn_readfirstlane(L.tinf[n & 1][0] & L.tinf[n & 1][1]); ++n) wp_barrier();
+      if (n && lane == 0) atomicAdd(ctl.nskip, n);
+    }
+    for (; n < nblk; ++n) {
+      const int t0 = n * WP_B;
+      if (t0 >= 64 && t0 + WP_B <= NC)
+        block(t0, n & 1, std::false_type());
       else
-        block(t0, buf, std::true_type());
+        block(t0, n & 1, std::true_type());
       wp_barrier();
     }
-    if (nskip && lane == 0) atomicAdd(ctl.nskip, nskip);
     wp_barrier();
     wp_barrier();
   } else if (wave == 1) {
     gfloat* __restrict__ T = gptr(sd.T);
     const unsigned row = (unsigned)prow<SA>(min(kg, NR), nzz);
-    const auto col = [&](int c) {  // (uniform address, the lane's offset in one register)
-      gfloat* p = T + (size_t)pcol<SB>(min(max(c, -1), NC), nxx) * nzz;
-      asm volatile("" : "+s"(p));
-      return p + row;
-    };
+    // column c, clamped to the grid, and the words from it to the next
+    gfloat* p = T + (size_t)pcol<SB>(0, nxx) * nzz;
+    const int pitch = SB * nzz;
     // second sweep: columns the first one has stored in this strip's rows (its
     // strips r0, r0 + 1)
     int seen = XMODE == 2 ? 0 : 1 << 30;
@@ -979,6 +988,7 @@ __device__ __forceinline__ void strip_walk(StripLds& L, const ShotDev sd, int r,
     const int sIdz = (int)((sd.sz + 0.5f * k.dz) / k.dz) + NB;
     const auto load = [&](int c0, float (&q)[WP_B]) {
       if (XMODE == 2) wait_for(c0 + WP_B - 1);
+      const bool inside = c0 + WP_B <= NC;
 #pragma unroll
       for (int u = 0; u < WP_B; ++u) {
         if (FIRST) {
@@ -992,29 +1002,58 @@ __device__ __forceinline__ void strip_walk(StripLds& L, const ShotDev sd, int r,
               q[u] = s_at(sd, nzz, i, j) * sqrtf(ddx * ddx + ddz * ddz);
             }
           }
-        } else if (XMODE == 2) {
-          q[u] = __hip_atomic_load(col(c0 + u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-          q[u] = *col(c0 + u);
+          asm volatile("" : "+s"(p));  // (uniform address, the lane's offset in one register)
+          q[u] = XMODE == 2 ? __hip_atomic_load(p + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : p[row];
+          p += inside || c0 + u < NC ? pitch : 0;
         }
       }
     };
     float q[WP_D][WP_B];
 #pragma unroll
     for (int d = 0; d < WP_D; ++d) load(d * WP_B, q[d]);
+    // the upper strip's words of a block's steps, read a block ahead
+    const unsigned long long* xup = sd.xh + (size_t)max(r - 1, 0) * sd.ldh;
+    const int ul = min(lane, WP_B - 1);
+    bool gave_up = false;
+    const auto word = [&](int n) {
+      return __hip_atomic_load((const gword*)(xup + min(n * WP_B + ul, NC - 1)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    };
+    unsigned long long w = r > 0 ? word(0) : 0ull;
     int run = 1 << 20;  // the last `run` columns are all TINF (those before the grid count)
     for (int n = -1; n < nblk + 2; n += WP_D)
 #pragma unroll
       for (int d = 0; d < WP_D; ++d)
         if (n + d < nblk + 2) {
           const int c_in = (n + d + 1) * WP_B;
-          const unsigned s0 = (unsigned)(c_in % WP_R) + lane;
+          const unsigned s0 = wp_column(c_in, lane);
 #pragma unroll
-          for (int u = 0; u < WP_B; ++u) {
-            L.ring[wp_wrap(s0 + u) * 64 + lane] = q[d][u];
-            run = __all(q[d][u] == TINF) ? run + 1 : 0;
+          for (int u = 0; u < WP_B; ++u) wp_word(L.ring, s0, u) = q[d][u];
+          // (only a first pair finds columns the front has not reached)
+          if (SB > 0) {
+#pragma unroll
+            for (int u = 0; u < WP_B; ++u) run = __all(q[d][u] == TINF) ? run + 1 : 0;
+            if (lane == 0) L.tinf[(n + d + 1) & 1][0] = run >= 64 + WP_B;
           }
-          if (lane == 0) L.tinf[(n + d + 1) & 1][0] = run >= 64 + WP_B;
+          float v = TINF;
+          if (r > 0 && n + d + 1 < nblk) {
+            for (int it = 0; !gave_up && !__all((unsigned)(w >> 32) == tagb); ++it) {
+              if (it > SPIN_LIMIT) {
+                if (lane == 0) atomicOr(ctl.err, 1);
+                gave_up = true;
+              }
+              __builtin_amdgcn_s_sleep(1);
+              w = word(n + d + 1);
+            }
+            if (c_in + ul < NC) v = __uint_as_float((unsigned)w);
+            w = word(n + d + 2);  // (before the column loads, which its wait then leaves in flight)
+          }
+          if (lane < WP_B) L.up[(n + d + 1) & 1][lane] = v;
+          if (SB > 0) {
+            const bool none = __all(v == TINF);
+            if (lane == 0) L.tinf[(n + d + 1) & 1][1] = none;
+          }
           load(c_in + WP_D * WP_B, q[d]);
           wp_barrier();
         }
@@ -1040,22 +1079,24 @@ __device__ __forceinline__ void strip_walk(StripLds& L, const ShotDev sd, int r,
       }
       // columns that lane 63 finished by the end of block n - 1
       if (c_out + WP_B > 0) {
-        const unsigned s0 = (unsigned)((c_out + WP_R) % WP_R) + lane;
+        const unsigned s0 = wp_column(c_out, lane);
         float v[WP_B];
 #pragma unroll
-        for (int u = 0; u < WP_B; ++u) v[u] = L.ring[wp_wrap(s0 + u) * 64 + lane];
+        for (int u = 0; u < WP_B; ++u) v[u] = wp_word(L.ring, s0, u);
+        gfloat* p = T + (size_t)pcol<SB>(c_out, nxx) * nzz;
+        if (row_ok) {
 #pragma unroll
-        for (int u = 0; u < WP_B; ++u)
-          if (row_ok && c_out + u >= 0 && c_out + u < NC) {
-            gfloat* p = T + (size_t)pcol<SB>(c_out + u, nxx) * nzz;
+          for (int u = 0; u < WP_B; ++u) {
             asm volatile("" : "+s"(p));
-            p[row] = v[u];
+            if (c_out + u >= 0 && c_out + u < NC) p[row] = v[u];
+            p += SB * nzz;
           }
+        }
       }
       wp_barrier();
     }
     if (XMODE == 1) progress(NC);
-  } else if (wave == 3) {
+  } else {
     // Cell (kap, lam) of step t: the z-other cell of lane k at lam = t - k + 1
     // (reference cell of step t + 1); lane 63's x-other cell is (64r + 64, t - 63).
     const int kap = 64 * r + lane;
@@ -1114,40 +1155,11 @@ __device__ __forceinline__ void strip_walk(StripLds& L, const ShotDev sd, int r,
           if (n + d + 1 + WP_D < nblk) load((n + d + 1 + WP_D) * WP_B, q[d], x63[d]);
           wp_barrier();
         }
-  } else {
-    const unsigned long long* xup = sd.xh + (size_t)max(r - 1, 0) * sd.ldh;
-    bool gave_up = false;
-    const int u = min(lane, WP_B - 1);
-    const auto word = [&](int n) {  // of block n's steps
-      return __hip_atomic_load((const gword*)(xup + min(n * WP_B + u, NC - 1)), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    };
-    unsigned long long w = r > 0 ? word(0) : 0ull;
-    for (int n = -1; n < nblk + 2; ++n) {
-      float v = TINF;
-      if (r > 0 && n + 1 < nblk) {
-        for (int it = 0; !gave_up && !__all((unsigned)(w >> 32) == tagb); ++it) {
-          if (it > SPIN_LIMIT) {
-            if (lane == 0) atomicOr(ctl.err, 1);
-            gave_up = true;
-          }
-          __builtin_amdgcn_s_sleep(1);
-          w = word(n + 1);
-        }
-        if ((n + 1) * WP_B + u < NC) v = __uint_as_float((unsigned)w);
-        w = word(n + 2);
-      }
-      const int buf = (n + 1) & 1;
-      if (lane < WP_B) L.up[buf][lane] = v;
-      const bool none = __all(v == TINF);
-      if (lane == 0) L.tinf[buf][1] = none;
-      wp_barrier();
-    }
   }
 }
 
 template <int SB, bool EQH, bool FD, bool FIRST_A>
-__global__ __launch_bounds__(WP_THREADS) void k_strip_pair(const ShotDev* __restrict__ shots_a,
+__global__ __launch_bounds__(WP_THREADS, STRIPS_PER_CU) void k_strip_pair(const ShotDev* __restrict__ shots_a,
                                                            const ShotDev* __restrict__ shots_b,
                                                            const int4* __restrict__ strips,
                                                            const int* __restrict__ qoff, int nzz, EikConsts k,
