@@ -112,22 +112,48 @@ class Eikonal:
         each position (x[k], z[k]): the tables of Migration::set_src_travel_times
         and set_rec_travel_times (src/migration/migration.cu:116-171), solved
         `chunk` positions per batch."""
+        out = None
+        for n, k, m, b in self._table_batches(x, z, type, schedule, chunk):
+            if out is None:
+                out = np.empty((n, self.nxx, self.nzz), np.float32)
+            for q in range(m):
+                out[k + q] = b.T(q)
+        return np.empty((0, self.nxx, self.nzz), np.float32) if out is None else out
+
+    def _device_tables(self, x, z, type=ISO, schedule=SCHED_TILED, chunk=64):
+        """The same grids as a CUDA tensor of the current device, without the
+        way through host memory."""
+        import torch
+
+        from .autograd import _DeviceArray
+        out = None
+        for n, k, m, b in self._table_batches(x, z, type, schedule, chunk):
+            if out is None:
+                out = torch.empty((n, self.nxx, self.nzz), dtype=torch.float32, device="cuda")
+            for q in range(m):
+                grid = torch.as_tensor(_DeviceArray(b.device_T_ptr(q)[0], self.nxx * self.nzz), device="cuda")
+                out[k + q].copy_(grid.view(self.nxx, self.nzz))
+            torch.cuda.current_stream().synchronize()  # the batch's grids go with it
+        if out is None:
+            out = torch.empty((0, self.nxx, self.nzz), dtype=torch.float32, device="cuda")
+        return out
+
+    def _table_batches(self, x, z, type, schedule, chunk):
+        """Solved batches of `chunk` whole-model shots: yields the number of
+        positions, the batch's first, its number, and the batch (closed afterwards)."""
         x = np.asarray(x, np.float64).ravel()
         z = np.asarray(z, np.float64).ravel()
         if x.shape != z.shape:
             raise ValueError("x and z must have the same length")
-        out = np.empty((len(x), self.nxx, self.nzz), np.float32)
         for k0 in range(0, len(x), chunk):
             shots = [(float(x[k]), float(z[k]), 0, self.nx, 0, 0) for k in range(k0, min(k0 + chunk, len(x)))]
             b = Batch(self, shots, None, None, type, schedule)
             try:
                 b.run()
                 b.status()
-                for q in range(len(shots)):
-                    out[k0 + q] = b.T(q)
+                yield len(x), k0, len(shots), b
             finally:
                 b.close()
-        return out
 
     def close(self):
         if getattr(self, "_h", None):

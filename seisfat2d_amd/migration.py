@@ -136,8 +136,8 @@ class Kirchhoff:
         check(lib().seisfat_kdm_create(eik._h, C.byref(p), self.nsrc, self.nrec, C.byref(h)))
         self._k = h
         if tables is None:
-            ts = eik.traveltime_tables(self.xsrc, zsrc, type=type)
-            tr = eik.traveltime_tables(self.xrec, zrec, type=type)
+            ts = eik._device_tables(self.xsrc, zsrc, type=type)
+            tr = eik._device_tables(self.xrec, zrec, type=type)
         else:
             ts, tr = tables
         self.set_tables(ts, tr)

@@ -490,3 +490,19 @@ def test_forward_tiles(oracle, torch, domain, nz, nx, nt, dt, shift):
         assert bad.mean() <= (1e-3 if domain == mig.ANGLE else 0.0)
     K.close()
     e.close()
+
+
+@pytest.mark.parametrize("n,chunk", [(0, 3), (1, 3), (3, 3), (7, 3)])
+def test_device_tables_are_the_host_tables(torch, n, chunk):
+    """The constructor's tables, solved into device memory batch by batch,
+    equal traveltime_tables bit for bit (batches partly filled, and none)."""
+    from seisfat2d_amd import Eikonal, models
+    w = models.rough(41, 77, 10.0, 10.0, seed=5, sigma=3.0, vlo=2000.0, vhi=3000.0)
+    e = Eikonal(41, 77, 10.0, 10.0)
+    e.set_slowness(w.s)
+    x = np.linspace(0.0, 700.0, n)
+    want = e.traveltime_tables(x, 0.0 * x, chunk=chunk)
+    got = e._device_tables(x, 0.0 * x, chunk=chunk)
+    assert got.is_cuda and got.dtype == torch.float32 and tuple(got.shape) == want.shape == (n, 83, 47)
+    assert np.array_equal(got.cpu().numpy(), want)
+    e.close()
