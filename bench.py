@@ -38,7 +38,7 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_sweep_pair_c3_256shots_traffic.txt")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_strip_pair_c3_256shots_traffic.txt")
 
 
 def profile_figure(key):
@@ -183,7 +183,7 @@ def bench_ani(steps):
                         "frac": achieved / HBM_PEAK_GBS,
                         "traffic": tr.get("traffic_bytes_per_step"),
                         "traffic_source": os.path.relpath(ANI_TRAFFIC_FILE, ROOT),
-                        "scope": "solve phase (4 k_sweep_pair launches + k_ani_table + k_quasi_slowness)",
+                        "scope": "solve phase (2 k_strip_pair and 2 k_sweep_pair launches + k_ani_table + k_quasi_slowness)",
                         "algorithmic_bytes_per_step": alg, "phase_ms": phase_s * 1e3}}
     b.close()
     e.close()
@@ -642,7 +642,7 @@ def main():
     nlaunch = b.num_sweep_launches
     # two launches: the fused sweep pairs (shots spread over the XCDs); four:
     # one persistent launch per sweep
-    sweep_kernel = "k_sweep_pair" if nlaunch == 2 else "k_sweep_persist"
+    sweep_kernel, unit = ("k_strip_pair", "64-row strips") if nlaunch == 2 else ("k_sweep_persist", "64x64 tiles")
     bytes_per_launch = BYTES_PER_CELL_UPDATE * cu / nlaunch
     avg_launch_s = sweep_ms / 1e3 / nlaunch
     achieved = bytes_per_launch / avg_launch_s / 1e9
@@ -722,7 +722,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": f"batched iso FSM, {len(w.shots)} shots on windows 1200-4001 wide of the "
                                f"1001x4001 dh=5 m layered model (seeded), one pass of 4 sweeps, tiled "
-                               f"schedule ({sweep_kernel} launches) on 64x64 tiles with schedule options "
+                               f"schedule ({sweep_kernel} launches) on {unit} with schedule options "
                                f"{json.dumps(sched, sort_keys=True)}"
                                f"{' (tuned on this device)' if tuned else ''}, one HIP graph per step",
                    "nz": w.nz, "nx": w.nx, "shots": len(w.shots), "cell_updates_per_step": cu,

@@ -844,12 +844,12 @@ __global__ __launch_bounds__(64) void k_sweep_pair(const ShotDev* __restrict__ s
 // costs 20 cycles of its block's barrier and first LDS reads (115 ns a step).  The
 // next strip starts 88 steps later (64 columns, a block, the words' way).  A 64 x
 // 64 tile, staged, run and written back by one wave, took twice that for its
-// hand-over.  With 256 shots four workgroups fit a CU (LDS), one wave 0 a SIMD; the
-// clock is lower then (1.9 GHz) and a step takes 190 ns.
+// hand-over.  With 256 shots four workgroups fit a CU (LDS), one wave 0 a SIMD, and
+// the launches move 4.0 TB/s (a large copy 4.7).
 // One shot of 201 x 1001: 313 + 376 us the two pairs by tiles, 194 + 210 by
 // strips; 1001 x 4001: 1305 + 1535 against 740 + 810; 24 windows of 403 x 1777:
 // 790 + 805 against 325 + 363; a solve of 256 windows of 1001 x 4001: 9.7 ms
-// against 8.1.  Blocks of 12 steps (two workgroups a CU): the same for one shot,
+// against 7.9.  Blocks of 12 steps (two workgroups a CU): the same for one shot,
 // 20 % more for 256; of 16 (one): 4 % less for one shot, twice the time for 256.
 // A fifth wave for the upper strip's words: the same for one shot, but workgroups
 // of 320 threads fit a CU three times (256 shots 9.0 ms); wave 3 reading them: 5 to
