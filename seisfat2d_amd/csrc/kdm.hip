@@ -49,6 +49,7 @@
 
 #include "../../include/seisfat2d_kdm.h"
 #include "eik_handle.h"
+#include "kdm_window.h"
 
 namespace seisfat {
 
@@ -72,7 +73,6 @@ struct KdmK {
   float da_m, r_da;     // da = da_m 2^da_e, da_m in [1, 2), and RN(1 / da_m)
   int da_e;
   unsigned nz_recip;    // floor(2^32 / nz) (nz > 1)
-  float ntf;     // (float)nt
   float tan_ap;  // tanf(aperture in radians), the reference's sigma / z
   float scale;   // 1 / (2 pi) as the reference rounds it
 };
@@ -286,18 +286,18 @@ __device__ __forceinline__ int t_index_mid(float xs, const KdmK& K) { return (in
 
 // Time index of a node for a trace with traveltime sum xs, as far as the
 // kernels use it: the reference's tId = f2i_rd(RN(xs / dt)) where that lies in
-// [0, nt) or xs is NaN (0), a value >= nt or negative otherwise.  When every
-// lane's sum lies in [2^-100, 2^100) (traveltimes are positive), RN(xs / dt)
-// comes from the two-instruction known-divisor division the exhaustive check
-// proved exact there and is floored after a clamp to nt: the index is then
-// >= nt exactly when xs >= thr.  Otherwise, for the whole wave, IEEE division
-// where that division is not proven, and thr, NaN and the sign decided
-// explicitly.
+// [0, nt) or xs is NaN (0), -1 or any value from nt to INT_MAX otherwise (so
+// nothing may be added to an index that is not known to be below nt).  When
+// every lane's sum lies in [2^-100, 2^100) (traveltimes are positive), RN(xs /
+// dt) comes from the two-instruction known-divisor division the exhaustive
+// check proved exact there, and the conversion truncates and saturates: the
+// index is then >= nt exactly when xs >= thr.  Otherwise, for the whole wave,
+// IEEE division where that division is not proven, and thr, NaN and the sign
+// decided explicitly.
 __device__ __forceinline__ int t_index(float xs, const KdmK& K) {
   const bool mid = __float_as_uint(xs) - 0x0d800000u < 0x64000000u;  // 2^-100 <= xs < 2^100
   const uint64_t all_mid = __builtin_amdgcn_ballot_w64(mid);
-  // a positive finite quotient: truncation is the floor, and the conversion
-  // saturates (far beyond nt)
+  // a positive finite quotient: truncation is the floor
   if (K.fastdiv_dt && all_mid == __builtin_amdgcn_read_exec()) return t_index_mid(xs, K);
   const float v = (K.fastdiv_dt && mid) ? fdiv(xs, K.zh_dt, K.zl_dt) : xs / K.dt;
   const int it = v != v ? 0 : (int)fminf(fmaxf(floorf(v), -1.0f), (float)K.nt);
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
 // tile (64 rows x FT_WAVES * NPT columns; lane = row, wave = NPT columns) and
 // slice of a source block's entries (the adjoint's blocks).  A node's source
 // quantities stay in registers for the whole slice and a receiver's are loaded
-// once for up to four traces, where the trace kernel below loads both for every
+// once for up to four traces, where the trace kernel above loads both for every
 // pair (32 B a pair: that, beyond L2, bounds it).  Each trace's contributions
 // gather in an LDS window of the samples the tile can reach: the index of the
 // tile's least and greatest traveltime sums bounds every node's (rounded
@@ -831,9 +831,10 @@ __global__ __launch_bounds__(64 * FT_WAVES) void k_kdm_forward_tile(
           E.cmp[k] = tcmp[E.t[k]];
           if (ANGLE) E.bin[k] = tcid[E.t[k]];
           // a NaN node's index is 0 and the lower bound NaN
-          E.lo[k] = lo != lo ? 0 : max(t_index(lo, K), 0);
-          E.len[k] = (lo != lo ? K.nt : min(t_index(hi, K) + 1, K.nt)) - E.lo[k];
-          if (E.len[k] <= 0) continue;  // every index negative
+          const SampleWindow win_k = lo != lo ? SampleWindow{0, K.nt} : sample_window(t_index(lo, K), t_index(hi, K), K.nt);
+          E.lo[k] = win_k.first;
+          E.len[k] = win_k.len;
+          if (win_k.len <= 0) continue;  // every index negative
           E.pass |= 1 << k;
           // every sum in [2^-100, 2^100)
           if (K.fastdiv_dt && lo >= 0x1p-100f && hi < 0x1p80f) E.pass |= 256 << k;
@@ -1245,7 +1246,6 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   K.nchunk = (int)((npts + 63) / 64);
   K.nsup = (K.nchunk + 63) / 64;
   K.nt = p->nt;
-  K.ntf = (float)p->nt;
   K.nang = p->domain == SEISFAT_KDM_ANGLE ? p->nang : 0;
   K.dx = h->dx;
   K.dz = h->dz;

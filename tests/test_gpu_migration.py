@@ -506,3 +506,48 @@ def test_device_tables_are_the_host_tables(torch, n, chunk):
     assert got.is_cuda and got.dtype == torch.float32 and tuple(got.shape) == want.shape == (n, 83, 47)
     assert np.array_equal(got.cpu().numpy(), want)
     e.close()
+
+
+# the forward's tile kernel, which a survey needs about 300 traces per tile and
+# block to be given (200 sources, 240 receivers): rows and columns at and beside
+# its tiles' edges, one slice of a block's entries and several, more entries than
+# one list, and tables that hold negative, NaN and finite or infinite "not
+# reached" values (1e30; 1e6 in a source and a receiver table), whose tiles'
+# windows end with the record and take several rounds of its 1024 samples.
+# Traces over the whole survey are compared, and those around the spoiled tables.
+@pytest.mark.parametrize("domain", [mig.IMAGE, mig.ANGLE])
+@pytest.mark.parametrize("nz,nx,nt,dt,shift,spoil", [
+    (63, 97, 400, 2e-3, 0.0, None), (64, 96, 400, 2e-3, 0.0, None), (65, 98, 900, 4e-4, 0.0, None),
+    (65, 98, 400, 2e-3, -0.05, 1e30), (130, 49, 700, 1e-3, 0.0, np.nan), (65, 98, 2100, 3.5e-4, 0.0, 1e30),
+    (65, 98, 2100, 3.5e-4, -0.05, 1e6), (65, 98, 900, 4e-4, 0.0, np.inf)])
+def test_forward_by_tiles(oracle, torch, domain, nz, nx, nt, dt, shift, spoil):
+    m, xs, xr = survey(nz=nz, nx=nx, nsrc=200, nrec=240, seed=nz)
+    e = Eikonal(nz, nx, m.dz, m.dx)
+    e.set_slowness(m.s)
+    ts, tr = (e.traveltime_tables(x, np.full_like(x, 11.0)) for x in (xs, xr))
+    tr += np.float32(shift)
+    if spoil is not None:
+        z = 25 if spoil == 1e6 else 35  # (where gradients are huge, no node beside both)
+        ts[70, 20:60, 30], tr[100, 30:44, z:z + 15] = spoil, spoil
+    K = make(e, m, xs, xr, domain, nt=nt, dt=dt, tables=(ts, tr), max_offset=1e4)
+    S = oracle.expand_boundary(m.s)
+    op = dict(dt=float(K.dt), dx=m.dx, dz=m.dz, aperture=30.0, da=float(K.da), nang=K.nang)
+    rng = np.random.default_rng(nz)
+    x = rng.standard_normal(K.model_shape).astype(np.float32)
+    got = torch.zeros((K.ntr, nt), device="cuda")
+    K.forward(torch.from_numpy(x).cuda(), got)
+    sub = np.arange(K.ntr)
+    near = (np.abs(K.src - 70) <= 1) & (np.abs(K.rec - 100) <= 6) | (sub % 997 == 0) | (sub >= K.ntr - 2)
+    sub = sub[near]
+    assert 60 <= len(sub) <= 120
+    got = got.cpu().numpy()[sub]
+    cid = None if domain == mig.IMAGE else K.cmp_id[sub]
+    a = (domain, False, S, ts, tr, K.src[sub], K.rec[sub], K.cmp[sub], cid)
+    want = oracle.kdm(*a, np.zeros((len(sub), nt), np.float32), x, **op)
+    bound = oracle.kdm(*a, np.zeros((len(sub), nt), np.float32), np.abs(x), **op)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin)
+    bad = np.abs(got - want)[fin] > (1e-5 * bound + 1e-30)[fin]
+    assert bad.mean() <= (1e-3 if domain == mig.ANGLE else 0.0)
+    K.close()
+    e.close()
