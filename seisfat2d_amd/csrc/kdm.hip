@@ -1064,6 +1064,7 @@ struct seisfat_kdm_s {
   unsigned long long* d_cnt = nullptr;  // k_kdm_tile_count's sums
   int ntz = 0, ntile = 0, tile_cols = 0;
   bool bounds_dirty = true;  // tables or traces changed since the bounds and the choice below
+  bool tables_in_graph = false;  // tables were set under capture: a replay may change them at any time
   bool by_tiles = false;     // the forward operator's kernel
   int nsplit = 1;            // its workgroups per tile and source block (slices of the entries)
   int* d_nonneg = nullptr;  // k_kdm_rec_nonneg's answer
@@ -1186,6 +1187,15 @@ void launch_forward(seisfat_kdm_s* k, const float* d_model, float* d_data, hipSt
   hipLaunchKernelGGL((k_kdm_forward<ANGLE, RDIV>), dim3(k->ntr), dim3(KDM_FWD_THREADS), lds, st, k->d_q, k->d_tmin,
                      k->h->d_spad, k->d_src, k->d_rec, k->d_cmp, k->d_cid, k->d_tmin2, k->nsrc, d_model, d_data,
                      k->K);
+}
+
+// After tables were set on a stream: the forward's bounds are stale.
+int tables_changed(seisfat_kdm_s* k, hipStream_t st) {
+  k->bounds_dirty = true;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  KHIP(hipStreamIsCapturing(st, &cap));
+  if (cap != hipStreamCaptureStatusNone) k->tables_in_graph = true;
+  return SEISFAT_OK;
 }
 
 bool cmp_ok(float c) { return c == 0.0f || (std::fabs(c) >= 0x1p-36f && std::fabs(c) < 0x1p40f); }
@@ -1333,8 +1343,7 @@ int seisfat_kdm_set_tables(seisfat_kdm_t k, const float* d_src, const float* d_r
   std::fill(k->tab_set.begin(), k->tab_set.end(), 1);
   k->tabs_missing = 0;
   k->rec_dirty = true;
-  k->bounds_dirty = true;
-  return SEISFAT_OK;
+  return tables_changed(k, st);
 }
 
 int seisfat_kdm_set_table(seisfat_kdm_t k, int which, int index, const float* d_table, void* stream) {
@@ -1352,8 +1361,7 @@ int seisfat_kdm_set_table(seisfat_kdm_t k, int which, int index, const float* d_
     --k->tabs_missing;
   }
   if (which) k->rec_dirty = true;
-  k->bounds_dirty = true;
-  return SEISFAT_OK;
+  return tables_changed(k, st);
 }
 
 namespace {
@@ -1367,8 +1375,12 @@ int ready(seisfat_kdm_s* k) {
 }
 
 // The forward operator's tile bounds and its choice between its two kernels,
-// once per tables and traces: it waits for two counts.  Where that cannot be
-// done (a stream under capture) the kernel that needs no bounds runs.  In units
+// once per tables and traces: it waits for two counts.  A stream under capture
+// cannot: there the choice stands as the last call made it (the kernel that
+// needs no bounds if tables or traces changed since), and the bounds' launch is
+// recorded with the tile kernel's, so that a replay follows tables set after the
+// capture.  The same launch precedes every tile kernel once tables were set
+// under capture.  In units
 // of a wave's column and round (0.1 ns on the whole chip), a tile kernel's
 // workgroup costs FT_COST before its first round, and the trace kernel takes
 // 1.4 (tables that stay in the caches) to 3 units per column; either one needs
@@ -1380,13 +1392,15 @@ int ready(seisfat_kdm_s* k) {
 // domain, 2292 traces of 1501 at 2 ms: 6.2 / 3.2.
 constexpr double FT_COST = 400.0, FT_TRACE = 1.6;
 int derive_bounds(seisfat_kdm_s* k, hipStream_t st) {
-  if (!k->bounds_dirty) return SEISFAT_OK;
-  k->by_tiles = false;
+  if (k->bounds_dirty) k->by_tiles = false;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   KHIP(hipStreamIsCapturing(st, &cap));
-  if (cap != hipStreamCaptureStatusNone) return SEISFAT_OK;
+  const bool captured = cap != hipStreamCaptureStatusNone;
+  const bool choose = !captured && k->bounds_dirty;
+  if (!choose && !(k->by_tiles && (captured || k->tables_in_graph))) return SEISFAT_OK;
   hipLaunchKernelGGL(k_kdm_tile_bounds, dim3((k->ntile + 3) / 4, std::min(k->nsrc + k->nrec, 65535)), dim3(256), 0, st,
                      k->d_q, k->kq, k->nsrc + k->nrec, k->ntz, k->ntile, k->tile_cols, k->K, k->d_tlo, k->d_thi);
+  if (!choose) return SEISFAT_OK;
   hipLaunchKernelGGL(k_kdm_clear, dim3(1), dim3(2), 0, st, k->d_cnt);
   hipLaunchKernelGGL(k_kdm_tile_count, dim3(k->ntr), dim3(64), 0, st, k->d_tlo, k->d_thi, k->ntile, k->d_src, k->d_rec,
                      k->nsrc, k->K, k->d_cnt);

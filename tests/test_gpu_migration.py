@@ -551,3 +551,48 @@ def test_forward_by_tiles(oracle, torch, domain, nz, nx, nt, dt, shift, spoil):
     assert bad.mean() <= (1e-3 if domain == mig.ANGLE else 0.0)
     K.close()
     e.close()
+
+
+@pytest.mark.parametrize("domain", [mig.IMAGE, mig.ANGLE])
+def test_captured_forward_follows_the_tables(torch, domain):
+    """A forward captured after an eager one (which took the tile kernel)
+    replays with the tables set since, and an eager one follows tables that a
+    replay has set."""
+    nz, nx, nt, dt = 65, 98, 400, 2e-3
+    m, xs, xr = survey(nz=nz, nx=nx, nsrc=200, nrec=240, seed=nz)
+    e = Eikonal(nz, nx, m.dz, m.dx)
+    e.set_slowness(m.s)
+    ts, tr = (torch.from_numpy(e.traveltime_tables(x, np.full_like(x, 11.0))).cuda() for x in (xs, xr))
+    K = make(e, m, xs, xr, domain, nt=nt, dt=dt, tables=(ts, tr), max_offset=1e4)
+    x = torch.rand(K.model_shape, device="cuda") + 0.5
+    K.forward(x)
+    out = torch.zeros((K.ntr, nt), device="cuda")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        K.forward(x, out)
+    for shift in (0.2, -0.05, 0.0):
+        K.set_tables(ts, tr + shift)
+        out.zero_()
+        g.replay()
+        want = K.forward(x)
+        torch.cuda.synchronize()
+        assert bool(want.abs().max() > 0)
+        assert float((out - want).abs().max()) <= 1e-4 * float(want.abs().max()), shift
+    rec = tr.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        K.set_tables(ts, rec)
+    K.set_tables(ts, rec)
+    K.forward(x)
+    for shift in (0.2, 0.1):
+        rec.copy_(tr + shift)
+        g.replay()
+        got = K.forward(x)
+        K.set_tables(ts, tr + shift)
+        want = K.forward(x)
+        assert float((got - want).abs().max()) <= 1e-4 * float(want.abs().max()), shift
+        rec.copy_(tr)
+        K.set_tables(ts, rec)
+        K.forward(x)
+    K.close()
+    e.close()
