@@ -237,26 +237,22 @@ __global__ __launch_bounds__(256) void k_kdm_tmin2(const float* __restrict__ tmi
   }
 }
 
-// Per table, the least of its super-chunk minima (NaN-propagating): one wave
-// per table.
-__global__ __launch_bounds__(64) void k_kdm_tmin3(const float* __restrict__ tmin2, KdmK K, float* __restrict__ tmin3) {
-  const int lane = threadIdx.x;
-  float v = __builtin_inff();
-  for (int k = lane; k < K.nsup; k += 64) v = min_nan(v, tmin2[(size_t)blockIdx.x * K.nsup + k]);
-  for (int off = 32; off >= 1; off >>= 1) v = min_nan(v, __shfl_xor(v, off, 64));
-  if (lane == 0) tmin3[blockIdx.x] = v;
-}
-
-// Whether no receiver-table value at an image point is negative or NaN: a
-// source may then be passed over on its own minimum.  On the device, so that
-// an operator's launch waits for nothing (reading the chunk minima back took
-// 1 ms on 201 tables of 1001 x 1001).
-__global__ __launch_bounds__(64) void k_kdm_rec_nonneg(const float* __restrict__ rec_tmin3, int nrec,
-                                                       int* __restrict__ flag) {
+// Whether a receiver table holds a negative value or a NaN at an image point
+// (its least super-chunk minimum, NaN-propagating): one wave per table writes
+// neg[r] and keeps *nneg the number of such tables.  While it is 0 a source may
+// be passed over on its own minimum.  Counted as tables are set, so that it
+// holds for whatever runs after them, on any stream and in a replayed graph
+// (reading the chunk minima back took 1 ms on 201 tables of 1001 x 1001).
+__global__ __launch_bounds__(64) void k_kdm_rec_neg(const float* __restrict__ tmin2, KdmK K, int* __restrict__ neg,
+                                                    int* __restrict__ nneg) {
+  const int lane = threadIdx.x, r = blockIdx.x;
   bool ok = true;
-  for (int k = threadIdx.x; k < nrec; k += 64) ok &= rec_tmin3[k] >= 0.0f;
-  const bool all = __all(ok);
-  if (threadIdx.x == 0) *flag = all ? 1 : 0;
+  for (int k = lane; k < K.nsup; k += 64) ok &= tmin2[(size_t)r * K.nsup + k] >= 0.0f;
+  const int now = __all(ok) ? 0 : 1, before = neg[r];
+  if (lane == 0 && now != before) {
+    neg[r] = now;
+    atomicAdd(nneg, now - before);
+  }
 }
 
 struct Q7 {
@@ -429,9 +425,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANGLE ? 6 :
                                                      const float* __restrict__ tcmp, const int* __restrict__ tcid,
                                                      int nb, int nsrc, const float* __restrict__ data,
                                                      float* __restrict__ model, float* __restrict__ part,
-                                                     const int* __restrict__ rec_flag, KdmK K) {
+                                                     const int* __restrict__ nneg, KdmK K) {
   constexpr int KQ = kq_words(ANGLE);
-  const bool rec_nonneg = *rec_flag != 0;
+  const bool rec_nonneg = *nneg == 0;
   const int p0 = blockIdx.x * blockDim.x + threadIdx.x;
   const int nparts = gridDim.y, h = blockIdx.y;
   const int b_begin = (int)((long long)nb * h / nparts), b_end = (int)((long long)nb * (h + 1) / nparts);
@@ -1058,7 +1054,6 @@ struct seisfat_kdm_s {
   int kq = 0;              // words per node and table (kq_words)
   float* d_tmin = nullptr; // per-table chunk minima of T, (nsrc + nrec) x nchunk
   float* d_tmin2 = nullptr; // per-table minima over 64 chunks, (nsrc + nrec) x nsup
-  float* d_tmin3 = nullptr; // per-table minimum, nsrc + nrec
   float* d_tlo = nullptr;   // tile bounds of the forward operator, (nsrc + nrec) x ntile each
   float* d_thi = nullptr;
   unsigned long long* d_cnt = nullptr;  // k_kdm_tile_count's sums
@@ -1067,7 +1062,7 @@ struct seisfat_kdm_s {
   bool tables_in_graph = false;  // tables were set under capture: a replay may change them at any time
   bool by_tiles = false;     // the forward operator's kernel
   int nsplit = 1;            // its workgroups per tile and source block (slices of the entries)
-  int* d_nonneg = nullptr;  // k_kdm_rec_nonneg's answer
+  int* d_neg = nullptr;     // per receiver table: a negative or NaN value; then their number (k_kdm_rec_neg)
   int* d_src = nullptr;    // trace tables
   int* d_rec = nullptr;
   int nb = 0;              // source blocks of the adjoint
@@ -1082,7 +1077,6 @@ struct seisfat_kdm_s {
   int tabs_missing = 0;
   unsigned s_version = 0;      // the handle's slowness the set tables were evaluated with
   bool taper_geom = false;     // the divisors and x positions allow rdiv for the taper (taper_geometry_ok)
-  bool rec_dirty = true;       // receiver minima changed since d_nonneg was derived
 };
 
 namespace {
@@ -1158,8 +1152,9 @@ void launch_prep(seisfat_kdm_s* k, const float* d_tables, int tab0, int ntab, hi
   const int blocks2 = (int)std::min<size_t>((ns + 3) / 4, 16384);
   hipLaunchKernelGGL(k_kdm_tmin2, dim3(blocks2), dim3(256), 0, st, tmin, ntab, k->K,
                      k->d_tmin2 + (size_t)tab0 * k->K.nsup);
-  hipLaunchKernelGGL(k_kdm_tmin3, dim3(ntab), dim3(64), 0, st, k->d_tmin2 + (size_t)tab0 * k->K.nsup, k->K,
-                     k->d_tmin3 + tab0);
+  if (tab0 >= k->nsrc)
+    hipLaunchKernelGGL(k_kdm_rec_neg, dim3(ntab), dim3(64), 0, st, k->d_tmin2 + (size_t)tab0 * k->K.nsup, k->K,
+                       k->d_neg + (tab0 - k->nsrc), k->d_neg + k->nrec);
 }
 
 // The operators' launches, one instantiation per domain and taper division.
@@ -1168,7 +1163,7 @@ void launch_adjoint(seisfat_kdm_s* k, const float* d_data, float* d_model, hipSt
   const dim3 grid((k->K.npts + 255) / 256, k->nparts);
   hipLaunchKernelGGL((k_kdm_adjoint<ANGLE, KDM_SB, RDIV>), grid, dim3(256), 0, st, k->d_q, k->d_tmin, k->h->d_spad,
                      k->d_bsrc, k->d_bent, k->d_ent, k->d_cmp, k->d_cid, k->nb, k->nsrc, d_data, d_model,
-                     ANGLE ? nullptr : k->d_part, k->d_nonneg, k->K);
+                     ANGLE ? nullptr : k->d_part, k->d_neg + k->nrec, k->K);
 }
 
 template <bool ANGLE, bool RDIV>
@@ -1287,8 +1282,8 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   hipError_t e = hipMalloc((void**)&k->d_q, (size_t)(nsrc + nrec) * k->kq * npts * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin, (size_t)(nsrc + nrec) * K.nchunk * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin2, (size_t)(nsrc + nrec) * K.nsup * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin3, (size_t)(nsrc + nrec) * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&k->d_nonneg, sizeof(int));
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_neg, ((size_t)nrec + 1) * sizeof(int));
+  if (e == hipSuccess) e = hipMemset(k->d_neg, 0, ((size_t)nrec + 1) * sizeof(int));
   k->ntz = (K.nz + 63) / 64;
   k->tile_cols = FT_WAVES * ft_npt(p->domain == SEISFAT_KDM_ANGLE);
   k->ntile = k->ntz * ((K.nx + k->tile_cols - 1) / k->tile_cols);
@@ -1316,8 +1311,7 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
     kfree(k->d_q);
     kfree(k->d_tmin);
     kfree(k->d_tmin2);
-    kfree(k->d_tmin3);
-    kfree(k->d_nonneg);
+    kfree(k->d_neg);
     kfree(k->d_tlo);
     kfree(k->d_thi);
     kfree(k->d_cnt);
@@ -1342,7 +1336,6 @@ int seisfat_kdm_set_tables(seisfat_kdm_t k, const float* d_src, const float* d_r
   KHIP(hipGetLastError());
   std::fill(k->tab_set.begin(), k->tab_set.end(), 1);
   k->tabs_missing = 0;
-  k->rec_dirty = true;
   return tables_changed(k, st);
 }
 
@@ -1360,7 +1353,6 @@ int seisfat_kdm_set_table(seisfat_kdm_t k, int which, int index, const float* d_
     k->tab_set[tab] = 1;
     --k->tabs_missing;
   }
-  if (which) k->rec_dirty = true;
   return tables_changed(k, st);
 }
 
@@ -1413,17 +1405,6 @@ int derive_bounds(seisfat_kdm_s* k, hipStream_t st) {
   const double by_trace = FT_TRACE * k->tile_cols * (double)n[0] / std::min(1.0, k->ntr / 512.0);
   k->by_tiles = by_tile < by_trace && k->ntile <= 8 * 65535 && 4096.0 * k->nb * k->nsplit < 0x1p32 && k->K.dt < 0x1p60f;
   k->bounds_dirty = false;
-  return SEISFAT_OK;
-}
-
-// d_nonneg from the current receiver minima, before an adjoint.  A launch that
-// is only being captured has not happened yet: the next call launches it too.
-int derive_nonneg(seisfat_kdm_s* k, hipStream_t st) {
-  if (!k->rec_dirty) return SEISFAT_OK;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  KHIP(hipStreamIsCapturing(st, &cap));
-  hipLaunchKernelGGL(k_kdm_rec_nonneg, dim3(1), dim3(64), 0, st, k->d_tmin3 + k->nsrc, k->nrec, k->d_nonneg);
-  if (cap == hipStreamCaptureStatusNone) k->rec_dirty = false;
   return SEISFAT_OK;
 }
 
@@ -1518,7 +1499,6 @@ int seisfat_kdm_adjoint(seisfat_kdm_t k, const float* d_data, float* d_model, vo
   if (const int rc = ready(k)) return rc;
   if (k->ntr == 0) return SEISFAT_OK;  // no traces: the model is unchanged
   if (!d_data || !d_model) return kfail(SEISFAT_EINVAL, "null buffer");
-  if (const int rc = derive_nonneg(k, st)) return rc;
   const bool rd = k->K.taper_rdiv != 0;
   if (k->p.domain == SEISFAT_KDM_IMAGE) {
     if (rd)
@@ -1566,8 +1546,7 @@ int seisfat_kdm_destroy(seisfat_kdm_t k) {
   kfree(k->d_q);
   kfree(k->d_tmin);
   kfree(k->d_tmin2);
-  kfree(k->d_tmin3);
-  kfree(k->d_nonneg);
+  kfree(k->d_neg);
   kfree(k->d_tlo);
   kfree(k->d_thi);
   kfree(k->d_cnt);

@@ -596,3 +596,45 @@ def test_captured_forward_follows_the_tables(torch, domain):
         K.forward(x)
     K.close()
     e.close()
+
+
+@pytest.mark.parametrize("domain", [mig.IMAGE, mig.ANGLE])
+def test_adjoint_knows_negative_receiver_tables_on_any_stream(torch, domain):
+    """Whether a source may be passed over on its own traveltimes depends on
+    the receivers' being non-negative: as the tables stand, also for an
+    adjoint on a second stream and for a captured one replayed."""
+    nz, nx, nt, dt = 64, 90, 100, 1e-3
+    m, xs, xr = survey(nz=nz, nx=nx, nsrc=3, nrec=50, seed=2)
+    e = Eikonal(nz, nx, m.dz, m.dx)
+    e.set_slowness(m.s)
+    ts, tr = (torch.from_numpy(e.traveltime_tables(x, np.full_like(x, 11.0))).cuda() for x in (xs, xr))
+    K = make(e, m, xs, xr, domain, nt=nt, dt=dt, tables=(ts, tr), max_offset=1e4)
+    d = torch.rand((K.ntr, nt), device="cuda") + 0.5
+    K.adjoint(d)
+    captured = torch.zeros(K.model_shape, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        K.adjoint(d, captured)
+    K.set_tables(ts, tr - 0.15)  # sums within the record where the source's time alone is past it
+    second, out = torch.cuda.Stream(), torch.zeros(K.model_shape, device="cuda")
+    second.wait_stream(torch.cuda.current_stream())
+    a = torch.randn(8192, 8192, device="cuda")
+    for _ in range(4):  # the first stream's adjoint has yet to start when the second's runs
+        torch.mm(a, a)
+    late = K.adjoint(d)
+    with torch.cuda.stream(second):
+        K.adjoint(d, out)
+    torch.cuda.synchronize()
+    captured.zero_()
+    g.replay()
+    want = K.adjoint(d)
+    torch.cuda.synchronize()
+    one_by_one = K.adjoint(d)
+    for got in (out, late, captured, one_by_one):
+        assert float((got - want).abs().max()) <= 1e-4 * float(want.abs().max())
+    # the sources' own times leave nothing of the model beyond the record
+    K.set_tables(ts, tr)
+    short = K.adjoint(d)
+    assert bool((want != 0).sum() > 1.5 * (short != 0).sum())
+    K.close()
+    e.close()
