@@ -193,7 +193,8 @@ int seisfat_batch_num_sweep_launches(seisfat_batch_t b);
 int seisfat_batch_sweep_ms(seisfat_batch_t b, float* ms);
 /* Tiles of the last completed run (or converged-mode pass) of the persistent
  * tiled schedule: *total = the tiles of all its sweeps (fused pairs of an
- * isotropic solve: its strips' blocks of 8 steps), *skipped = those whose
+ * isotropic solve: its strips' blocks of 8 steps, not those of a
+ * converged-mode pass, which runs by tiles), *skipped = those whose
  * every input (old traveltimes, upwind row, carry-in) was the "not reached"
  * value 1e6, which the geometry provably keeps at 1e6, so the kernel did not
  * run their steps (results unchanged).  Diagnostics with no reference

@@ -754,13 +754,13 @@ int run_batch(seisfat_batch_s* b, hipStream_t st) {
 // skipped at once after convergence), and the picks; the host reads the skip
 // word after each chunk.
 int run_converged(seisfat_batch_s* b, int max_passes, int chunk, int* passes, hipStream_t st) {
-  b->last_run_plain = false;  // gated passes leave their queues untouched
   seisfat_eik_s* h = b->h;
   if (b->type != SEISFAT_ISO || b->schedule != SEISFAT_SCHED_TILED)
     return fail(SEISFAT_EINVAL, "converged mode covers isotropic batches of the tiled schedule");
   if (max_passes < 1 || max_passes > (1 << 20)) return fail(SEISFAT_EINVAL, "max_passes must be in [1, 2^20]");
   if (chunk < 2 || chunk > 256) return fail(SEISFAT_EINVAL, "chunk must be in [2, 256]");
   if (!h->has_s) return fail(SEISFAT_ESTATE, "slowness rejected or not set since the batch was created");
+  b->last_run_plain = false;  // gated passes leave their queues untouched
   chunk += chunk & 1;  // even: the change words alternate by pass parity
   if (!b->d_conv)
     if (int rc = dalloc(&b->d_conv, (size_t)CONV_WORDS)) return rc;
@@ -1361,8 +1361,10 @@ int seisfat_batch_status(seisfat_batch_t b) {
 int seisfat_batch_tile_counts(seisfat_batch_t b, long long* total, long long* skipped) {
   if (!b || !total || !skipped) return fail(SEISFAT_EINVAL, "null batch or output");
   if (!b->d_ctl) return fail(SEISFAT_EINVAL, "tile counts exist for the persistent tiled schedule only");
-  const long long tiles = b->pairs ? 2LL * (long long)b->pair_tiles.size() : 4LL * b->ntiles;
-  *total = (b->pairs ? 2 * b->strip_blocks : tiles) + (b->type == SEISFAT_ANI ? tiles : 0);
+  // the fused pairs' isotropic solve counts its strips' blocks; a converged-mode
+  // pass runs by tiles whatever the option
+  const long long tiles = 4LL * b->ntiles;
+  *total = (b->pairs && b->last_run_plain ? 2 * b->strip_blocks : tiles) + (b->type == SEISFAT_ANI ? tiles : 0);
   int n = 0;
   HIPCHK(hipEventSynchronize(b->ev_done));
   HIPCHK(hipMemcpyAsync(&n, b->d_ctl + CTL_SKIP, sizeof(int), hipMemcpyDeviceToHost, b->h->stream));

@@ -77,3 +77,24 @@ def test_converged_mode_rejects_other_schedules():
     assert ex.value.code == capi.EINVAL
     b.close()
     e.close()
+
+
+def test_tile_counts_follow_the_kind_of_run():
+    """Totals of a run by fused pairs (8-step blocks of 64-row strips) and of a
+    converged-mode pass (64 x 64 tiles), in either order."""
+    nz, dh, widths = 150, 10.0, (200, 67)
+    e = Eikonal(nz, 200, dh, dh)
+    e.set_slowness(np.full((200, nz), 5e-4, np.float32))
+    b = e.batch([(100.0, 0.0, 0, w, 0, 0) for w in widths], schedule=SCHED_TILED)
+    strips = -(-(nz + 4) // 64)
+    tiles = 4 * strips * sum(-(-(w + 4 + 63) // 64) for w in widths)
+    blocks = 4 * strips * sum(-(-(w + 4 + 63) // 8) for w in widths)
+    for _ in range(2):
+        b.run()
+        total, skipped = b.tile_counts()
+        assert total == (blocks if b.num_sweep_launches == 2 else tiles) and skipped <= total
+        b.run_converged()
+        total, skipped = b.tile_counts()
+        assert total == tiles and skipped <= total
+    b.close()
+    e.close()
