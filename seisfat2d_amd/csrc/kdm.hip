@@ -974,12 +974,16 @@ __global__ __launch_bounds__(256) void k_trace_conv(const float* __restrict__ in
 // thread per sample reads and converts two operands per tap).  A product of
 // two floats is exact in double, so the fma is the plain sum's rounding, and a
 // sample outside the trace adds h * 0 (the host checks that h is finite): the
-// same bits.  A workgroup's threads (at most 256) take `tpw` traces of `groups`
-// groups each, or one segment of CONV_SEG samples of a longer one; the samples lie in
-// LDS with one word of padding per eight, so the threads' reads (stride 9) meet
-// no bank conflict.  Bound by FP64 issue: 3609 traces of 8001 samples, 234
-// taps: 0.282 ms (24 T fma/s), 1.77 ms with a sample per thread; 1001 samples:
-// 0.053 against 0.132-0.144 ms.
+// same bits.  A wave passes over the taps that meet no sample of the trace from
+// any of its sums, most of them where the wavelet is longer than the record
+// (1000 traces of 1000 samples, 13000 taps, forward and adjoint: 109 and 32 us;
+// 1318 when every tap was walked, 464 and 82 with a sample per thread).  A
+// workgroup's threads (at most 256) take `tpw` traces of `groups` groups each, or
+// one segment of CONV_SEG samples of a longer one; the samples lie in LDS with one
+// word of padding per eight, so the threads' reads (stride 9) meet no bank
+// conflict.  Bound by FP64 issue: 3609 traces of 8001 samples, 234 taps: 0.282 ms
+// (24 T fma/s), 1.77 ms with a sample per thread; 1001 samples: 0.053 against
+// 0.132-0.144 ms.
 constexpr int CONV_R = 8, CONV_SEG = 256 * CONV_R;
 constexpr int CONV_TAPS = 896;  // wavelet samples per k_put_taps launch (its argument's size)
 struct Taps {
@@ -999,23 +1003,33 @@ __global__ __launch_bounds__(256) void k_trace_conv_reg(const float* __restrict_
   const int tl = threadIdx.x / groups;  // the thread's trace in the workgroup
   const int t0 = blockIdx.x * tpw, k0 = blockIdx.y * CONV_SEG;
   const int pitch = span + span / CONV_R + 1;
+  // the taps that meet the trace from the groups a .. b of the workgroup (the
+  // first one a multiple of CONV_R)
+  const auto tap0 = [&](int b) { return max(-(k0 + b * CONV_R + CONV_R - 1 + off), 0) / CONV_R * CONV_R; };
+  const auto tap1 = [&](int a) { return min(nw, nt - (max(k0 + a * CONV_R, first) + off)); };
+  const int base = tap0(groups - 1), need = groups * CONV_R + max(tap1(0) - base, 0) + 2 * CONV_R;
   for (int tr = 0; tr < tpw; ++tr)
-    for (int q = threadIdx.x; q < span; q += blockDim.x) {
-      const int x = k0 + off + q;
+    for (int q = threadIdx.x; q < need; q += blockDim.x) {
+      const int x = k0 + off + base + q;
       sm[tr * pitch + q + q / CONV_R] = (t0 + tr < ntr && x >= 0 && x < nt) ? in[(size_t)(t0 + tr) * nt + x] : 0.0f;
     }
   __syncthreads();
   const int g = threadIdx.x - tl * groups, k = k0 + g * CONV_R;
+  // (a wave's lanes of one trace: its first and last group; of several: any)
+  const int ga = __builtin_amdgcn_readfirstlane(g), gb = __builtin_amdgcn_readlane(g, 63);
+  const bool one = __builtin_amdgcn_readfirstlane(tl) == __builtin_amdgcn_readlane(tl, 63);
+  const int i0 = tap0(one ? gb : groups - 1);
+  const int i1 = k0 + (one ? gb : groups - 1) * CONV_R + CONV_R - 1 < first ? i0 : tap1(one ? ga : 0);
   if (tl >= tpw || t0 + tl >= ntr || k >= nt) return;
-  const float* __restrict__ x = sm + tl * pitch + g * (CONV_R + 1);
+  const float* __restrict__ x = sm + tl * pitch + (g + (i0 - base) / CONV_R) * (CONV_R + 1);
   double acc[CONV_R], X[2 * CONV_R];
 #pragma unroll
   for (int o = 0; o < CONV_R; ++o) {
     acc[o] = 0.0;
     X[o] = x[o];
   }
-  int i = 0;
-  for (; i + CONV_R <= nw; i += CONV_R) {
+  int i = i0;
+  for (; i + CONV_R <= i1; i += CONV_R) {
     x += CONV_R + 1;
 #pragma unroll
     for (int o = 0; o < CONV_R; ++o) X[CONV_R + o] = x[o];
@@ -1031,7 +1045,7 @@ __global__ __launch_bounds__(256) void k_trace_conv_reg(const float* __restrict_
   for (int o = 0; o < CONV_R - 1; ++o) X[CONV_R + o] = x[o];
 #pragma unroll
   for (int u = 0; u < CONV_R - 1; ++u) {
-    if (i + u >= nw) break;
+    if (i + u >= i1) break;
 #pragma unroll
     for (int o = 0; o < CONV_R; ++o) acc[o] = __builtin_fma(h[i + u], X[u + o], acc[o]);
   }
@@ -1565,24 +1579,32 @@ int seisfat_trace_convolve(int adjoint, int ntr, int nt, const float* wavelet, i
   const int shift = nw / 2 + nw / 10;
   hipStream_t st = (hipStream_t)stream;
   const size_t n = (size_t)ntr * nt;
-  // samples a workgroup stages per trace: its outputs, the taps, and up to the next whole group
+  // out[k] = nfft sum_i h[i] in[k + off + i] for k >= first, and the taps that
+  // meet a sample of the trace from any of these outputs
+  const int first = adjoint ? shift : 0;
+  long long off = adjoint ? -(long long)shift : (long long)shift - nw + 1;
+  const int tap0 = (int)std::max<long long>(0, -(nt - 1 + off));
+  const int ntap = first >= nt ? 0 : (int)std::max<long long>(0, std::min<long long>(nw, nt - (first + off)) - tap0);
+  off += tap0;
+  // samples a workgroup stages per trace: its outputs, its taps, and up to the next whole group
   const int groups = std::min((nt + CONV_R - 1) / CONV_R, 256);
-  const long long span = (long long)groups * CONV_R + ((nw + CONV_R - 1) / CONV_R + 1) * CONV_R;
+  const long long taps = std::min<long long>(ntap, (long long)nt + (groups + 1) * CONV_R);
+  const long long span = (long long)groups * CONV_R + (taps + CONV_R - 1) / CONV_R * CONV_R + 2 * CONV_R;
   const size_t lds1 = (size_t)(span + span / CONV_R + 1) * sizeof(float);
   if (lds1 <= 65536 && std::all_of(wavelet, wavelet + nw, [](float v) { return std::isfinite(v); })) {
     // several short traces per workgroup, within 40 KB (four workgroups per CU)
     const int tpw = (int)std::max<size_t>(1, std::min<size_t>(256 / groups, 40960 / lds1));
     double* d_h = nullptr;
-    KHIP(hipMallocAsync((void**)&d_h, nw * sizeof(double), st));
-    for (int i0 = 0; i0 < nw; i0 += CONV_TAPS) {
+    KHIP(hipMallocAsync((void**)&d_h, std::max(ntap, 1) * sizeof(double), st));
+    for (int i0 = 0; i0 < ntap; i0 += CONV_TAPS) {
       Taps a;
-      const int m = std::min(CONV_TAPS, nw - i0);
-      for (int i = 0; i < m; ++i) a.w[i] = adjoint ? wavelet[i0 + i] : wavelet[nw - 1 - (i0 + i)];
+      const int m = std::min(CONV_TAPS, ntap - i0), t = tap0 + i0;
+      for (int i = 0; i < m; ++i) a.w[i] = adjoint ? wavelet[t + i] : wavelet[nw - 1 - (t + i)];
       hipLaunchKernelGGL(k_put_taps, dim3(1), dim3(256), 0, st, a, m, d_h + i0);
     }
     const dim3 grid((ntr + tpw - 1) / tpw, (nt + CONV_SEG - 1) / CONV_SEG);
-    hipLaunchKernelGGL(k_trace_conv_reg, grid, dim3((tpw * groups + 63) / 64 * 64), tpw * lds1, st, d_in, d_out, ntr, nt, d_h, nw,
-                       adjoint ? -shift : shift - nw + 1, adjoint ? shift : 0, (double)nfft, tpw, groups, (int)span);
+    hipLaunchKernelGGL(k_trace_conv_reg, grid, dim3((tpw * groups + 63) / 64 * 64), tpw * lds1, st, d_in, d_out, ntr,
+                       nt, d_h, ntap, (int)off, first, (double)nfft, tpw, groups, (int)span);
     const hipError_t e = hipGetLastError();
     KHIP(hipFreeAsync(d_h, st));
     KHIP(e);

@@ -638,3 +638,24 @@ def test_adjoint_knows_negative_receiver_tables_on_any_stream(torch, domain):
     assert bool((want != 0).sum() > 1.5 * (short != 0).sum())
     K.close()
     e.close()
+
+
+# wavelets as long as the record and much longer: the register-blocked kernel
+# passes over the taps that meet no sample, by wave, with several traces to a
+# wave (9, 64), one (100, 512) and several segments (2100, 6000); one that leaves
+# no output beyond its shift
+@pytest.mark.parametrize("adjoint", [False, True])
+@pytest.mark.parametrize("ntr,nt,nw", [(70, 9, 5000), (33, 64, 700), (3, 100, 13000), (5, 512, 513), (2, 2100, 9000),
+                                       (2, 6000, 10384), (1, 40, 13640)])
+def test_convolution_wavelet_longer_than_the_record(oracle, torch, adjoint, ntr, nt, nw):
+    import ctypes as C
+    from seisfat2d_amd import capi
+    rng = np.random.default_rng(nt + nw)
+    w = rng.standard_normal(nw).astype(np.float32)
+    x = rng.standard_normal((ntr, nt)).astype(np.float32)
+    xi = torch.from_numpy(x).cuda()
+    out = torch.full_like(xi, 7.0)
+    capi.check(capi.lib().seisfat_trace_convolve(int(adjoint), ntr, nt, capi._ptr(w), nw, C.c_void_p(xi.data_ptr()),
+                                                 C.c_void_p(out.data_ptr()),
+                                                 C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert np.array_equal(out.cpu().numpy(), oracle.trace_convolve(x, w, adjoint))
