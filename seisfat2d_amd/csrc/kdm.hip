@@ -331,7 +331,8 @@ __device__ __forceinline__ float exp_mhalf(float y) {
   return __builtin_ldexpf(__builtin_amdgcn_exp2f((hi - n) + lo), (int)n);
 }
 
-// The aperture taper of x about cmp: r_sig = RN(1 / sig_e).
+// The aperture taper of x about cmp: r_sig = RN(1 / sig_e) or its refined
+// reciprocal.
 template <bool RDIV>
 __device__ __forceinline__ float kdm_taper(float x, float cmp, float sig_e, float r_sig) {
   const float n = x - cmp;
@@ -339,10 +340,8 @@ __device__ __forceinline__ float kdm_taper(float x, float cmp, float sig_e, floa
     const float a = n / sig_e;
     return expf(-0.5f * a * a);
   }
-  // |a| < 2^61, so a a is finite and >= 0.  With r_sig the correctly rounded
-  // reciprocal one correction of q0 gives RN(n / sig_e) (see cdiv in
-  // eik_adjoint.hip; r_sig refined twice or not, the quotient is within
-  // 0.5 + 2^-22 ulp)
+  // |a| < 2^61, so a a is finite and >= 0.  One correction of q0 (off by at most
+  // a few ulp, the residual exact) leaves the quotient within 0.5 + 2^-20 ulp
   const float q0 = n * r_sig;
   const float a = __builtin_fmaf(__builtin_fmaf(-sig_e, q0, n), r_sig, q0);
   return exp_mhalf(a * a);
@@ -610,9 +609,8 @@ __global__ __launch_bounds__(256) void k_kdm_sum_parts(float* __restrict__ model
 // minima keep them beyond the last sample with one test, then over 64 when
 // the chunk minima do.
 // Threads per trace (one workgroup, sixteen waves sharing the trace's LDS
-// histogram).  Measured on the 1001 x 1001 survey against 256 and 512 (FP32
-// histogram): the 1 s record's forward 0.224 ms against 0.269 and 0.233 (image),
-// 0.32 against 0.44 and 0.37 (angle).
+// histogram).  A call on the 1001 x 1001 survey's 1 s record with 256, 512 and
+// 1024 threads: 268, 235 and 199 us (image), 500, 435 and 359 us (angle).
 #ifndef SEISFAT_KDM_FWD_THREADS
 #define SEISFAT_KDM_FWD_THREADS 1024
 #endif
@@ -662,9 +660,15 @@ __global__ __launch_bounds__(KDM_FWD_THREADS) void k_kdm_forward(const float* __
         }
         const int i = p % K.nz, j = p / K.nz;
         const float z = (float)i * K.dz, x = (float)j * K.dx;
-        const float sS = K.scale * S[(i + 3) + (size_t)(j + 3) * K.nzz];
+        float sS = K.scale * S[(i + 3) + (size_t)(j + 3) * K.nzz];
         const float sig_e = K.tan_ap * z + KDM_EPS;
-        const float w = kdm_weight<RDIV>(qs, qr, sS, x, sig_e, 1.0f / sig_e, cmp);
+        // the weight's words in flight with the bin's: left alone the compiler
+        // loads them behind the bin's range test, a memory latency later
+        // (sample record 476 against 357 us)
+        if (ANGLE)
+          asm volatile("" : "+v"(sS), "+v"(qs.amp), "+v"(qs.ch), "+v"(qs.sh), "+v"(qr.amp), "+v"(qr.ch), "+v"(qr.sh),
+                       "+v"(qs.dx), "+v"(qs.dz), "+v"(qs.norm), "+v"(qr.dx), "+v"(qr.dz), "+v"(qr.norm));
+        const float w = kdm_weight<RDIV>(qs, qr, sS, x, sig_e, recip_refined(sig_e), cmp);
         if (ANGLE) {
           const int a = kdm_angle_bin(qs, qr, K);
           if (a >= 0 && a < K.nang) atomicAdd(hist + it, (double)(w * model[moff + i + (size_t)a * K.nz]));
