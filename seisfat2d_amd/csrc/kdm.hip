@@ -734,30 +734,41 @@ __global__ __launch_bounds__(256) void k_kdm_tile_bounds(const float* __restrict
   }
 }
 
-// For launch_forward's choice: cnt[0] += the tiles that each trace reaches,
-// cnt[1] += the window rounds these take.  One wave per trace.
+// For launch_forward's choice, over the entries of the adjoint's list and the
+// tiles that one of their traces reaches: cnt[0] += the traces that reach the
+// tile, cnt[1] += the rounds of windows the entry takes.  One wave per entry.
+template <int SB>
 __global__ __launch_bounds__(64) void k_kdm_tile_count(const float* __restrict__ tlo, const float* __restrict__ thi,
-                                                       int ntile, const int* __restrict__ tsrc,
-                                                       const int* __restrict__ trec, int nsrc, KdmK K,
+                                                       int ntile, const int* __restrict__ bsrc,
+                                                       const int* __restrict__ bent, int nb,
+                                                       const int* __restrict__ ent, int nsrc, KdmK K,
                                                        unsigned long long* __restrict__ cnt) {
-  const float* __restrict__ sl = tlo + (size_t)tsrc[blockIdx.x] * ntile;
-  const float* __restrict__ sh = thi + (size_t)tsrc[blockIdx.x] * ntile;
-  const float* __restrict__ rl = tlo + (size_t)(nsrc + trec[blockIdx.x]) * ntile;
-  const float* __restrict__ rh = thi + (size_t)(nsrc + trec[blockIdx.x]) * ntile;
-  unsigned a = 0, b = 0;
+  const int e = blockIdx.x;
+  int b = 0, b1 = nb;  // the entry's block: bent[b] <= e < bent[b + 1]
+  while (b1 - b > 1) {
+    const int m = (b + b1) / 2;
+    (bent[m] <= e ? b : b1) = m;
+  }
+  const int* __restrict__ El = ent + (size_t)e * (1 + SB);
+  const size_t r = (size_t)(nsrc + El[0]) * ntile;
+  unsigned n[2] = {0, 0};
   for (int t = threadIdx.x; t < ntile; t += 64) {
-    if (beyond(sl[t], rl[t], K)) continue;
-    const float w = (fminf(sh[t] + rh[t], K.thr) - fmaxf(sl[t] + rl[t], 0.0f)) / K.dt;
-    ++a;
-    b += 1 + (unsigned)(fminf(fmaxf(w, 0.0f), 16384.0f) / FT_WIN);
+    unsigned most = 0;
+#pragma unroll
+    for (int k = 0; k < SB; ++k) {
+      if (El[1 + k] < 0) continue;
+      const size_t s = (size_t)bsrc[b * SB + k] * ntile;
+      if (beyond(tlo[s + t], tlo[r + t], K)) continue;
+      const float w = (fminf(thi[s + t] + thi[r + t], K.thr) - fmaxf(tlo[s + t] + tlo[r + t], 0.0f)) / K.dt;
+      ++n[0];
+      most = max(most, 1 + (unsigned)(fminf(fmaxf(w, 0.0f), 16384.0f) / FT_WIN));
+    }
+    n[1] += most;
   }
-  for (int off = 32; off >= 1; off >>= 1) {
-    a += __shfl_xor(a, off, 64);
-    b += __shfl_xor(b, off, 64);
-  }
-  if (threadIdx.x == 0 && a) {
-    atomicAdd(cnt, (unsigned long long)a);
-    atomicAdd(cnt + 1, (unsigned long long)b);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    for (int off = 32; off >= 1; off >>= 1) n[c] += __shfl_xor(n[c], off, 64);
+    if (threadIdx.x == 0 && n[c]) atomicAdd(cnt + c, (unsigned long long)n[c]);
   }
 }
 
@@ -1090,6 +1101,7 @@ struct seisfat_kdm_s {
   int* d_src = nullptr;    // trace tables
   int* d_rec = nullptr;
   int nb = 0;              // source blocks of the adjoint
+  int nent = 0;            // entries of its list
   int* d_bsrc = nullptr;   // per block and slot: source table (-1: none)
   int* d_bent = nullptr;   // per block: first entry (nb + 1)
   int* d_ent = nullptr;    // entries {receiver, trace per slot}
@@ -1396,17 +1408,30 @@ int ready(seisfat_kdm_s* k) {
 // needs no bounds if tables or traces changed since), and the bounds' launch is
 // recorded with the tile kernel's, so that a replay follows tables set after the
 // capture.  The same launch precedes every tile kernel once tables were set
-// under capture.  In units
-// of a wave's column and round (0.1 ns on the whole chip), a tile kernel's
-// workgroup costs FT_COST before its first round, and the trace kernel takes
-// 1.4 (tables that stay in the caches) to 3 units per column; either one needs
-// 512 workgroups to fill the chip.  The line lies at 1.6, so that the tiles are
-// taken only where they are surely no slower.  Measured, trace / tile kernel, ms:
-// 1001x1001, 3609 traces: nt 1001 0.25 / 0.67, 1401 0.55 / 0.99, 2001 1.44 / 1.33,
-// 4001 13.1 / 4.6, 8001 16.8 / 6.1; 501x701, 2424 traces of 1251 at 2 ms:
-// 1.68 / 1.05; 499x209, 820 traces of 425 at 4 ms: 0.163 / 0.210; 603x801 angle
-// domain, 2292 traces of 1501 at 2 ms: 6.2 / 3.2.
-constexpr double FT_COST = 400.0, FT_TRACE = 1.6;
+// under capture.
+//
+// The two kernels' times in ns, fitted over 350 surveys (120 to 1001 rows, 200 to
+// 1001 columns, 400 to 8001 samples, both domains).  Tiles: `round` for an entry's
+// round in a tile it reaches, `entry` for each entry of a workgroup's slice (they
+// are taken one after another), `group` for a workgroup.  By traces: for each tile
+// a trace reaches, `near` (more where the image has fewer super-chunks than half
+// of a workgroup's waves: 48000 traces on 65 x 98 take 5.6 ms, by tiles 1.4), up
+// to `far` more as a table outgrows the caches, and `few` more as the traces are
+// too few to fill the chip; its workgroups are larger, 8 us more a launch.
+// The chosen kernel is 1.4 % (image) and 3 % (angle) slower in the mean than the
+// faster one; of 261 surveys in the angle domain 12 run more than 5 % slower than
+// by traces (at most 1.23 times).  Trace / tile kernel, ms: 1001x1001, 3691 traces
+// at 1 ms, image: nt 701 0.102 / 0.128, 1001 0.203 / 0.192, 1501 0.444 / 0.305,
+// 2501 1.18 / 0.65, 5001 4.5 / 2.3; angle: nt 600 0.124 / 0.248, 1001 0.363 /
+// 0.405, 1401 0.79 / 0.65, 2001 1.65 / 1.11, 8001 21.6 / 10.8; 499x209, 1120 traces
+// at 4 ms, angle: nt 425 0.267 / 0.219, 900 0.58 / 0.40.
+struct FtCosts {
+  double round, entry, group, near, far, few;
+};
+constexpr FtCosts ft_costs(bool angle) {
+  return angle ? FtCosts{8.0, 1400.0, 3.0, 1.8, 2.0, 0.6} : FtCosts{6.0, 1300.0, 2.0, 2.1, 1.0, 1.1};
+}
+constexpr double FT_LAUNCH = 8000.0, FT_CACHED = 3e5;  // (image points of a table that the caches hold)
 int derive_bounds(seisfat_kdm_s* k, hipStream_t st) {
   if (k->bounds_dirty) k->by_tiles = false;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1418,15 +1443,18 @@ int derive_bounds(seisfat_kdm_s* k, hipStream_t st) {
                      k->d_q, k->kq, k->nsrc + k->nrec, k->ntz, k->ntile, k->tile_cols, k->K, k->d_tlo, k->d_thi);
   if (!choose) return SEISFAT_OK;
   hipLaunchKernelGGL(k_kdm_clear, dim3(1), dim3(2), 0, st, k->d_cnt);
-  hipLaunchKernelGGL(k_kdm_tile_count, dim3(k->ntr), dim3(64), 0, st, k->d_tlo, k->d_thi, k->ntile, k->d_src, k->d_rec,
-                     k->nsrc, k->K, k->d_cnt);
+  hipLaunchKernelGGL(k_kdm_tile_count<KDM_SB>, dim3(k->nent), dim3(64), 0, st, k->d_tlo, k->d_thi, k->ntile, k->d_bsrc,
+                     k->d_bent, k->nb, k->d_ent, k->nsrc, k->K, k->d_cnt);
   KHIP(hipGetLastError());
   unsigned long long n[2] = {0, 0};
   KHIP(hipMemcpyAsync(n, k->d_cnt, sizeof(n), hipMemcpyDeviceToHost, st));
   KHIP(hipStreamSynchronize(st));
-  const double wgs = (double)k->ntile * k->nb * k->nsplit;
-  const double by_tile = (k->tile_cols * (double)n[1] + FT_COST * wgs) / std::min(1.0, wgs / 512);
-  const double by_trace = FT_TRACE * k->tile_cols * (double)n[0] / std::min(1.0, k->ntr / 512.0);
+  const FtCosts f = ft_costs(k->p.domain == SEISFAT_KDM_ANGLE);
+  const double by_tile = f.round * n[1] + f.entry * k->nent / ((double)k->nb * k->nsplit) +
+                         f.group * k->ntile * k->nb * k->nsplit;
+  const double by_trace =
+      FT_LAUNCH + n[0] * (f.near / std::min(1.0, k->K.nsup / (KDM_FWD_THREADS / 128.0)) +
+                          f.far * std::min(1.0, k->K.npts / FT_CACHED) + f.few / std::min(1.0, k->ntr / 512.0));
   k->by_tiles = by_tile < by_trace && k->ntile <= 8 * 65535 && 4096.0 * k->nb * k->nsplit < 0x1p32 && k->K.dt < 0x1p60f;
   k->bounds_dirty = false;
   return SEISFAT_OK;
@@ -1496,6 +1524,7 @@ int seisfat_kdm_set_traces(seisfat_kdm_t k, int ntr, const int* src, const int* 
   KHIP(hipMemcpy(k->d_bent, bent.data(), bent.size() * sizeof(int), hipMemcpyHostToDevice));
   KHIP(hipMemcpy(k->d_ent, ent.data(), ent.size() * sizeof(int), hipMemcpyHostToDevice));
   k->nb = nb;
+  k->nent = (int)(ent.size() / (1 + KDM_SB));
   // the forward's tiles: enough workgroups for the chip, at least 8 entries each
   const long long wgs = (long long)k->ntile * nb, per_block = (long long)(ent.size() / (1 + KDM_SB)) / nb;
   k->nsplit = (int)std::max<long long>(1, std::min((1024 + wgs - 1) / wgs, per_block / 8));
