@@ -568,7 +568,7 @@ def main():
     ap.add_argument("--tune", type=int, default=1, help="tune the batch's schedule options on this device first "
                                                         "(seisfat2d_amd.tune, not cached)")
     ap.add_argument("--opts", type=str, default=None,
-                    help='schedule options as JSON (e.g. \'{"wpcu": 8}\'); no tuning')
+                    help='schedule options as JSON (e.g. \'{"wpcu": 3}\'); no tuning')
     ap.add_argument("--profile", action="store_true",
                     help="profiler run: the batched steps only, plus a 256 MiB device copy that calibrates "
                          "per-dispatch byte counters")

@@ -1,23 +1,26 @@
 """Schedule tuner for batched solves of the persistent tiled schedule.
 
-The tile is fixed at 64 x 64: one node row per lane of a 64-wide wave (the
-DPP shifts between neighbouring rows need the whole strip in one wave) and
-64 steps, which is what a 16 KB LDS ring of old traveltimes holds.  What
-varies per workload is how the tiles are launched and ordered, the options
-of seisfat_sched_opts:
+The rows of a strip are fixed at 64: one node row per lane of a 64-wide wave
+(the DPP shifts between neighbouring rows need the whole strip in one wave).
+The fused pairs of an isotropic solve walk whole strips in blocks of 8 steps;
+every other solve of the schedule runs 64 x 64 tiles.  What varies per workload
+is how these are launched and ordered, the options of seisfat_sched_opts:
 
   pairs     both sweeps of a pair of sweeps in one launch (1) or one
             persistent launch per sweep (0)
-  wpcu      persistent workgroups per CU (0 = as many as fit)
-  skip      tiles whose every input is the not-reached value are not run
-            where that is exact (1) or every tile runs (0)
-  priority  wave priorities from each shot's scheduling slack (1) or equal (0)
+  wpcu      persistent workgroups per CU (0 = as many as fit; of the strips'
+            workgroups 4 fit)
+  skip      blocks or tiles whose every input is the not-reached value are not
+            run where that is exact (1) or all run (0)
+  priority  wave priorities of the tiles from each shot's scheduling slack (1)
+            or equal (0)
 
 Every combination gives bit-identical traveltimes, so tuning only times
 them: coordinate descent from the defaults, each candidate a fresh batch
 timed by the median device time of its sweep phase (HIP events inside the
 graph) over `runs` runs after `warmup`; a candidate replaces the best only
-when at least 0.5% faster.  The result is cached on disk per workload key:
+when at least 0.5% faster.  Options that amount to a launch already timed are
+not tried.  The result is cached on disk per workload key:
 device name, grid, spacings, solve type, shot count and the histogram of
 window widths in 64-column bins (so two batches with the same geometry and
 width mix share an entry), in the JSON file named by SEISFAT_TUNE_CACHE, or
@@ -36,8 +39,9 @@ from .capi import ISO
 
 VERSION = 1
 DEFAULT = {"pairs": 1, "wpcu": 0, "skip": 1, "priority": 1}
-SPACE = {"pairs": (1, 0), "wpcu": (0, 8, 7, 6), "skip": (1, 0), "priority": (1, 0)}
+SPACE = {"pairs": (1, 0), "wpcu": (0, 8, 7, 6, 3, 2), "skip": (1, 0), "priority": (1, 0)}
 ORDER = ("pairs", "wpcu", "skip", "priority")
+STRIPS_PER_CU = 4  # workgroups of the strip walk that fit a CU
 MIN_GAIN = 0.005
 
 
@@ -92,6 +96,16 @@ def _store(path, key, entry):
     os.replace(tmp, path)
 
 
+def in_effect(opts, type=ISO):
+    """What the options amount to: the fused pairs of an isotropic solve hold at
+    most STRIPS_PER_CU workgroups a CU and have no priorities."""
+    o = dict(opts)
+    if o["pairs"] and type == ISO:
+        o["wpcu"] = 0 if o["wpcu"] >= STRIPS_PER_CU else o["wpcu"]
+        o["priority"] = DEFAULT["priority"]
+    return o
+
+
 def measure(eik, shots, rx, rz, type, opts, runs=5, warmup=2):
     """Median device time (ms) of the sweep phase of a batch with these
     options, and the options it ran with."""
@@ -105,9 +119,12 @@ def measure(eik, shots, rx, rz, type, opts, runs=5, warmup=2):
             b.run()
             t.append(b.sweep_ms())
         b.status()
-        return float(np.median(t)), b.opts
+        return float(np.median(t)), in_effect(b.opts, type)
     finally:
         b.close()
+
+
+measure.in_effect = in_effect
 
 
 def tune(eik, shots, rx=None, rz=None, type=ISO, runs=5, warmup=2, cache=True, force=False, measure=measure,
@@ -124,9 +141,10 @@ def tune(eik, shots, rx=None, rz=None, type=ISO, runs=5, warmup=2, cache=True, f
             return {"opts": dict(hit["opts"]), "ms": hit.get("ms"), "key": key, "cached": True, "trials": []}
     trials = []
     seen = {}
+    effect = getattr(measure, "in_effect", lambda opts, type: opts)
 
     def run(opts):
-        k = tuple(opts[n] for n in ORDER)
+        k = tuple(effect(opts, type)[n] for n in ORDER)
         if k not in seen:
             ms, eff = measure(eik, shots, rx, rz, type, dict(opts), runs=runs, warmup=warmup)
             seen[k] = ms

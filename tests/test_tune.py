@@ -57,6 +57,25 @@ def test_descent_finds_the_optimum_and_caches_it(tmp_path, monkeypatch, best):
     assert not r3["cached"] and r3["opts"] == best and len(calls) == 2 * len(r["trials"])
 
 
+def test_equal_launches_are_timed_once_and_never_chosen_for_noise(tmp_path, monkeypatch):
+    """The strips of an isotropic batch's fused pairs hold 4 workgroups a CU and
+    take no priorities: options that only differ there are the same launch."""
+    monkeypatch.setenv("SEISFAT_TUNE_CACHE", str(tmp_path / "c.json"))
+    calls = []
+
+    def measure(eik, shots, rx, rz, type, opts, runs=5, warmup=2):
+        calls.append(dict(opts))
+        return 10.0 * 0.98 ** len(calls) * (1.0 if opts["pairs"] else 2.0), tune.in_effect(opts, type)
+    measure.in_effect = tune.measure.in_effect
+    r = tune.tune(EIK, SHOTS, measure=measure, device="dev", cache=False)
+    assert r["opts"]["pairs"] == 1 and r["opts"]["wpcu"] in (0, 3, 2) and r["opts"]["priority"] == 1
+    fused = [tuple(tune.in_effect(c, capi.ISO).items()) for c in calls if c["pairs"]]
+    assert len(fused) == len(set(fused)) and {c["wpcu"] for c in calls if c["pairs"]} == {0, 3, 2}
+    assert tune.in_effect({"pairs": 1, "wpcu": 8, "skip": 1, "priority": 0}, capi.ANI)["wpcu"] == 8
+    assert tune.in_effect({"pairs": 0, "wpcu": 8, "skip": 1, "priority": 0}) == \
+        {"pairs": 0, "wpcu": 8, "skip": 1, "priority": 0}
+
+
 def test_small_gains_keep_the_defaults(tmp_path, monkeypatch):
     monkeypatch.setenv("SEISFAT_TUNE_CACHE", str(tmp_path / "c.json"))
 
