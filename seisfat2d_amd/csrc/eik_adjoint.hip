@@ -70,12 +70,6 @@ __device__ __forceinline__ double dpp_shr1_d(double old, double src) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// wave_shl:1: lane k receives lane k+1's `src`; lane 63 keeps `old`.
-__device__ __forceinline__ float dpp_shl1f(float old, float src) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), 0x130, 0xf, 0xf,
-                                                    false));
-}
-
 // time_set + time_init in fp64 (T0 holds 1e6 elsewhere for good).
 __global__ void k_fwd64_init(const AdjShot* __restrict__ shots, int nshots, int nzz, double dx, double dz,
                              double* __restrict__ T0) {

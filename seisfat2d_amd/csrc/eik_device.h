@@ -288,8 +288,10 @@ __device__ __forceinline__ float eik_local_sel(float tv, float te, float tev, co
   // bits(d) <= bits(thr) as unsigned words (floats order as their bit patterns,
   // negatives above all; a difference is never -0).  The conditions exclude
   // d = 0, which changes nothing: its candidate is t0 + h2 RN(sqrt(RN(s^2))) =
-  // t0 + h2 s, not below that axis' 1-D candidate, and where it takes C's place
-  // (de = 0 < dv <= thrC < s dx) branch A holds.
+  // t0 + h2 s, not below that axis' 1-D candidate; and where it takes C's place
+  // (de = 0 < dv <= thrC <= s dx) branch A holds, or te + s dx is below tv
+  // (possible where dx is thousands of dz), and with it the x-axis' 1-D candidate
+  // below both, C's not being below tv.
   // EQH: dx s = dz s, so of the first two only the one for the larger of tv and
   // te can fail.
   const bool cA = EQH ? vmin3(vmin(te, tv) + r.dzs - vmax(te, tv), de, dv) >= 0.0f

@@ -113,8 +113,6 @@ __device__ __forceinline__ float recip_refined(float b) {
 // holds no node that reaches the trace.  The minimum propagates NaN: a chunk
 // holding a NaN traveltime is never passed over (its node's time index would
 // be 0).
-__device__ __forceinline__ float min_nan(float a, float b) { return (a != a || b != b) ? __builtin_nanf("") : fminf(a, b); }
-
 //
 // The kernel is bound by instruction issue, so the usual node (prep_rdiv, the
 // nine traveltimes of magnitude in [2^-30, 2^40)) takes a short path: every
@@ -129,7 +127,7 @@ __device__ __forceinline__ float min_nan(float a, float b) { return (a != a || b
 // 1001 x 1001, 252 tables, image domain: 1.85 ms; 3.15 ms with IEEE division,
 // two FP64 roots and a division per node and seven words written in either
 // domain.
-__device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+__device__ __forceinline__ float min_nan(float a, float b) { return (a != a || b != b) ? __builtin_nanf("") : fminf(a, b); }
 __device__ __forceinline__ float min3f(float a, float b, float c) { return fminf(fminf(a, b), c); }
 
 template <bool ANGLE>
@@ -311,11 +309,11 @@ __device__ __forceinline__ bool beyond(float a, float b, const KdmK& K) { return
 // angle (by the half angles' cosines and sines), and the aperture taper about
 // the trace's CMP.  sS = S / (2 pi) and sig_e = sigma + EPS (with its refined
 // reciprocal r_sig) come in evaluated per node.  The taper is the reference's
-// expression and roundings: (x - cmp) / sig_e, by rdiv with the refined
-// reciprocal and one correction when the host found that no operand needs
-// rescaling (RDIV, the
-// operator's taper_rdiv: every divisor in [EPS, 2^40), every dividend 0 or of
-// magnitude in [2^-59, 2^41)), then expf(-0.5 a a).
+// expression: a = (x - cmp) / sig_e, by the reciprocal and one correction when the
+// host found that no operand needs rescaling (RDIV, the operator's taper_rdiv:
+// every divisor in [EPS, 2^40), every dividend 0 or of magnitude in [2^-59,
+// 2^41)), then exp(-0.5 a a).
+
 // e^(-y / 2) for a finite y >= 0: 2^(-y log2(e) / 2), the exponent split into
 // its rounded product hi and the residual fma(y, L, -hi) + y Llo (L + Llo =
 // -log2(e) / 2), the nearest integer n of hi applied by ldexp to the hardware
