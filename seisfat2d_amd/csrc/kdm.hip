@@ -1095,7 +1095,7 @@ struct seisfat_kdm_s {
   bool tables_in_graph = false;  // tables were set under capture: a replay may change them at any time
   bool by_tiles = false;     // the forward operator's kernel
   int nsplit = 1;            // its workgroups per tile and source block (slices of the entries)
-  int* d_neg = nullptr;     // per receiver table: a negative or NaN value; then their number (k_kdm_rec_neg)
+  int* d_neg = nullptr;     // behind d_cnt: per receiver table, a negative or NaN value; then their number (k_kdm_rec_neg)
   int* d_src = nullptr;    // trace tables
   int* d_rec = nullptr;
   int nb = 0;              // source blocks of the adjoint
@@ -1316,15 +1316,16 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
   hipError_t e = hipMalloc((void**)&k->d_q, (size_t)(nsrc + nrec) * k->kq * npts * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin, (size_t)(nsrc + nrec) * K.nchunk * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tmin2, (size_t)(nsrc + nrec) * K.nsup * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&k->d_neg, ((size_t)nrec + 1) * sizeof(int));
-  if (e == hipSuccess) e = hipMemset(k->d_neg, 0, ((size_t)nrec + 1) * sizeof(int));
   k->ntz = (K.nz + 63) / 64;
   k->tile_cols = FT_WAVES * ft_npt(p->domain == SEISFAT_KDM_ANGLE);
   k->ntile = k->ntz * ((K.nx + k->tile_cols - 1) / k->tile_cols);
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_tlo, (size_t)(nsrc + nrec) * k->ntile * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&k->d_thi, (size_t)(nsrc + nrec) * k->ntile * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&k->d_cnt, 2 * sizeof(unsigned long long));
+  const size_t words = 4 + ((size_t)nrec + 1);  // the two counts, then the receivers' flags and their number
+  if (e == hipSuccess) e = hipMalloc((void**)&k->d_cnt, words * sizeof(int));
   if (e == hipSuccess) {
+    k->d_neg = (int*)(k->d_cnt + 2);
+    launch_fill((float*)k->d_cnt, words, 0.0f, nullptr);
     // exhaustive check of the known-divisor division by dt (every dividend of
     // magnitude in [2^-100, 2^100)) against IEEE division
     float* d = nullptr;
@@ -1345,7 +1346,6 @@ int seisfat_kdm_create(seisfat_eik_t h, const seisfat_kdm_params* p, int nsrc, i
     kfree(k->d_q);
     kfree(k->d_tmin);
     kfree(k->d_tmin2);
-    kfree(k->d_neg);
     kfree(k->d_tlo);
     kfree(k->d_thi);
     kfree(k->d_cnt);
@@ -1597,7 +1597,6 @@ int seisfat_kdm_destroy(seisfat_kdm_t k) {
   kfree(k->d_q);
   kfree(k->d_tmin);
   kfree(k->d_tmin2);
-  kfree(k->d_neg);
   kfree(k->d_tlo);
   kfree(k->d_thi);
   kfree(k->d_cnt);
